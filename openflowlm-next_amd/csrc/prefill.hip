@@ -94,14 +94,15 @@ __device__ __forceinline__ u32x4 dequant8(uint32_t w, uint32_t s, uint32_t nib2,
 // 2^(s_t + e_n) when the operands were scaled (texp / wexp not null), exactly; accum adds
 // the result to what y holds (the second pass of f32 activations). tmap: token t's exponent
 // is texp[tmap[t]] (activations gathered from another row order), else texp[t].
-template <int FN, int FT, bool SCALED>
+// Token fragment j starts TS * j tokens after wt0.
+template <int FN, int FT, int TS, bool SCALED>
 __device__ __forceinline__ void store_tile(const f32x4 (&acc)[FN][FT], float* __restrict__ y,
                                            const int* __restrict__ texp, const int* __restrict__ wexp, int T, int N,
                                            int wt0, int wn0, int accum, const int* __restrict__ tmap = nullptr) {
     const int lane = threadIdx.x & 63, i16 = lane & 15, kg = lane >> 4;
 #pragma unroll
     for (int j = 0; j < FT; ++j) {
-        const int t = wt0 + j * 16 + i16;
+        const int t = wt0 + j * TS + i16;
         if (t >= T) continue;
         const int st = SCALED ? texp[tmap ? max(tmap[t], 0) : t] : 0;
 #pragma unroll
@@ -124,25 +125,26 @@ __device__ __forceinline__ void store_tile(const f32x4 (&acc)[FN][FT], float* __
 }
 
 // The SwiGLU epilogue of the gate/up GEMM over an interleaved matrix (per 128-row pair p,
-// 64 gate rows of F, then the same 64 rows of up: N = 2F). A 256-row tile's wave holds one
-// pair, fragments 0..3 gate and 4..7 up at the same lane positions, so
+// 64 gate rows of F, then the same 64 rows of up: N = 2F). A wave's first FN / 2 fragments are
+// gate rows (from wn0), the others the up rows 64 further on, at the same lane positions, so
 // h = bf16(silu(g) * u) (q4_swiglu_prepare's arithmetic) is formed from the accumulators and
-// only h [T][F] bf16 is stored: the f32 gate/up output never reaches memory.
-template <int FT, bool SCALED>
-__device__ __forceinline__ void store_swiglu(const f32x4 (&acc)[8][FT], uint16_t* __restrict__ h,
+// only h [T][F] bf16 is stored: the f32 gate/up output never reaches memory. Token fragment j
+// starts at wt0 + 64 j.
+template <int FN, int FT, bool SCALED>
+__device__ __forceinline__ void store_swiglu(const f32x4 (&acc)[FN][FT], uint16_t* __restrict__ h,
                                              const int* __restrict__ texp, const int* __restrict__ wexp, int T, int N,
                                              int wt0, int wn0, const int* __restrict__ tmap = nullptr) {
     const int lane = threadIdx.x & 63, i16 = lane & 15, kg = lane >> 4;
-    const int F = N >> 1, f0 = wn0 >> 1;          // wn0 = 128 p: gate rows from 64 p
+    const int F = N >> 1, f0 = (wn0 >> 7) * 64 + (wn0 & 127);   // wn0 = 128 p + c: gate rows from 64 p + c
 #pragma unroll
     for (int j = 0; j < FT; ++j) {
-        const int t = wt0 + j * 16 + i16;
+        const int t = wt0 + j * 64 + i16;
         if (t >= T) continue;
         const int st = SCALED ? texp[tmap ? max(tmap[t], 0) : t] : 0;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < FN / 2; ++i) {
             const int ng = wn0 + i * 16 + kg * 4;
-            f32x4 g = acc[i][j], u = acc[i + 4][j];
+            f32x4 g = acc[i][j], u = acc[i + FN / 2][j];
             if constexpr (SCALED) {
                 const int4 eg = *(const int4*)(wexp + ng), eu = *(const int4*)(wexp + ng + 64);
                 g[0] = ldexpf(g[0], st + eg.x), g[1] = ldexpf(g[1], st + eg.y);
@@ -289,7 +291,7 @@ __global__ __launch_bounds__(64 * WGN * WGT) void prefill_kernel(const uint8_t* 
         __syncthreads();
     }
 
-    store_tile<FN, FT, PREC == 0>(acc, y, texp, wexp, T, N, t0 + wt * WT, n0 + wn * WN, accum);
+    store_tile<FN, FT, 16, PREC == 0>(acc, y, texp, wexp, T, N, t0 + wt * WT, n0 + wn * WN, accum);
 }
 
 // ---------------------------------------------------------------------------
@@ -322,11 +324,7 @@ constexpr int kXRing = 2 * kTileB;               // LDS offset of the activation
 // s_waitcnt immediates (gfx9 encoding: vmcnt[3:0] + vmcnt_hi[15:14], expcnt[6:4], lgkmcnt[11:8]).
 constexpr int wait_imm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | (lgkm << 8); }
 constexpr int kWaitVm0 = wait_imm(0, 15);
-constexpr int kWaitVm6 = wait_imm(6, 15);
-constexpr int kWaitVm10 = wait_imm(10, 15);
 constexpr int kWaitVm0Lgkm0 = wait_imm(0, 0);
-constexpr int kWaitVm4Lgkm0 = wait_imm(4, 0);
-constexpr int kWaitVm6Lgkm0 = wait_imm(6, 0);
 constexpr int kWaitLgkm0 = wait_imm(63, 0);
 
 // 16 bytes per lane from global memory (uniform base + 32-bit lane offset) into LDS at
@@ -368,83 +366,98 @@ __device__ __forceinline__ int xcd_group(int b, int count) {
 }
 __device__ __forceinline__ void vgpr_landed(u32x4& v) { asm volatile("" : "+v"(v)); }
 
-// One output tile of the pipelined kernel: 32 * FN weight rows from n0 x 256 tokens from
-// 256 * bt, K split `split` of `splits` (split s covers stages [st0, st0 + NST) of K / 64 and
+// One output tile of the pipelined kernel: 32 * FN weight rows from n0 x 64 * FT tokens from
+// t0, K split `split` of `splits` (split s covers stages [st0, st0 + NST) of K / (32 KBS) and
 // writes its partial sums to y + s * T * N; the host sums the splits in order).
-// FN = 8: 256 rows, 128x64 wave tiles. FN = 6: 192 rows, 96x64 wave tiles, with the 256-row
-// tile's loads, DMA and dequant unchanged: the waves of row group 3 load row group 2's mx
-// tile again and store it to LDS rows 192..255, which no fragment reads, so every wave
-// issues the same loads and the wait counts below hold for both.
+// KBS: 32-K blocks per stage. A stage always holds eight mx tiles, one per wave, so the row
+// tile narrows as the stage deepens: KBS = 2: 256 rows x 64 K, KBS = 4: 128 rows x 128 K.
+// Waves are 2 along N x 4 along T. A wave's weight rows are [16 FN wn, +16 FN), its token
+// fragments the 16-token groups wt, wt + 4, ... (FT of them), so a tile with few valid tokens
+// (the ragged last tile of T, an expert's tokens) runs an instance with a smaller FT in which
+// every wave does the same, smaller share of the MFMAs, fragment reads and DMA.
+// KBS = 2, FN = 8: 256 rows. FN = 6: 192 rows, with the 256-row tile's loads, DMA and dequant
+// unchanged: the waves of row group 3 load row group 2's mx tile again and store it to LDS
+// rows 192..255, which no fragment reads, so every wave issues the same loads and the wait
+// counts below hold for both.
 // Invariant: every wave issues the same loads, DMA, dequant, waits and barriers in every
-// stage. Wave w's loads and dequant fill row group w & 3, K block w >> 2 of the shared weight
-// buffer for all waves; its DMA copies token rows [32 w, 32 w + 32) of the stage; its wait
-// counts cover only its own loads. Only a wave's fragment reads and MFMAs are private (its
-// accumulators reach memory only for its tokens [64 (w >> 1), +64) below T).
+// stage. Wave w's loads and dequant fill row group w % (8 / KBS), K block w / (8 / KBS) of the
+// shared weight buffer for all waves; its DMAs copy XD 1 KB units (16 token rows x 32 K) of
+// the stage; its wait counts cover only its own loads. Only a wave's fragment reads and MFMAs
+// are private (its accumulators reach memory only for its tokens below T).
 // GATHER: x16 is a row-major 16-bit matrix of K columns instead of the pre-tiled image, and
-// tile row s (token slot 256 bt + s) is DMA'd from its row gmap[256 bt + s] (gmap null: row
-// 256 bt + s itself) through a buffer resource over x16. A padding slot (a negative entry, or
+// token slot t0 + s is DMA'd from its row gmap[t0 + s] (gmap null: row t0 + s itself)
+// through a buffer resource over x16. A padding slot (a negative entry, or
 // a slot at or past T, the tile's valid end) gets a lane offset past the resource's range, so
 // its LDS row is zeros and no memory is read: its products feed only that slot's
 // accumulators, which are never stored, and zero operands spare the MFMAs' power. Each lane
 // fetches the 16-byte chunk that its LDS slot holds under the swizzle, so the LDS image is
 // the pre-tiled one's. The token exponents (PREC 0) are then indexed by source row too:
 // texp[gmap[s]].
-template <int PREC, int FN, bool SWI = false, bool GATHER = false>
+// SWI: the matrix alternates 64 gate and 64 up rows. A 256-row tile's wave holds one such pair
+// as fragments 0..3 and 4..7; in a 128-row tile (one pair) wave wn holds the pair's gate rows
+// [32 wn, +32) as fragments 0, 1 and the same up rows as fragments 2, 3.
+template <int PREC, int KBS, int FN, int FT, bool SWI = false, bool GATHER = false>
 __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict__ packed,
                                          const uint16_t* __restrict__ x16, const int* __restrict__ texp,
                                          const int* __restrict__ wexp, const uint32_t* __restrict__ s16,
-                                         float* __restrict__ y, int T, int N, int K, int n0, int bt, int split,
+                                         float* __restrict__ y, int T, int N, int K, int n0, int t0, int split,
                                          int splits, int accum, const int* __restrict__ gmap = nullptr) {
-    static_assert(FN == 8 || FN == 6, "256- or 192-row tiles");
-    static_assert(!SWI || FN == 8, "the SwiGLU epilogue pairs a 256-row tile's gate and up halves");
-    constexpr int WN = 16 * FN, WT = 64, FT = WT / 16, RG = FN / 2;
+    static_assert((KBS == 2 && (FN == 8 || FN == 6)) || (KBS == 4 && FN == 4), "256-, 192- or 128-row tiles");
+    static_assert(FT >= 1 && FT * KBS <= 8, "a ring slot holds 32 KB of activations");
+    static_assert(!SWI || FN != 6, "the SwiGLU epilogue pairs gate and up rows");
+    constexpr int WN = 16 * FN, RGS = 8 / KBS, RG = FN / 2;
+    constexpr int WPB = RGS * 64 * 64;               // one 32-K plane of the weight buffer
+    constexpr int XPB = FT * 64 * 64;                // one 32-K plane of an activation slot
+    constexpr int XD = FT * KBS / 2;                 // activation DMAs per wave and stage
     typedef typename std::conditional<PREC == 0, f16x8, bf16x8>::type frag_t;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn = wave & 1, wt = wave >> 1;
-    const int t0 = bt * 256;
-    const int KB = K >> 5, NSTK = KB >> 1;
+    const int KB = K >> 5, NSTK = KB / KBS;
     const int st0 = (int)((int64_t)split * NSTK / splits), NST = (int)((int64_t)(split + 1) * NSTK / splits) - st0;
     y += (int64_t)split * T * N;
     const int G = N >> 6;
     const int i16 = lane & 15, kg = lane >> 4;
     const uint32_t lane_row = i16 * 64 + ((kg ^ ((i16 >> 1) & 3)) << 4);   // row i16, chunk kg, swizzled
 
-    // weights: this wave's mx tile of each stage (row group wave & 3, 32-K block wave >> 2)
-    const int rgl = wave & 3, kbl = wave >> 2;
+    // weights: this wave's mx tile of each stage (row group wave % RGS, 32-K block wave / RGS)
+    const int rgl = wave % RGS, kbl = wave / RGS;
     const int rg = min(n0 / 64 + min(rgl, RG - 1), G - 1);              // clamp ragged N
-    const uint8_t* const wsrc = packed + ((int64_t)rg * KB + kbl + 2 * st0) * kTileBytes;
+    const uint8_t* const wsrc = packed + ((int64_t)rg * KB + kbl + KBS * st0) * kTileBytes;
     // scale words: PREC 0 from the fp16 side plane (256 B per tile), PREC 1 from the tile
     constexpr int SSTR = PREC == 0 ? 256 : kTileBytes;
-    const uint8_t* const ssrc = PREC == 0 ? (const uint8_t*)s16 + ((int64_t)rg * KB + kbl + 2 * st0) * 256
+    const uint8_t* const ssrc = PREC == 0 ? (const uint8_t*)s16 + ((int64_t)rg * KB + kbl + KBS * st0) * 256
                                           : wsrc + kCodeBytes;
     const uint32_t coff = lane * 16, soff = i16 * 16;
-    const uint32_t wst = kbl * kPlaneB + rgl * 64 * 64 + lane_row;     // + buffer + r * 1 KB
+    const uint32_t wst = kbl * WPB + rgl * 64 * 64 + lane_row;         // + buffer + r * 1 KB
 
-    // activations: pre-tiled as the LDS image of each stage (32 KB contiguous per token tile
-    // and stage, zero-padded to whole tiles); this wave copies its 32 rows as 4 DMAs of 1 KB.
-    const uint8_t* const xsrc = (const uint8_t*)x16 + (((int64_t)bt * NSTK + st0) * kTileB + wave * 32 * 64);
+    // activations: pre-tiled as the LDS image of each stage ([256-token tile][32-K plane][256
+    // rows], 16 KB per plane, zero-padded to whole 64-token groups); this wave copies the units
+    // XD wave .. + XD of the stage, unit u = 16-row group u / KBS of plane u % KBS.
+    const uint8_t* const xsrc = (const uint8_t*)x16 + (((int64_t)(t0 >> 8) * KB + KBS * st0) * kPlaneB + (t0 & 255) * 64);
     const uint32_t xoff = lane * 16;
-    const uint32_t xdst = (uint32_t)(uintptr_t)lds + kXRing + wave * 32 * 64;   // LDS byte address
-    // GATHER: the byte offset of this lane's chunk in its two token rows (rows 32 w + 16 h +
-    // lane / 4 of the tile; LDS slot lane & 3 holds chunk (lane & 3) ^ ((lane >> 3) & 3))
-    uint32_t goff[2] = {0u, 0u};
+    const uint32_t xdst = (uint32_t)(uintptr_t)lds + kXRing;            // LDS byte address
+    // GATHER: the byte offset of this lane's chunk in its token row of each unit (row lane / 4
+    // of the group; LDS slot lane & 3 holds chunk (lane & 3) ^ ((lane >> 3) & 3))
+    constexpr int GQ = FT % 2 ? 1 : KBS;             // units of a wave that share a row group
+    uint32_t goff[XD / GQ];
     const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc((void*)x16, 0, (int)(kPadOffset - 1),
                                                                          kBufferWord3);   // GATHER only
     if constexpr (GATHER) {
         const uint32_t chunk = (uint32_t)((lane & 3) ^ ((lane >> 3) & 3)) * 16;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int slot = t0 + wave * 32 + h * 16 + (lane >> 2);
+        for (int q = 0; q < XD / GQ; ++q) {
+            const int slot = t0 + (XD * wave + q * GQ) / KBS * 16 + (lane >> 2);
             const int r = slot >= T ? -1 : gmap ? gmap[slot] : slot;
-            goff[h] = r < 0 ? kPadOffset : (uint32_t)r * (uint32_t)(2 * K) + chunk;
+            goff[q] = r < 0 ? kPadOffset : (uint32_t)r * (uint32_t)(2 * K) + chunk;
         }
     }
 
-    // fragment bases: A = weight rows wn*128 + 16i + i16, B = token rows wt*64 + 16j + i16
-    const uint32_t abase = (wn * WN) * 64 + lane_row;
-    const uint32_t bbase = kXRing + (wt * WT) * 64 + lane_row;
+    // fragment bases: A = weight rows (frag_row), B = token rows 64 j + 16 wt + i16
+    constexpr bool kPair = SWI && KBS == 4;
+    const uint32_t abase = (kPair ? wn * 32 : wn * WN) * 64 + lane_row;
+    const uint32_t bbase = kXRing + wt * 1024 + lane_row;
     const uint32_t bbase2 = bbase + 2 * kTileB;                         // ring slot 2 (offset > 64 KB)
     const uint32_t nib2 = vgpr_const(kNib2);
     const uint32_t magic = vgpr_const(PREC == 0 ? kMagic1024 : kMagic128);
@@ -457,26 +470,20 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
 
     u32x4 wc[3], ws[3];                          // three register sets of weight codes + scales
     auto issue_x = [&](int st, int slot) {
-        const uint32_t dst = xdst + slot * kTileB;
-        if constexpr (GATHER) {
-            const uint32_t col = (uint32_t)(st0 + st) * 128;   // uniform: columns 64 (st0 + st)
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int kk = 0; kk < 2; ++kk)
-                    lds_dma16_buf(xrs, goff[h], col + kk * 64, dst + kk * kPlaneB + h * 1024);
-        } else {
-            const uint8_t* src = xsrc + (int64_t)st * kTileB;           // uniform
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int kk = 0; kk < 2; ++kk)
-                    lds_dma16(src + kk * kPlaneB + h * 1024, xoff, dst + kk * kPlaneB + h * 1024);
+        for (int q = 0; q < XD; ++q) {
+            const int u = XD * wave + q;                                // uniform
+            const int unit = u / KBS, plane = u % KBS;
+            const uint32_t dst = xdst + slot * kTileB + plane * XPB + unit * 1024;
+            if constexpr (GATHER)
+                lds_dma16_buf(xrs, goff[q / GQ], (uint32_t)(KBS * (st0 + st) + plane) * 64, dst);
+            else
+                lds_dma16(xsrc + ((int64_t)(KBS * st + plane) * kPlaneB + unit * 1024), xoff, dst);
         }
     };
     auto issue_w = [&](int st, u32x4& c, u32x4& sc) {
-        load16_async(c, wsrc + st * (2 * kTileBytes), coff);           // uniform bases
-        load16_async(sc, ssrc + st * (2 * SSTR), soff);
+        load16_async(c, wsrc + st * (KBS * kTileBytes), coff);         // uniform bases
+        load16_async(sc, ssrc + st * (KBS * SSTR), soff);
     };
     auto store_w = [&](int buf, const u32x4& c, const u32x4& sc, int r0, int r1) {
 #pragma unroll
@@ -484,12 +491,12 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
             *(u32x4*)(lds + wst + buf * kTileB + r * 1024) = dequant8<PREC>(c[r], sc[r], nib2, magic);
     };
     auto read_frags = [&](int buf, int slot, int kk, frag_t (&a)[FN], frag_t (&b)[FT]) {
-        const uint8_t* xp = lds + (slot == 2 ? bbase2 : bbase + slot * kTileB) + kk * kPlaneB;
-        const uint8_t* wp = lds + abase + buf * kTileB + kk * kPlaneB;
+        const uint8_t* xp = lds + (slot == 2 ? bbase2 : bbase + slot * kTileB) + kk * XPB;
+        const uint8_t* wp = lds + abase + buf * kTileB + kk * WPB;
 #pragma unroll
-        for (int j = 0; j < FT; ++j) b[j] = *(const frag_t*)(xp + j * 1024);
+        for (int j = 0; j < FT; ++j) b[j] = *(const frag_t*)(xp + j * 4096);
 #pragma unroll
-        for (int i = 0; i < FN; ++i) a[i] = *(const frag_t*)(wp + i * 1024);
+        for (int i = 0; i < FN; ++i) a[i] = *(const frag_t*)(wp + (kPair ? (i >> 1) * 4096 + (i & 1) * 1024 : i * 1024));
     };
     auto mfmas = [&](const frag_t (&a)[FN], const frag_t (&b)[FT]) {
 #pragma unroll
@@ -500,13 +507,13 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
 
     // Issue order: stage s's weights two stages before its activations (W(s+3) and X(s+2) at
     // the start of stage s), so the in-order vmcnt lets each wait name the youngest loads it
-    // may leave in flight. Prologue: W(0), W(1), X(0), W(2), X(1).
+    // may leave in flight (2 per W, XD per X). Prologue: W(0), W(1), X(0), W(2), X(1).
     issue_w(0, wc[0], ws[0]);
     if (NST > 1) issue_w(1, wc[1], ws[1]);
     issue_x(0, 0);
     if (NST > 2) issue_w(2, wc[2], ws[2]);
     if (NST > 1) issue_x(1, 1);
-    if (NST > 2) __builtin_amdgcn_s_waitcnt(kWaitVm6);        // W(0), W(1), X(0) landed
+    if (NST > 2) __builtin_amdgcn_s_waitcnt(wait_imm(2 + XD, 15));   // W(0), W(1), X(0) landed
     else __builtin_amdgcn_s_waitcnt(kWaitVm0);
     vgpr_landed(wc[0]);
     vgpr_landed(ws[0]);
@@ -518,42 +525,46 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
     // Start: wait for W(st+1) (issued at the start of stage st-2); W(st+3) -> register set
     // P % 3 (W(st)'s, dequantized in stage st-1); X(st+2) -> slot (P+2) % 3 (X(st-1)'s,
     // released by the barrier that ended stage st-1). The dequantization of W(st+1) into the
-    // other weight buffer is spread over both halves of the MFMAs: an MFMA hides about two
+    // other weight buffer is spread over the stage's K blocks: an MFMA hides about two
     // independent VALU instructions, not more. End: wait for X(st+1) and the LDS stores,
     // barrier.
+    constexpr int DW = 4 / KBS;                           // codes dwords dequantized per K block
+    constexpr int NM = FN * FT;                           // MFMAs per K block
+    constexpr int VG = NM >= 22 ? 20 : NM - DW;           // MFMAs with VALU work behind them
+    constexpr int VN = NM >= 22 ? 2 : (20 * DW + VG - 1) / VG;
     auto stage = [&](auto phase, int st) {
         constexpr int P = decltype(phase)::value;
         constexpr int cur = P & 1, slot = P % 3, nslot = (P + 2) % 3, wset = P % 3, nset = (P + 1) % 3;
         const bool w3 = st + 3 < NST, x2 = st + 2 < NST;
-        if (x2) __builtin_amdgcn_s_waitcnt(kWaitVm10);        // W(st+1) landed
+        if (x2) __builtin_amdgcn_s_waitcnt(wait_imm(2 + 2 * XD, 15));   // W(st+1) landed
         else __builtin_amdgcn_s_waitcnt(kWaitVm0);
         vgpr_landed(wc[nset]);
         vgpr_landed(ws[nset]);
         if (w3) issue_w(st + 3, wc[wset], ws[wset]);
         if (x2) issue_x(st + 2, nslot);
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
+        for (int kk = 0; kk < KBS; ++kk) {
             frag_t a[FN], b[FT];
             read_frags(cur, slot, kk, a, b);
-            store_w(cur ^ 1, wc[nset], ws[nset], 2 * kk, 2 * kk + 2);   // rows 16r.., r in [2kk, 2kk+2)
+            store_w(cur ^ 1, wc[nset], ws[nset], DW * kk, DW * kk + DW);
             mfmas(a, b);
             __builtin_amdgcn_sched_group_barrier(0x100, FN + FT, 0);
 #pragma unroll
-            for (int g = 0; g < 20; ++g) {
+            for (int g = 0; g < VG; ++g) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, VN, 0);
             }
 #pragma unroll
-            for (int g = 0; g < 2; ++g) {
+            for (int g = 0; g < DW; ++g) {
                 __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
             }
-            __builtin_amdgcn_sched_group_barrier(0x008, FN * FT - 22, 0);
+            if constexpr (NM > VG + DW) __builtin_amdgcn_sched_group_barrier(0x008, NM - VG - DW, 0);
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (w3) __builtin_amdgcn_s_waitcnt(kWaitVm6Lgkm0);    // X(st+1) landed, LDS stores done
-        else if (x2) __builtin_amdgcn_s_waitcnt(kWaitVm4Lgkm0);
+        if (w3) __builtin_amdgcn_s_waitcnt(wait_imm(2 + XD, 0));        // X(st+1) landed, LDS stores done
+        else if (x2) __builtin_amdgcn_s_waitcnt(wait_imm(XD, 0));
         else __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0);
         asm volatile("s_barrier" ::: "memory");
     };
@@ -581,9 +592,25 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
     // gathered activations carry their exponents by source row
     const int* tmap = GATHER ? gmap : nullptr;
     if constexpr (SWI)
-        store_swiglu<FT, PREC == 0>(acc, (uint16_t*)y, texp, wexp, T, N, t0 + wt * WT, n0 + wn * WN, tmap);
+        store_swiglu<FN, FT, PREC == 0>(acc, (uint16_t*)y, texp, wexp, T, N, t0 + wt * 16,
+                                        n0 + (kPair ? wn * 32 : wn * WN), tmap);
     else
-        store_tile<FN, FT, PREC == 0>(acc, y, texp, wexp, T, N, t0 + wt * WT, n0 + wn * WN, accum, tmap);
+        store_tile<FN, FT, 64, PREC == 0>(acc, y, texp, wexp, T, N, t0 + wt * 16, n0 + wn * WN, accum, tmap);
+}
+
+// dma_tile with the smallest token tile that covers the valid tokens [t0, T) of a tile of
+// 64 * FTMAX (workgroup-uniform). A 256-row stage takes ~0.55, 0.68, 0.85 and 1.0 us with 1 to 4
+// groups of 64 tokens: the dequantization and the LDS traffic of the weights remain.
+template <int PREC, int KBS, int FN, int FTMAX, bool SWI = false, bool GATHER = false, class... A>
+__device__ __forceinline__ void dma_tile_valid(uint8_t* lds, const uint8_t* packed, const uint16_t* x16,
+                                               const int* texp, const int* wexp, const uint32_t* s16, float* y, int T,
+                                               int N, int K, int n0, int t0, A... rest) {
+    const int groups = (T - t0 + 63) >> 6;
+    if (groups >= FTMAX)
+        dma_tile<PREC, KBS, FN, FTMAX, SWI, GATHER>(lds, packed, x16, texp, wexp, s16, y, T, N, K, n0, t0, rest...);
+    else if constexpr (FTMAX > 1)
+        dma_tile_valid<PREC, KBS, FN, FTMAX - 1, SWI, GATHER>(lds, packed, x16, texp, wexp, s16, y, T, N, K, n0, t0,
+                                                              rest...);
 }
 
 // Workgroups [0, wide_wgs) take the 256-row tiles of rows [0, narrow_row0), the rest the
@@ -604,18 +631,39 @@ __global__ __launch_bounds__(512) void prefill_dma_kernel(const uint8_t* __restr
                                          : wide + xcd_group((int)blockIdx.x - wide, G - wide);
     if (!MIXED || b < wide_wgs) {
         const int tile = b / splits;
-        dma_tile<PREC, 8>(lds, packed, x16, texp, wexp, s16, y, T, N, K, (tile / tiles_t) * 256, tile % tiles_t,
-                          b % splits, splits, accum);
+        dma_tile_valid<PREC, 2, 8, 4>(lds, packed, x16, texp, wexp, s16, y, T, N, K, (tile / tiles_t) * 256,
+                                      (tile % tiles_t) * 256, b % splits, splits, accum);
     } else {
         const int i = b - wide_wgs, tile = i / splits;
-        dma_tile<PREC, 6>(lds, packed, x16, texp, wexp, s16, y, T, N, K, narrow_row0 + (tile / tiles_t) * 192,
-                          tile % tiles_t, i % splits, splits, accum);
+        dma_tile_valid<PREC, 2, 6, 4>(lds, packed, x16, texp, wexp, s16, y, T, N, K,
+                                      narrow_row0 + (tile / tiles_t) * 192, (tile % tiles_t) * 256, i % splits, splits,
+                                      accum);
     }
 }
 
-// The gate/up GEMM with the SwiGLU epilogue: workgroup b takes the 256-row tile of pair rows
-// (b / tiles_t) * 256 and token tile b % tiles_t over all of K (no split), writing h.
+// The same GEMM in 128 x 128 tiles of 128-K stages (K % 128 == 0): four times the tiles of the
+// 256 x 256 form, so short prompts and small matrices fill the CUs with fewer K splits, and a
+// workgroup's epilogue stores a quarter of the bytes. What bounds a call here is the start-up,
+// the tile stores and the split planes, not the MFMAs. GEMM + reduce at 4096 x 4096, each
+// form at its best split (graph replays): T = 64 18.9 -> 15.4 us, 128 25.3 -> 21.4, 256 33.4 ->
+// 22.5, 512 40.0 -> 31.3; at 14336 x 4096 T = 512 the 256-row form wins (74.9 against 82.2).
 template <int PREC>
+__global__ __launch_bounds__(512) void prefill_dma128_kernel(const uint8_t* __restrict__ packed,
+                                                             const uint16_t* __restrict__ x16,
+                                                             const int* __restrict__ texp,
+                                                             const int* __restrict__ wexp,
+                                                             const uint32_t* __restrict__ s16, float* __restrict__ y,
+                                                             int T, int N, int K, int tiles_t, int splits, int accum) {
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[5 * kTileB];
+    const int b = xcd_group((int)blockIdx.x, (int)gridDim.x), tile = b / splits;
+    dma_tile_valid<PREC, 4, 4, 2>(lds, packed, x16, texp, wexp, s16, y, T, N, K, (tile / tiles_t) * 128,
+                                  (tile % tiles_t) * 128, b % splits, splits, accum);
+}
+
+// The gate/up GEMM with the SwiGLU epilogue: workgroup b takes the row tile of pair rows
+// (b / tiles_t) and token tile b % tiles_t over all of K (no split), writing h. KBS = 2: 256 x
+// 256 tiles, KBS = 4: 128 x 128.
+template <int PREC, int KBS>
 __global__ __launch_bounds__(512) void prefill_swiglu_kernel(const uint8_t* __restrict__ packed,
                                                              const uint16_t* __restrict__ x16,
                                                              const int* __restrict__ texp,
@@ -625,8 +673,9 @@ __global__ __launch_bounds__(512) void prefill_swiglu_kernel(const uint8_t* __re
                                                              int tiles_t) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[5 * kTileB];
     const int b = xcd_group((int)blockIdx.x, (int)gridDim.x);
-    dma_tile<PREC, 8, true>(lds, packed, x16, texp, wexp, s16, (float*)h, T, N, K, (b / tiles_t) * 256, b % tiles_t,
-                            0, 1, 0);
+    constexpr int R = 512 / KBS;
+    dma_tile_valid<PREC, KBS, 16 / KBS, 8 / KBS, true>(lds, packed, x16, texp, wexp, s16, (float*)h, T, N, K,
+                                                       (b / tiles_t) * R, (b % tiles_t) * R, 0, 1, 0);
 }
 
 // The exponent that puts a positive finite magnitude v in [2^14, 2^15) after scaling by
@@ -940,9 +989,10 @@ constexpr TileCfg kCfgs[] = {
     {128, 128, 2, 4, 2},     // 8 waves, 64x32
     {256, 256, 2, 2, 1},     // 4 waves, 128x128 wave tiles, 32-K stages
     {256, 256, 2, 4, 2},     // the LDS-DMA pipelined kernel (prefill_dma_kernel)
+    {128, 128, 2, 4, 4},     // its 128 x 128 form (prefill_dma128_kernel)
 };
-constexpr int kDmaCfg = 5;
-constexpr int kNumCfgs = sizeof(kCfgs) / sizeof(kCfgs[0]);
+constexpr int kDmaCfg = 5, kDma128Cfg = 6;
+constexpr bool dma_cfg(int cfg) { return cfg >= kDmaCfg; }   // reads the tiled activation image
 
 // Kernel variant: the pipelined kernel whenever K % 64 == 0 (K splits keep small grids
 // busy); otherwise the generic variant with the fewest rounds of 256 workgroups
@@ -952,7 +1002,7 @@ int choose_cfg(int T, int N, int K) {
         const char* e = getenv("Q4MI_PREFILL_CFG");
         return e ? atoi(e) : -1;
     }();
-    if (forced >= 0 && forced < kNumCfgs && K % (32 * kCfgs[forced].ks) == 0) return forced;
+    if (forced >= 0 && forced < kDmaCfg && K % (32 * kCfgs[forced].ks) == 0) return forced;
     if (K % 64 == 0) return kDmaCfg;
     const double eff[] = {1.0, 0.9, 0.9, 0.75, 0.8};   // relative per-workgroup efficiency
     double best = 1e300;
@@ -988,6 +1038,10 @@ void launch_prefill(int cfg, int64_t grid, hipStream_t st, const uint8_t* w, con
         case 2: launch_cfg<2, PREC>(grid, st, w, x16, te, we, s16, y, T, N, K, tiles_t, accum); break;
         case 3: launch_cfg<3, PREC>(grid, st, w, x16, te, we, s16, y, T, N, K, tiles_t, accum); break;
         case 4: launch_cfg<4, PREC>(grid, st, w, x16, te, we, s16, y, T, N, K, tiles_t, accum); break;
+        case kDma128Cfg:
+            hipLaunchKernelGGL((prefill_dma128_kernel<PREC>), dim3((unsigned)grid), dim3(512), 0, st, w, x16, te, we,
+                               s16, y, T, N, K, tiles_t, splits, accum);
+            break;
         default:
             if (wide_wgs < grid)
                 hipLaunchKernelGGL((prefill_dma_kernel<PREC, true>), dim3((unsigned)grid), dim3(512), 0, st, w, x16, te,
@@ -1026,18 +1080,34 @@ int device_cus() {
 }
 
 // Launch plan of one prefill GEMM: the kernel variant, its token tiles and K splits, and for
-// the pipelined kernel the rows covered by 256-row tiles ([0, narrow_row0), wide_wgs
-// workgroups) and by 192-row tiles (the rest). That kernel holds one workgroup per CU (160 KB
-// of LDS). Two levers fit its work to the CUs: a K split (partial sums reduced in order
-// afterwards) and 192-row tiles, which fill the CUs the last round of 256-row tiles leaves
-// idle without any partial traffic (Llama-3-8B gate_up at T = 2048: 448 tiles of 256 rows
-// run in 2 rounds of 256 CUs; 256 of 256 rows + 256 of 192 rows in 1 + 3/4). 192-row
-// strips also cover N % 256 != 0 without repeating rows.
-// Q4MI_PREFILL_SPLITS and Q4MI_PREFILL_NARROW (the count of 192-row strips) override.
+// the 256-row form of the pipelined kernel the rows covered by 256-row tiles ([0,
+// narrow_row0), wide_wgs workgroups) and by 192-row tiles (the rest). Both forms hold one
+// workgroup per CU (160 KB of LDS). Three levers fit the work to the CUs: the tile (256 x 256,
+// or 128 x 128 when K % 128 == 0: four times the tiles, so small grids need fewer K splits
+// and their partial traffic, at two thirds of the MFMA rate), a K split (partial sums
+// reduced in order afterwards) and 192-row tiles, which fill the CUs the last round of 256-row
+// tiles leaves idle without any partial traffic (Llama-3-8B gate_up at T = 2048: 448 tiles of
+// 256 rows run in 2 rounds of 256 CUs; 256 of 256 rows + 256 of 192 rows in 1 + 3/4).
+// 192-row strips also cover N % 256 != 0 without repeating rows.
+// Q4MI_PREFILL_SPLITS and Q4MI_PREFILL_NARROW (the count of 192-row strips) override (256-row
+// tiles only).
 struct PrefillPlan {
     int cfg, tiles_t, splits, wide_wgs, narrow_row0;
     int64_t grid;
 };
+
+// Microseconds of one workgroup of the pipelined kernel: nst stages of a tile of `rows` rows x
+// 64 ft tokens, a start-up and the store of its tile (out_bytes per row and token, at a CU's
+// share of ~4.5 TB/s). Per-stage times measured by varying the K split at T = 64 .. 256 on
+// 14336 x 4096, 4096 x 14336 and 4096 x 4096 (a stage holds eight mx tiles in either form, so
+// its dequantization is the same; the MFMAs grow with ft). 192-row tiles take 0.9 of a
+// 256-row tile's stage (gate_up at T = 2048: 236.6 us as 2 rounds of 256-row tiles, 224.9 as
+// 1 round of each).
+double tile_us(int rows, int ft, int nst, double out_bytes) {
+    static constexpr double s256[5] = {0, 0.55, 0.68, 0.85, 1.0}, s128[3] = {0, 0.66, 0.95};
+    const double stage = rows == 128 ? s128[ft] : rows == 192 ? 0.9 * s256[ft] : s256[ft];
+    return nst * stage + 4.0 + rows * 64.0 * ft * out_bytes / 17600.0;
+}
 
 // Finish time of A units of cost cw followed by B units of cost cn when each starts on the
 // earliest free of C CUs (workgroups dispatch in index order, one per CU).
@@ -1074,13 +1144,12 @@ PrefillPlan make_plan_uncached(int T, int64_t N, int64_t K) {
             const char* e = getenv("Q4MI_PREFILL_NARROW");
             return e ? atoi(e) : -1;
         }();
-        // kNarrowRel: a 192-row tile's time relative to a 256-row tile's over the same stages,
-        // measured: gate_up at T = 2048 took 236.6 us as 2 rounds of 256-row tiles and 224.9 us
-        // as 1 round of each, so the 192-row round ran at ~0.9 of a 256-row one.
-        constexpr double kStageSec = 1.0e-6, kReduceBytesPerSec = 4.0e12, kNarrowRel = 0.9;
         const int nst = (int)(K / 64), cap = nst < 16 ? nst : 16;
         const int64_t G = N / 64, tt = p.tiles_t;
         const int cus = device_cus();
+        const int ftl = (int)ceil_div(T - (tt - 1) * 256, 64);         // 64-token groups of the last token tile
+        // the split reduce: a launch and its traffic
+        auto reduce_us = [&](int S) { return S > 1 ? 3.0 + (double)(S + 1) * T * N * 4 / 5.0e6 : 0.0; };
         // a forced strip count is used only where it fits: 3b <= G and 4 | G - 3b
         const int64_t fb = forced_narrow > 0 && 3 * (int64_t)forced_narrow <= G &&
                                    (G - 3 * (int64_t)forced_narrow) % 4 == 0
@@ -1097,11 +1166,17 @@ PrefillPlan make_plan_uncached(int T, int64_t N, int64_t K) {
             for (int S = 1; S <= cap; ++S) {
                 if (forced > 0 && S != (forced < cap ? forced : cap)) continue;
                 if (b > 0 && b != fb && b * tt * S > 2 * cus) break;
-                const double cw = (double)ceil_div(nst, S) * kStageSec;
-                double cost = makespan(a * tt * S, b * tt * S, cus, cw, cw * kNarrowRel);
-                if (S > 1) cost += (double)(S + 1) * T * N * 4 / kReduceBytesPerSec;
+                const int ns = (int)ceil_div(nst, S);
+                const double full = tile_us(256, 4, ns, 4), last = tile_us(256, ftl, ns, 4);
+                double cost;
+                if (b > 0) {        // every tile at the mean of the full and the ragged token tiles
+                    const double mean = ((double)(tt - 1) + last / full) / (double)tt;
+                    cost = makespan(a * tt * S, b * tt * S, cus, mean * full, mean * tile_us(192, 4, ns, 4));
+                } else {
+                    cost = makespan(a * (tt - 1) * S, a * S, cus, full, last);
+                }
                 // ties: fewer rows computed (a clamped last 256-row strip repeats rows)
-                cost += 1e-12 * (double)(256 * a + 192 * b);
+                cost += reduce_us(S) + 1e-6 * (double)(256 * a + 192 * b);
                 if (cost < best) {
                     best = cost;
                     p.splits = S;
@@ -1111,9 +1186,42 @@ PrefillPlan make_plan_uncached(int T, int64_t N, int64_t K) {
                 }
             }
         }
+        // 128 x 128 tiles, 128-K stages
+        if (K % 128 == 0 && forced <= 0 && forced_narrow < 0) {
+            const int64_t r2 = ceil_div(G, 2), t2 = ceil_div(T, 128);
+            const int nst2 = (int)(K / 128), cap2 = nst2 < 16 ? nst2 : 16;
+            const int ftl2 = (int)ceil_div(T - (t2 - 1) * 128, 64);
+            for (int S = 1; S <= cap2; ++S) {
+                const int ns = (int)ceil_div(nst2, S);
+                const double cost = makespan(r2 * (t2 - 1) * S, r2 * S, cus, tile_us(128, 2, ns, 4),
+                                             tile_us(128, ftl2, ns, 4)) + reduce_us(S);
+                if (cost < best) {
+                    best = cost;
+                    p.cfg = kDma128Cfg;
+                    p.tiles_t = (int)t2;
+                    p.splits = S;
+                    p.wide_wgs = 0;
+                    p.narrow_row0 = (int)N;
+                    tiles = r2 * t2;
+                }
+            }
+        }
     }
     p.grid = tiles * p.splits;
     return p;
+}
+
+// Whether the SwiGLU gate/up GEMM (no K split; bf16 h, one value per gate and up row pair) is
+// planned to finish sooner in 128 x 128 tiles than in 256 x 256 ones.
+bool swiglu_tile128(int T, int64_t N, int64_t K) {
+    if (K % 128) return false;
+    const int cus = device_cus();
+    auto finish = [&](int tile, int nst) {
+        const int64_t tt = ceil_div(T, tile), rows = N / tile;
+        const int ftl = (int)ceil_div(T - (tt - 1) * tile, 64);
+        return makespan(rows * (tt - 1), rows, cus, tile_us(tile, tile / 64, nst, 1), tile_us(tile, ftl, nst, 1));
+    };
+    return finish(128, (int)(K / 128)) < finish(256, (int)(K / 64));
 }
 
 // The plans of the last few shapes per host thread (the workspace query and the call that
@@ -1250,9 +1358,10 @@ int prefill_impl(const uint8_t* packed, const void* scales, const void* x, int x
     uint16_t* x16 = (uint16_t*)workspace;
     int* te = (int*)((char*)workspace + x16_bytes(T, K));
     float* part = (float*)((char*)workspace + xprep_bytes(T, K));
-    const bool tiled = make_plan(T, N, K).cfg == kDmaCfg;
+    const bool tiled = dma_cfg(make_plan(T, N, K).cfg);
     for (int pass = 0; pass < activation_passes(x_dtype, precision); ++pass) {
-        launch_xprep(x_dtype == Q4MI_F32, precision, tiled, dim3((unsigned)padded_tokens(T)), st, x, x16, te, T,
+        // rows up to whole 64-token groups: the kernels read no others
+        launch_xprep(x_dtype == Q4MI_F32, precision, tiled, dim3((unsigned)(ceil_div(T, 64) * 64)), st, x, x16, te, T,
                      (int)K, pass);
         if (launch_status() != Q4MI_OK) return Q4MI_E_LAUNCH;
         const int rc = gemm_pass(packed, scales, x16, te, y, T, N, K, precision, part, pass, st);
@@ -1428,16 +1537,17 @@ extern "C" int q4_gemm_prefill_swiglu(const uint8_t* gate_up, const void* scales
     const int64_t N = 2 * F;
     const int* we = precision == 0 ? (const int*)scales : nullptr;
     const uint32_t* s16 = precision == 0 ? (const uint32_t*)((const char*)scales + scales_wexp_bytes(N)) : nullptr;
-    const int* te = (const int*)((const char*)prepared + x16_bytes(T, K));
-    const int tiles_t = (int)ceil_div(T, 256);
-    const dim3 grid((unsigned)((N / 256) * tiles_t)), block(512);
+    const int* te = precision == 0 ? (const int*)((const char*)prepared + x16_bytes(T, K)) : nullptr;
+    const bool t128 = swiglu_tile128(T, N, K);
+    const int tile = t128 ? 128 : 256, tiles_t = (int)ceil_div(T, tile);
+    const dim3 grid((unsigned)((N / tile) * tiles_t)), block(512);
     const hipStream_t st = (hipStream_t)stream;
-    if (precision == 0)
-        hipLaunchKernelGGL(prefill_swiglu_kernel<0>, grid, block, 0, st, gate_up, (const uint16_t*)prepared, te, we,
-                           s16, (uint16_t*)h, T, (int)N, (int)K, tiles_t);
-    else
-        hipLaunchKernelGGL(prefill_swiglu_kernel<1>, grid, block, 0, st, gate_up, (const uint16_t*)prepared, nullptr,
-                           nullptr, nullptr, (uint16_t*)h, T, (int)N, (int)K, tiles_t);
+#define Q4MI_SG(PR, KBS)                                                                                              \
+    hipLaunchKernelGGL((prefill_swiglu_kernel<PR, KBS>), grid, block, 0, st, gate_up, (const uint16_t*)prepared, te, we, \
+                       s16, (uint16_t*)h, T, (int)N, (int)K, tiles_t)
+    if (precision == 0) { if (t128) Q4MI_SG(0, 4); else Q4MI_SG(0, 2); }
+    else { if (t128) Q4MI_SG(1, 4); else Q4MI_SG(1, 2); }
+#undef Q4MI_SG
     return launch_status();
 }
 
@@ -1455,7 +1565,7 @@ extern "C" int q4_gemm_prefill_prepared(const uint8_t* packed, const void* scale
     if (a != Q4MI_OK) return a > 0 ? Q4MI_OK : a;
     if (precision == 0 && (!scales || misaligned16(scales))) return Q4MI_E_ARG;
     const PrefillPlan plan = make_plan(T, N, K);
-    if ((plan.cfg == kDmaCfg) != (K % 64 == 0)) return Q4MI_E_ARG;   // a forced generic variant reads rows
+    if (dma_cfg(plan.cfg) != (K % 64 == 0)) return Q4MI_E_ARG;   // a forced generic variant reads rows
     if (plan.splits > 1 && (!workspace || workspace_bytes < q4_gemm_prefill_prepared_workspace_bytes(T, N, K)))
         return Q4MI_E_WORKSPACE;
     const int passes = activation_passes(x_dtype, precision);
@@ -1483,7 +1593,7 @@ extern "C" int q4_gemm_prefill_prepared_partials(const uint8_t* packed, const vo
     if (a != Q4MI_OK) return a > 0 ? Q4MI_OK : a;
     if (precision == 0 && (!scales || misaligned16(scales))) return Q4MI_E_ARG;
     const PrefillPlan plan = make_plan(T, N, K);
-    if ((plan.cfg == kDmaCfg) != (K % 64 == 0)) return Q4MI_E_ARG;
+    if (dma_cfg(plan.cfg) != (K % 64 == 0)) return Q4MI_E_ARG;
     // the planes this call writes follow this process's plan, not a count queried elsewhere
     if (part_bytes < (size_t)plan.splits * T * N * sizeof(float)) return Q4MI_E_WORKSPACE;
     const int* te = (const int*)((const char*)prepared + x16_bytes(T, K));
@@ -1798,9 +1908,10 @@ __global__ __launch_bounds__(512) void moe_dma_kernel(const uint8_t* __restrict_
     const int b = blockIdx.x, tt = b / tiles_n, rt = b % tiles_n;
     if (tt >= meta[0]) return;
     const int e = tile_e[tt];
-    dma_tile<PREC, 8, SWI, GATHER>(lds, packed + e * ebytes, x16, texp, PREC == 0 ? wexp + (int64_t)e * N : nullptr,
-                                   PREC == 0 ? s16 + e * s16_words : nullptr, y, tile_end[tt], N, K, rt * 256, tt, 0,
-                                   1, accum, gmap);
+    dma_tile_valid<PREC, 2, 8, 4, SWI, GATHER>(lds, packed + e * ebytes, x16, texp,
+                                               PREC == 0 ? wexp + (int64_t)e * N : nullptr,
+                                               PREC == 0 ? s16 + e * s16_words : nullptr, y, tile_end[tt], N, K,
+                                               rt * 256, tt * 256, 0, 1, accum, gmap);
 }
 
 // out[t][n..n+3] = sum_j w[t][j] Y[slot(t, j)][n..n+3], slot order j.
