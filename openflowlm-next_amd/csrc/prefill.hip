@@ -881,52 +881,106 @@ __global__ __launch_bounds__(256) void prefill_xprep(const void* __restrict__ x,
 //   xn = bf16((y * r) * w) with r as q4_rmsnorm_add forms it (norm_core.h),
 // then xn goes through prefill_xprep's conversion (bf16 source) from an LDS copy of the row.
 // The same bits as q4_rmsnorm_add (bf16 xn) followed by q4_prefill_prepare(xn, bf16), with
-// one launch and no bf16 row in memory. PER values per thread (K <= 256 PER); extra j terms
-// are zeros, which leave the fp64 sum of squares unchanged.
+// one launch and no bf16 row in memory. Bound by the loads of x and the planes (T = 512, K = 4096:
+// 8 MB each), so a thread takes PER / 4 groups of four neighbouring values and issues all of a
+// row's loads, PB planes at a time, before the first is used (16 bytes each; vec 0: some pointer
+// is not 16-byte aligned, four 4-byte loads). One plane and one value at a time, each behind the
+// last, took 29.7 us at five planes, this 14.7 (4.3 TB/s). The row also goes to LDS, from which thread
+// tid sums the squares of elements tid + 256 j, j ascending, as rmsnorm_add_kernel does (values
+// past K are zeros there and are skipped here: the fp64 sum is the same).
 template <int PER, int PREC, bool TILED>
 __global__ __launch_bounds__(256) void rmsnorm_prepare_kernel(const float* x, const float* __restrict__ add,
                                                               int add_planes, const void* __restrict__ w, int w_bf16,
-                                                              float* y, uint16_t* __restrict__ x16,
+                                                              int vec, float* y, uint16_t* __restrict__ x16,
                                                               int* __restrict__ texp, int T, int K, float eps) {
+    constexpr int C = PER / 4, PB = PER <= 16 ? 4 : PER <= 32 ? 2 : 1;
     __shared__ double part[4];
-    __shared__ __attribute__((aligned(16))) uint16_t xs[256 * PER];
+    __shared__ __attribute__((aligned(16))) float row[256 * PER];   // f32 x, then the bf16 xn
+    uint16_t* const xs = (uint16_t*)row;
     const int t = blockIdx.x, tid = threadIdx.x;
     if (t < T) {
+        auto ld4 = [&](const float* p) -> f32x4 {
+            if (vec) return load_global<f32x4>(p);
+            return f32x4{load_global<float>(p), load_global<float>(p + 1), load_global<float>(p + 2),
+                         load_global<float>(p + 3)};
+        };
         const float* xr = x + (int64_t)t * K;
-        const float* ar = add ? add + (int64_t)t * K : nullptr;
         const int64_t pstride = (int64_t)T * K;      // plane q of add at add + q T K
-        float v[PER], wv[PER];
+        f32x4 v[C], wv[C];
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int i = min(4 * (tid + 256 * c), K - 4);          // loads stay in the row
+            v[c] = ld4(xr + i);
+            if (w_bf16) {
+                const uint16_t* p = (const uint16_t*)w + i;
+                u32x2 d;
+                if (vec) d = load_global<u32x2>(p);
+                else d = u32x2{load_global<uint16_t>(p) | ((uint32_t)load_global<uint16_t>(p + 1) << 16),
+                               load_global<uint16_t>(p + 2) | ((uint32_t)load_global<uint16_t>(p + 3) << 16)};
+                wv[c] = f32x4{bf16_lo_to_f32(d[0]), bf16_hi_to_f32(d[0]), bf16_lo_to_f32(d[1]), bf16_hi_to_f32(d[1])};
+            } else {
+                wv[c] = ld4((const float*)w + i);
+            }
+        }
+        if (add) {                                   // the planes in prefill_reduce_kernel's order
+            const float* ar = add + (int64_t)t * K;
+            f32x4 s[C];
+            for (int q0 = 0; q0 < add_planes; q0 += PB) {
+                f32x4 a[PB][C];
+#pragma unroll
+                for (int u = 0; u < PB; ++u)
+#pragma unroll
+                    for (int c = 0; c < C; ++c)
+                        a[u][c] = ld4(ar + (int64_t)min(q0 + u, add_planes - 1) * pstride +
+                                      min(4 * (tid + 256 * c), K - 4));
+#pragma unroll
+                for (int u = 0; u < PB; ++u)
+                    if (q0 + u < add_planes) {
+#pragma unroll
+                        for (int c = 0; c < C; ++c) s[c] = q0 + u == 0 ? a[u][c] : s[c] + a[u][c];
+                    }
+            }
+#pragma unroll
+            for (int c = 0; c < C; ++c) v[c] = v[c] + s[c];
+        }
+        float* yr = y ? y + (int64_t)t * K : nullptr;
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int i = 4 * (tid + 256 * c);
+            if (i < K) *(f32x4*)(row + i) = v[c];
+        }
+        __syncthreads();
         double ss = 0.0;
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
             const int i = tid + 256 * j;
-            float a = 0.0f;
-            if (ar && i < K) {          // the planes in prefill_reduce_kernel's order
-                a = ar[i];
-                for (int q = 1; q < add_planes; ++q) a += ar[q * pstride + i];
-            }
-            v[j] = i < K ? (ar ? xr[i] + a : xr[i]) : 0.0f;
-            wv[j] = i >= K ? 0.0f
-                           : (w_bf16 ? bf16_hi_to_f32((uint32_t)((const uint16_t*)w)[i] << 16) : ((const float*)w)[i]);
+            if (i < K) ss += (double)row[i] * (double)row[i];
         }
-#pragma unroll
-        for (int j = 0; j < PER; ++j) ss += (double)v[j] * (double)v[j];
         const double ws = wave_sum_ss(ss);
         if ((tid & 63) == 0) part[tid >> 6] = ws;
-        __syncthreads();
-        if (y) {
-            float* yr = y + (int64_t)t * K;
+        __syncthreads();                             // row free: xs takes its place
+        if (yr) {                                    // y may be x: the row was read above
 #pragma unroll
-            for (int j = 0; j < PER; ++j) {
-                const int i = tid + 256 * j;
-                if (i < K) yr[i] = v[j];
+            for (int c = 0; c < C; ++c) {
+                const int i = 4 * (tid + 256 * c);
+                if (i >= K) continue;
+                if (vec) {
+                    *(f32x4*)(yr + i) = v[c];
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) yr[i + e] = v[c][e];
+                }
             }
         }
         const float r = inv_rms(part, K, eps);
 #pragma unroll
-        for (int j = 0; j < PER; ++j) {
-            const int i = tid + 256 * j;
-            if (i < K) xs[i] = (uint16_t)f32_to_bf16_rne(v[j] * r * wv[j]);
+        for (int c = 0; c < C; ++c) {
+            const int i = 4 * (tid + 256 * c);
+            if (i < K)
+                *(u32x2*)(xs + i) = u32x2{f32_to_bf16_rne(v[c][0] * r * wv[c][0]) |
+                                              (f32_to_bf16_rne(v[c][1] * r * wv[c][1]) << 16),
+                                          f32_to_bf16_rne(v[c][2] * r * wv[c][2]) |
+                                              (f32_to_bf16_rne(v[c][3] * r * wv[c][3]) << 16)};
         }
         __syncthreads();
     }
@@ -1054,13 +1108,22 @@ void launch_prefill(int cfg, int64_t grid, hipStream_t st, const uint8_t* w, con
 }
 
 // y = sum of the S partials in split order (deterministic), 4 floats per thread; accum adds
-// it to what y holds.
+// it to what y holds. Eight planes' loads go out together: one load behind the other took 0.5
+// to 0.9 us longer per call (T = 64, N = 2048, 8 planes: 4.3 -> 3.4 us).
 __global__ __launch_bounds__(256) void prefill_reduce_kernel(const f32x4* __restrict__ part, f32x4* __restrict__ y,
                                                              int64_t MN4, int S, int accum) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= MN4) return;
-    f32x4 s = part[i];
-    for (int q = 1; q < S; ++q) s += part[(int64_t)q * MN4 + i];
+    constexpr int B = 8;
+    f32x4 s;
+    for (int q = 0; q < S; q += B) {
+        f32x4 t[B];
+#pragma unroll
+        for (int u = 0; u < B; ++u) t[u] = part[(int64_t)min(q + u, S - 1) * MN4 + i];
+#pragma unroll
+        for (int u = 0; u < B; ++u)
+            if (q + u < S) s = q + u == 0 ? t[u] : s + t[u];
+    }
     y[i] = accum ? y[i] + s : s;
 }
 
@@ -1476,17 +1539,20 @@ extern "C" int q4_rmsnorm_prepare(const float* x, const float* add, int add_plan
     const dim3 grid((unsigned)padded_tokens(T)), block(256);
     const hipStream_t st = (hipStream_t)stream;
     const int wb = w_dtype == Q4MI_BF16;
-    const bool tiled = K % 64 == 0, small = K <= 256 * 16;
+    const bool tiled = K % 64 == 0;
+    const int vec = !misaligned16(x) && !misaligned16(add) && !misaligned16(w) && !misaligned16(y);
 #define Q4MI_RP(PER, PR, TL)                                                                                   \
-    hipLaunchKernelGGL((rmsnorm_prepare_kernel<PER, PR, TL>), grid, block, 0, st, x, add, add_planes, w, wb, y, x16, \
-                       te, T, (int)K, eps)
-    if (precision == 0) {
-        if (small) { if (tiled) Q4MI_RP(16, 0, true); else Q4MI_RP(16, 0, false); }
-        else { if (tiled) Q4MI_RP(64, 0, true); else Q4MI_RP(64, 0, false); }
-    } else {
-        if (small) { if (tiled) Q4MI_RP(16, 1, true); else Q4MI_RP(16, 1, false); }
-        else { if (tiled) Q4MI_RP(64, 1, true); else Q4MI_RP(64, 1, false); }
-    }
+    hipLaunchKernelGGL((rmsnorm_prepare_kernel<PER, PR, TL>), grid, block, 0, st, x, add, add_planes, w, wb, vec, y, \
+                       x16, te, T, (int)K, eps)
+#define Q4MI_RP_K(PR, TL)                                                                            \
+    do {                                                                                             \
+        if (K <= 256 * 16) Q4MI_RP(16, PR, TL);                                                      \
+        else if (K <= 256 * 32) Q4MI_RP(32, PR, TL);                                                 \
+        else Q4MI_RP(64, PR, TL);                                                                    \
+    } while (0)
+    if (precision == 0) { if (tiled) Q4MI_RP_K(0, true); else Q4MI_RP_K(0, false); }
+    else { if (tiled) Q4MI_RP_K(1, true); else Q4MI_RP_K(1, false); }
+#undef Q4MI_RP_K
 #undef Q4MI_RP
     return launch_status();
 }
