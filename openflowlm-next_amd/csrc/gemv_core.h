@@ -75,6 +75,14 @@ __device__ __forceinline__ void load_xfrag(const void* __restrict__ x, int64_t K
     }
 }
 
+// The two bf16 halves of an f32 activation that the MFMA takes, v = hi + lo up to 2^-18 |v|. No
+// contraction: v may be a product, and v - hi is the rounded one's remainder.
+__device__ __forceinline__ void split_bf16(float v, __bf16& hi, __bf16& lo) {
+#pragma clang fp contract(off)
+    hi = (__bf16)v;
+    lo = (__bf16)(v - (float)hi);
+}
+
 // Accumulate this wave's share of tiles [kb0, kb1) of row group g: with WAVES waves in
 // the workgroup, wave w takes tiles kb0 + w, kb0 + w + WAVES, ...
 // Loads are unconditional (a tile index past kb1 is clamped to kb1 - 1 and
@@ -498,8 +506,9 @@ __device__ __forceinline__ void static_for(F&& f) {
 // position b as soon as b has been used, so the wait before each position is "all but the
 // (UNR - 1) younger positions' loads"; the last chunk waits down to zero. Positions of the
 // last chunk past cnt load the wave's last tile again (at most UNR - 1, cache hits) and
-// are not accumulated.
-template <int NTL, bool XF32, int NG, int UNR, int WAVES, class Rows>
+// are not accumulated. SPLIT (with XF32): a row of x is stored as its two bf16 halves, K hi values
+// and then the K lo values (split_bf16), instead of K f32 values that every workgroup splits.
+template <int NTL, bool XF32, int NG, int UNR, int WAVES, bool SPLIT = false, class Rows>
 __device__ __forceinline__ void gemv_rows_pipe(const uint8_t* const (&gbase)[NG], const void* __restrict__ x, Rows rows,
                                                int64_t K, int kb0, int kb1, float (&acc)[NG][4][NTL]) {
     constexpr int XL = XF32 ? 2 : 1;                // activation loads per K position
@@ -515,8 +524,8 @@ __device__ __forceinline__ void gemv_rows_pipe(const uint8_t* const (&gbase)[NG]
     const int i16 = lane & 15, kg = lane >> 4;
     const uint32_t coff = lane * 16, soff = kCodeBytes + i16 * 16;
     const CodeConsts kc = code_consts();
-    const int64_t es = XF32 ? 4 : 2;
-    const uint8_t* xp = (const uint8_t*)x + (rows(token_of_row(i16)) * K + kg * 8) * es;
+    const int64_t es = XF32 && !SPLIT ? 4 : 2, hs = SPLIT ? 2 * K : 16;   // bytes to the second load of a fragment
+    const uint8_t* xp = (const uint8_t*)x + (rows(token_of_row(i16)) * (SPLIT ? 2 : 1) * K + kg * 8) * es;
     u32x4 c[UNR][NG], s[UNR][NG], xr[UNR][XL];
     auto issue = [&](int b, int slot) {
         const int t = first + WAVES * min(b, cnt - 1);
@@ -528,7 +537,7 @@ __device__ __forceinline__ void gemv_rows_pipe(const uint8_t* const (&gbase)[NG]
         }
         const uint8_t* xa = xp + (int64_t)t * 32 * es;
 #pragma unroll
-        for (int h = 0; h < XL; ++h) pipe_load_x(xr[slot][h], xa + 16 * h);
+        for (int h = 0; h < XL; ++h) pipe_load_x(xr[slot][h], xa + hs * h);
     };
     auto land = [&](int slot) {
 #pragma unroll
@@ -541,7 +550,10 @@ __device__ __forceinline__ void gemv_rows_pipe(const uint8_t* const (&gbase)[NG]
     };
     auto run = [&](int u) {
         bf16x8 xh, xl;
-        if constexpr (XF32) {
+        if constexpr (SPLIT) {
+            xh = __builtin_bit_cast(bf16x8, xr[u][0]);
+            xl = __builtin_bit_cast(bf16x8, xr[u][1]);
+        } else if constexpr (XF32) {
             const f32x4 a = __builtin_bit_cast(f32x4, xr[u][0]), bb = __builtin_bit_cast(f32x4, xr[u][1]);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -555,6 +567,134 @@ __device__ __forceinline__ void gemv_rows_pipe(const uint8_t* const (&gbase)[NG]
             xh = __builtin_bit_cast(bf16x8, xr[u][0]);
         }
         multi_tile<NTL, XF32, NG>(c[u], s[u], xh, xl, kc, acc);
+    };
+#pragma unroll
+    for (int u = 0; u < UNR; ++u) issue(u, u);
+    int b0 = 0;
+    for (; b0 + UNR < cnt; b0 += UNR) {
+#pragma unroll
+        for (int u = 0; u < UNR; ++u) {
+            __builtin_amdgcn_s_waitcnt(pipe_wait_imm((UNR - 1) * L));
+            land(u);
+            run(u);
+            issue(b0 + u + UNR, u);
+        }
+    }
+    static_for<0, UNR>([&](auto U) {      // the last chunk: nothing more to issue
+        constexpr int u = decltype(U)::value;
+        __builtin_amdgcn_s_waitcnt(pipe_wait_imm((UNR - 1 - u) * L));
+        land(u);
+        if (b0 + u < cnt) run(u);
+    });
+}
+
+// gemv_rows_pipe for up to 32 rows: two 16-token blocks share each tile's code and scale loads and
+// the codes' conversion to bf16. Block b holds tokens 16 b .. 16 b + 15 in acc[b]; each block is
+// the 16-token case (its own fragment, -128 sum and MFMAs), so a token's bits are
+// gemv_rows_pipe's with four accumulators.
+template <bool XF32, int NG, int UNR, int WAVES, bool SPLIT = false, class Rows>
+__device__ __forceinline__ void gemv_rows_pipe_tb2(const uint8_t* const (&gbase)[NG], const void* __restrict__ x,
+                                                   Rows rows, int64_t K, int kb0, int kb1,
+                                                   float (&acc)[2][NG][4][4]) {
+    constexpr int XL = XF32 ? 2 : 1;                // activation loads per K position and block
+    constexpr int L = 2 * NG + 2 * XL;              // loads per K position
+    static_assert((UNR - 1) * L <= 63, "vmcnt holds 6 bits");
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    kb0 = __builtin_amdgcn_readfirstlane(kb0);
+    kb1 = __builtin_amdgcn_readfirstlane(kb1);
+    const int first = kb0 + wave;
+    if (first >= kb1) return;
+    const int cnt = (kb1 - first + WAVES - 1) / WAVES;
+    const int i16 = lane & 15, kg = lane >> 4;
+    const uint32_t coff = lane * 16, soff = kCodeBytes + i16 * 16;
+    const CodeConsts kc = code_consts();
+    const int64_t es = XF32 && !SPLIT ? 4 : 2, hs = SPLIT ? 2 * K : 16;
+    const uint8_t* xp[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+        xp[b] = (const uint8_t*)x + (rows(16 * b + token_of_row(i16)) * (SPLIT ? 2 : 1) * K + kg * 8) * es;
+    u32x4 c[UNR][NG], s[UNR][NG], xr[UNR][2][XL];
+    auto issue = [&](int p, int slot) {
+        const int t = first + WAVES * min(p, cnt - 1);
+        const uint32_t toff = (uint32_t)t * kTileBytes;
+#pragma unroll
+        for (int i = 0; i < NG; ++i) {
+            pipe_load_w(c[slot][i], gbase[i], toff + coff);
+            pipe_load_w(s[slot][i], gbase[i], toff + soff);
+        }
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int h = 0; h < XL; ++h) pipe_load_x(xr[slot][b][h], xp[b] + (int64_t)t * 32 * es + hs * h);
+    };
+    auto land = [&](int slot) {
+#pragma unroll
+        for (int i = 0; i < NG; ++i) {
+            pipe_landed(c[slot][i]);
+            pipe_landed(s[slot][i]);
+        }
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int h = 0; h < XL; ++h) pipe_landed(xr[slot][b][h]);
+    };
+    const bf16x8 neg128 = __builtin_bit_cast(bf16x8, u32x4{0xC300C300u, 0xC300C300u, 0xC300C300u, 0xC300C300u});
+    const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
+    auto run = [&](int u) {
+        bf16x8 xh[2], xl[2];
+        f32x4 ns[2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            if constexpr (SPLIT) {
+                xh[b] = __builtin_bit_cast(bf16x8, xr[u][b][0]);
+                xl[b] = __builtin_bit_cast(bf16x8, xr[u][b][1]);
+            } else if constexpr (XF32) {
+                const f32x4 v0 = __builtin_bit_cast(f32x4, xr[u][b][0]), v1 = __builtin_bit_cast(f32x4, xr[u][b][1]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const __bf16 ha = (__bf16)v0[e], hb = (__bf16)v1[e];
+                    xh[b][e] = ha;
+                    xh[b][e + 4] = hb;
+                    xl[b][e] = (__bf16)(v0[e] - (float)ha);
+                    xl[b][e + 4] = (__bf16)(v1[e] - (float)hb);
+                }
+            } else {
+                xh[b] = __builtin_bit_cast(bf16x8, xr[u][b][0]);
+            }
+            ns[b] = mfma_bf16(xh[b], neg128, zero4);
+            if constexpr (XF32) ns[b] = mfma_bf16(xl[b], neg128, ns[b]);
+        }
+        float sx[2][4];
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sx[b][j] = ns[b][j] * (-1.0f / 128.0f);
+#pragma unroll
+        for (int i = 0; i < NG; ++i) {
+            f32x4 p[4][2];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const bf16x8 w = codes_to_bf16(c[u][i][r], kc);
+#pragma unroll
+                for (int b = 0; b < 2; ++b) p[r][b] = mfma_bf16(xh[b], w, ns[b]);
+                if constexpr (XF32) {
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) p[r][b] = mfma_bf16(xl[b], w, p[r][b]);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float d = bf16_hi_to_f32(s[u][i][r]), m = bf16_lo_to_f32(s[u][i][r]);
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        acc[b][i][r][j] = __builtin_fmaf(d, p[r][b][j], acc[b][i][r][j]);
+                        acc[b][i][r][j] = __builtin_fmaf(m, sx[b][j], acc[b][i][r][j]);
+                    }
+            }
+        }
     };
 #pragma unroll
     for (int u = 0; u < UNR; ++u) issue(u, u);

@@ -45,7 +45,7 @@ constexpr int kDnWaves = 4, kDnUnr = 2, kDnGroups = 4;
 // come first in the grid and the rest leave at once. The ids are also left in sids (LDS, P
 // entries) for collect_pairs, so the routing reads them from memory once.
 template <int WAVES>
-__device__ int active_expert(const int32_t* __restrict__ ids, int P, int E, int a, int* sids) {
+__device__ __forceinline__ int active_expert(const int32_t* __restrict__ ids, int P, int E, int a, int* sids) {
     __shared__ uint32_t bits[kMaxExperts / 32];
     __shared__ int wsum[WAVES];
     __shared__ int found;
@@ -104,7 +104,7 @@ __device__ int active_expert(const int32_t* __restrict__ ids, int P, int E, int 
 // pairs from t times that on (read as 16-byte vectors), so a block-wide prefix sum of the
 // threads' counts orders the matches, in one pass for any P <= kMaxPairs.
 template <int WAVES>
-__device__ int collect_pairs_runs(const int* sids, int P, int e, int* list) {
+__device__ __forceinline__ int collect_pairs_runs(const int* sids, int P, int e, int* list) {
     constexpr int kPer = kMaxPairs / (64 * WAVES);
     static_assert(kPer % 4 == 0, "whole 16-byte groups per thread");
     __shared__ int wave_cnt[WAVES];
@@ -147,7 +147,7 @@ __device__ int collect_pairs_runs(const int* sids, int P, int e, int* list) {
 // (every thread calls it; barriers inside). sids: the ids as active_expert left them in LDS.
 // Up to one pair per thread (decode batches): a ballot compaction; more: collect_pairs_runs.
 template <int WAVES>
-__device__ int collect_pairs(const int* sids, int P, int e, int* list) {
+__device__ __forceinline__ int collect_pairs(const int* sids, int P, int e, int* list) {
     if (P > 64 * WAVES) return collect_pairs_runs<WAVES>(sids, P, e, list);
     __shared__ int wave_cnt[WAVES];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -167,9 +167,28 @@ __device__ int collect_pairs(const int* sids, int P, int e, int* list) {
     return total;
 }
 
+// A pointer every lane agrees on, in scalar registers.
+__device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
+    const uint64_t v = (uint64_t)p;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return (const uint8_t*)(((uint64_t)hi << 32) | lo);
+}
+
 __device__ __forceinline__ float silu(float g) { return g / (1.0f + expf(-g)); }
 
-template <int NTL, bool XF32, int WAVES, int UNR>
+// h of a pair's row p: f32 [F], or with SPLIT its bf16 halves ([F] hi, then [F] lo; as many bytes).
+template <bool SPLIT>
+__device__ __forceinline__ void store_h(float* hbuf, int64_t p, int F, int64_t f, float v) {
+    if constexpr (SPLIT) {
+        __bf16* const row = (__bf16*)(hbuf + p * F);
+        split_bf16(v, row[f], row[F + f]);
+    } else {
+        hbuf[p * F + f] = v;
+    }
+}
+
+template <int NTL, bool XF32, int WAVES, int UNR, bool SPLIT = false>
 __device__ __forceinline__ void up_chunk(const uint8_t* wexp, const void* x, int H, int F, int rgp, const int* rows,
                                          const int* pairs, int M, float* red, float* __restrict__ hbuf) {
     // the gate rows (row group 2 rgp) and the up rows next to them (2 rgp + 1) in one stream
@@ -195,7 +214,7 @@ __device__ __forceinline__ void up_chunk(const uint8_t* wexp, const void* x, int
 #pragma unroll
     for (int j = 0; j < NTL; ++j) {
         const int tok = token_of(kg, j);
-        if (tok < M) hbuf[(int64_t)pairs[tok] * F + f] = silu(vg[j]) * vu[j];
+        if (tok < M) store_h<SPLIT>(hbuf, pairs[tok], F, f, silu(vg[j]) * vu[j]);
     }
 }
 
@@ -270,7 +289,7 @@ __global__ __launch_bounds__(64 * kUpWaves) void moe_up_kernel(const uint8_t* __
 
 // NG 64-row groups of H per down workgroup: K = F is short, so one group alone is
 // latency-bound.
-template <int NTL, int NG, int WAVES, int UNR>
+template <int NTL, int NG, int WAVES, int UNR, bool SPLIT = false>
 __device__ __forceinline__ void down_chunk(const uint8_t* wexp, const float* hbuf, int H, int F, int rg0,
                                            const int* pairs, int M, float* red, float* __restrict__ ypair) {
     float acc[NG][4][NTL];
@@ -284,7 +303,7 @@ __device__ __forceinline__ void down_chunk(const uint8_t* wexp, const float* hbu
     const uint8_t* gb[NG];
 #pragma unroll
     for (int i = 0; i < NG; ++i) gb[i] = wexp + (int64_t)(rg0 + i) * KB * kTileBytes;
-    gemv_rows_pipe<NTL, true, NG, UNR, WAVES>(gb, hbuf, GatherRows{pairs, M}, F, 0, KB, acc);
+    gemv_rows_pipe<NTL, true, NG, UNR, WAVES, SPLIT>(gb, hbuf, GatherRows{pairs, M}, F, 0, KB, acc);
     float (*rd)[4][NTL][64] = (float (*)[4][NTL][64])red;
     const int tid = threadIdx.x, lane = tid & 63, r = tid >> 6, i16 = lane & 15, kg = lane >> 4;
 #pragma unroll
@@ -349,6 +368,225 @@ __global__ __launch_bounds__(64 * kDnWaves) void moe_down_kernel(const uint8_t* 
         }
         __syncthreads();
     }
+}
+
+// ---------------------------------------------------------------------------
+// Many pairs per expert (more than kManyPerExpert on average): work items are (expert, 32 of its
+// pairs), so an expert's pairs run side by side instead of chunk by chunk in one workgroup, and
+// two 16-token blocks share each weight tile's loads and conversion (gemv_rows_pipe_tb2). The up
+// kernel stores h as the two bf16 halves that the down kernel's MFMAs take. Same arithmetic and
+// bits as the kernels above. Bound by the time of a chunk (~1 us per chunk of 128 experts' or 16
+// experts' rows alike: the FMAs of d and m and the code conversions), no longer by streaming the
+// weights once per 16 tokens. Graph replays, before -> after: 128 experts of 2048 x 768, 2400 pairs
+// 163 -> 136 us, 4096 pairs 236 -> 194; 16 experts of 1792 x 768 with a shared expert, 1024 pairs
+// 105 -> 67, 3912 pairs 346 -> 151. One row group per down workgroup: 154 at 2400 pairs;
+// resident workgroups walking runs of items (routing once each): 130 to 164 there, slower
+// below; accumulators kept out of the AGPRs: 139.
+// ---------------------------------------------------------------------------
+constexpr int kManyPerExpert = 12;
+constexpr int kManyExperts = kMaxPairs / kManyPerExpert;   // P > kManyPerExpert E: fewer experts than this
+constexpr int kChunk = 32;
+constexpr int kManyDnGroups = 2;
+
+// Item a of the list (experts ascending, each with ceil(pairs / kChunk) chunks): its expert and
+// chunk, {-1, 0} past the end. Every thread of the workgroup calls it (barriers inside). The
+// ids are left in sids (LDS) for collect_pairs.
+template <int WAVES>
+__device__ __forceinline__ int2 many_item(const int32_t* __restrict__ ids, int P, int E, int a, int* sids) {
+    constexpr int kR = 8, NT = 64 * WAVES, kPer = (kManyExperts + NT - 1) / NT;
+    __shared__ int hist[kManyExperts];
+    __shared__ int wsum[WAVES];
+    __shared__ int found_e, found_c;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int e = tid; e < E; e += NT) hist[e] = 0;
+    if (tid == 0) found_e = -1, found_c = 0;
+    __syncthreads();
+    for (int p0 = 0; p0 < P; p0 += NT * kR) {
+        int ev[kR];
+#pragma unroll
+        for (int j = 0; j < kR; ++j) {
+            const int p = p0 + tid + NT * j;
+            ev[j] = p < P ? ids[p] : -1;
+        }
+#pragma unroll
+        for (int j = 0; j < kR; ++j) {
+            const int p = p0 + tid + NT * j;
+            if (p < P) sids[p] = ev[j];
+            if (ev[j] >= 0 && ev[j] < E) atomicAdd(&hist[ev[j]], 1);
+        }
+    }
+    __syncthreads();
+    int n[kPer], c = 0;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int e = tid * kPer + j;
+        n[j] = e < E ? (hist[e] + kChunk - 1) / kChunk : 0;
+        c += n[j];
+    }
+    int incl = c;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(incl, o);
+        if (lane >= o) incl += v;
+    }
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    int at = incl - c;
+    for (int i = 0; i < wave; ++i) at += wsum[i];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        if (a >= at && a < at + n[j]) found_e = tid * kPer + j, found_c = a - at;
+        at += n[j];
+    }
+    __syncthreads();
+    return make_int2(__builtin_amdgcn_readfirstlane(found_e), __builtin_amdgcn_readfirstlane(found_c));
+}
+
+// up_chunk for 17 to 32 tokens
+template <bool XF32, int WAVES, int UNR>
+__device__ __forceinline__ void up_chunk2(const uint8_t* wexp, const void* x, int H, int F, int rgp, const int* rows,
+                                          const int* pairs, int M, float* red, float* __restrict__ hbuf) {
+    float acc[2][2][4][4];
+#pragma unroll
+    for (int i = 0; i < 64; ++i) (&acc[0][0][0][0])[i] = 0.f;
+    const int KB = H >> 5;
+    const uint8_t* const gb[2] = {wexp + (int64_t)(2 * rgp) * KB * kTileBytes,
+                                  wexp + (int64_t)(2 * rgp + 1) * KB * kTileBytes};
+    gemv_rows_pipe_tb2<XF32, 2, UNR, WAVES>(gb, x, GatherRows{rows, M}, H, 0, KB, acc);
+    float (*rd)[4][4][64] = (float (*)[4][4][64])red;
+    const int tid = threadIdx.x, lane = tid & 63, r = tid >> 6, i16 = lane & 15, kg = lane >> 4;
+    const int64_t f = (int64_t)rgp * 64 + r * 16 + i16;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        float vg[4], vu[4];
+        if (b) __syncthreads();
+        wave_sum<4, WAVES>(acc[b][0], rd, vg);
+        __syncthreads();
+        wave_sum<4, WAVES>(acc[b][1], rd, vu);
+        if (r < 4) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int tok = 16 * b + token_of(kg, j);
+                if (tok < M) store_h<true>(hbuf, pairs[tok], F, f, silu(vg[j]) * vu[j]);
+            }
+        }
+    }
+}
+
+// down_chunk for 17 to 32 tokens
+template <int NG, int WAVES, int UNR>
+__device__ __forceinline__ void down_chunk2(const uint8_t* wexp, const float* hbuf, int H, int F, int rg0,
+                                            const int* pairs, int M, float* red, float* __restrict__ ypair) {
+    float acc[2][NG][4][4];
+#pragma unroll
+    for (int i = 0; i < 32 * NG; ++i) (&acc[0][0][0][0])[i] = 0.f;
+    const int KB = F >> 5;
+    const uint8_t* gb[NG];
+#pragma unroll
+    for (int i = 0; i < NG; ++i) gb[i] = wexp + (int64_t)(rg0 + i) * KB * kTileBytes;
+    gemv_rows_pipe_tb2<true, NG, UNR, WAVES, true>(gb, hbuf, GatherRows{pairs, M}, F, 0, KB, acc);
+    float (*rd)[4][4][64] = (float (*)[4][4][64])red;
+    const int tid = threadIdx.x, lane = tid & 63, r = tid >> 6, i16 = lane & 15, kg = lane >> 4;
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int i = 0; i < NG; ++i) {
+            float v[4];
+            if (b || i) __syncthreads();
+            wave_sum<4, WAVES>(acc[b][i], rd, v);
+            const int64_t n = (int64_t)(rg0 + i) * 64 + r * 16 + i16;
+            if (r < 4) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int tok = 16 * b + token_of(kg, j);
+                    if (tok < M) ypair[(int64_t)pairs[tok] * H + n] = v[j];
+                }
+            }
+        }
+}
+
+// Workgroup (item, rgp): gate/up row-group pair rgp for the item's pairs; the shared expert's
+// (token chunk, row-group pair) workgroups come first.
+template <bool XF32>
+__global__ __launch_bounds__(64 * kUpWaves) void moe_up_many_kernel(const uint8_t* __restrict__ gate_up,
+                                                                    const void* __restrict__ x,
+                                                                    const int32_t* __restrict__ ids, int P, int E,
+                                                                    int topk, int H, int F, float* __restrict__ hbuf,
+                                                                    SharedExpert sh) {
+    __shared__ __attribute__((aligned(16))) int sids[kMaxPairs];
+    __shared__ int list[kMaxPairs];
+    __shared__ int rows[kChunk];
+    __shared__ float red[kUpWaves * 4 * 4 * 64];
+    const uint8_t* wexp;
+    const int* pairs;
+    float* out;
+    int rgp, M, Fx;
+    if ((int)blockIdx.x < sh.wgs) {
+        const int fgs = sh.Fs >> 6, c0 = (blockIdx.x / fgs) * kChunk;
+        rgp = blockIdx.x % fgs;
+        M = min(kChunk, sh.T - c0);
+        if (threadIdx.x < kChunk) {
+            rows[threadIdx.x] = c0 + min((int)threadIdx.x, M - 1);
+            list[threadIdx.x] = c0 + threadIdx.x;
+        }
+        wexp = sh.w, pairs = list, out = sh.out, Fx = sh.Fs;
+    } else {
+        const int fg = F >> 6, b = (int)blockIdx.x - sh.wgs;
+        const int2 it = many_item<kUpWaves>(ids, P, E, b / fg, sids);
+        if (it.x < 0) return;
+        rgp = b % fg;
+        const int cnt = collect_pairs_runs<kUpWaves>(sids, P, it.x, list);
+        pairs = list + it.y * kChunk;
+        M = min(kChunk, cnt - it.y * kChunk);
+        if (threadIdx.x < kChunk) rows[threadIdx.x] = pairs[min((int)threadIdx.x, M - 1)] / topk;
+        wexp = gate_up + (int64_t)it.x * (2 * F / 64) * (H / 32) * kTileBytes;
+        out = hbuf, Fx = F;
+    }
+    __syncthreads();
+    wexp = uniform_ptr(wexp);
+    if (M > 16) up_chunk2<XF32, kUpWaves, kUpUnr>(wexp, x, H, Fx, rgp, rows, pairs, M, red, out);
+    else if (M > 8) up_chunk<4, XF32, kUpWaves, kUpUnr, true>(wexp, x, H, Fx, rgp, rows, pairs, M, red, out);
+    else up_chunk<2, XF32, kUpWaves, kUpUnr, true>(wexp, x, H, Fx, rgp, rows, pairs, M, red, out);
+}
+
+// Workgroup (item, g): kManyDnGroups (NG) row groups of H for the item's pairs.
+template <int NG>
+__global__ __launch_bounds__(64 * kDnWaves) void moe_down_many_kernel(const uint8_t* __restrict__ down,
+                                                                      const float* __restrict__ hbuf,
+                                                                      const int32_t* __restrict__ ids, int P, int E,
+                                                                      int H, int F, float* __restrict__ ypair,
+                                                                      SharedExpert sh) {
+    __shared__ __attribute__((aligned(16))) int sids[kMaxPairs];
+    __shared__ int list[kMaxPairs];
+    __shared__ float red[kDnWaves * 4 * 4 * 64];
+    const int wg_per_e = (H >> 6) / NG;
+    const uint8_t* wexp;
+    const float* h;
+    const int* pairs;
+    float* out;
+    int rg0, M, Fx;
+    if ((int)blockIdx.x < sh.wgs) {
+        const int c0 = (blockIdx.x / wg_per_e) * kChunk;
+        rg0 = (blockIdx.x % wg_per_e) * NG;
+        M = min(kChunk, sh.T - c0);
+        if (threadIdx.x < kChunk) list[threadIdx.x] = c0 + threadIdx.x;
+        __syncthreads();
+        wexp = sh.w, h = sh.h, pairs = list, out = sh.out, Fx = sh.Fs;
+    } else {
+        const int b = (int)blockIdx.x - sh.wgs;
+        const int2 it = many_item<kDnWaves>(ids, P, E, b / wg_per_e, sids);
+        if (it.x < 0) return;
+        rg0 = (b % wg_per_e) * NG;
+        const int cnt = collect_pairs_runs<kDnWaves>(sids, P, it.x, list);
+        pairs = list + it.y * kChunk;
+        M = min(kChunk, cnt - it.y * kChunk);
+        wexp = down + (int64_t)it.x * (H / 64) * (F / 32) * kTileBytes;
+        h = hbuf, out = ypair, Fx = F;
+    }
+    wexp = uniform_ptr(wexp);
+    if (M > 16) down_chunk2<NG, kDnWaves, kDnUnr>(wexp, h, H, Fx, rg0, pairs, M, red, out);
+    else if (M > 8) down_chunk<4, NG, kDnWaves, kDnUnr, true>(wexp, h, H, Fx, rg0, pairs, M, red, out);
+    else down_chunk<2, NG, kDnWaves, kDnUnr, true>(wexp, h, H, Fx, rg0, pairs, M, red, out);
 }
 
 // out[t][n..n+3] = sum_j w[t][j] y_pair[t][j][n..n+3], slot order j (H % 4 == 0). Workgroup
@@ -487,53 +725,52 @@ static int moe_impl(const uint8_t* gate_up, const uint8_t* down, const void* x, 
     // Workgroups for every expert that could be routed (at most min(E, P)); those past the
     // routed count leave at once.
     const int64_t routed_max = E < P ? E : P;
-    const int ng = H % (64 * kDnGroups) == 0 ? kDnGroups : 1;
     // At most 2 routed pairs per expert on average (decode batches): the one-accumulator
     // instances, whose lower register use keeps more waves per SIMD. Larger batches stream
-    // each expert's rows once per 16 tokens instead of once per 4.
-    const bool few = P <= 2 * E;
+    // each expert's rows once per 16 tokens instead of once per 4, from kManyPerExpert pairs
+    // per expert on once per 32, the 32s side by side (at 8 pairs per expert
+    // 91 -> 96 us over 128 experts, at 10 102 -> 101, at 12.5 116 -> 109).
+    const bool few = P <= 2 * E, many = P > kManyPerExpert * E;
+    const int ng = many ? (H % (64 * kManyDnGroups) == 0 ? kManyDnGroups : 1)
+                        : H % (64 * kDnGroups) == 0 ? kDnGroups : 1;
+    const int64_t items = many ? routed_max + P / kChunk : routed_max;   // many: chunks, at most one short per expert
     SharedExpert su{}, sd{};
-    if (with_shared) {   // its buffers follow the routed ones; T / (4 MAXNTL) token chunks
-        const int chunks = (int)ceil_div(T, few ? 4 : 16);
+    if (with_shared) {   // its buffers follow the routed ones; T / chunk token chunks
+        const int chunks = (int)ceil_div(T, few ? 4 : many ? kChunk : 16);
         float* hs = (float*)((char*)ypair + align256((size_t)P * H * 4));
         float* ys = (float*)((char*)hs + align256((size_t)T * Fs * 4));
         su = SharedExpert{shared_gu, hs, nullptr, (int)Fs, T, chunks * (int)(Fs / 64)};
         sd = SharedExpert{shared_dn, ys, hs, (int)Fs, T, chunks * (int)(H / (64 * ng))};
         shared = ys;
     }
-    const dim3 gu((unsigned)(su.wgs + routed_max * (F / 64))), dn((unsigned)(sd.wgs + routed_max * (H / (64 * ng))));
+    const dim3 gu((unsigned)(su.wgs + items * (F / 64))), dn((unsigned)(sd.wgs + items * (H / (64 * ng))));
     const dim3 bu(64 * kUpWaves), bd(64 * kDnWaves);
+#define Q4MI_MOE_UP(KERN) \
+    hipLaunchKernelGGL(KERN, gu, bu, 0, st, gate_up, x, topk_ids, P, E, topk, (int)H, (int)F, hbuf, su)
+#define Q4MI_MOE_DOWN(KERN) \
+    hipLaunchKernelGGL(KERN, dn, bd, 0, st, down, hbuf, topk_ids, P, E, (int)H, (int)F, ypair, sd)
     if (x_dtype == Q4MI_F32) {
-        if (few)
-            hipLaunchKernelGGL((moe_up_kernel<true, 1>), gu, bu, 0, st, gate_up, x, topk_ids, P, E, topk, (int)H,
-                               (int)F, hbuf, su);
-        else
-            hipLaunchKernelGGL((moe_up_kernel<true, 4>), gu, bu, 0, st, gate_up, x, topk_ids, P, E, topk, (int)H,
-                               (int)F, hbuf, su);
+        if (few) Q4MI_MOE_UP((moe_up_kernel<true, 1>));
+        else if (many) Q4MI_MOE_UP((moe_up_many_kernel<true>));
+        else Q4MI_MOE_UP((moe_up_kernel<true, 4>));
     } else {
-        if (few)
-            hipLaunchKernelGGL((moe_up_kernel<false, 1>), gu, bu, 0, st, gate_up, x, topk_ids, P, E, topk, (int)H,
-                               (int)F, hbuf, su);
-        else
-            hipLaunchKernelGGL((moe_up_kernel<false, 4>), gu, bu, 0, st, gate_up, x, topk_ids, P, E, topk, (int)H,
-                               (int)F, hbuf, su);
+        if (few) Q4MI_MOE_UP((moe_up_kernel<false, 1>));
+        else if (many) Q4MI_MOE_UP((moe_up_many_kernel<false>));
+        else Q4MI_MOE_UP((moe_up_kernel<false, 4>));
     }
     if (launch_status() != Q4MI_OK) return Q4MI_E_LAUNCH;
-    if (ng == kDnGroups) {
-        if (few)
-            hipLaunchKernelGGL((moe_down_kernel<kDnGroups, 1>), dn, bd, 0, st, down, hbuf, topk_ids, P, E, (int)H,
-                               (int)F, ypair, sd);
-        else
-            hipLaunchKernelGGL((moe_down_kernel<kDnGroups, 4>), dn, bd, 0, st, down, hbuf, topk_ids, P, E, (int)H,
-                               (int)F, ypair, sd);
+    if (many) {
+        if (ng == kManyDnGroups) Q4MI_MOE_DOWN((moe_down_many_kernel<kManyDnGroups>));
+        else Q4MI_MOE_DOWN((moe_down_many_kernel<1>));
+    } else if (ng == kDnGroups) {
+        if (few) Q4MI_MOE_DOWN((moe_down_kernel<kDnGroups, 1>));
+        else Q4MI_MOE_DOWN((moe_down_kernel<kDnGroups, 4>));
     } else {
-        if (few)
-            hipLaunchKernelGGL((moe_down_kernel<1, 1>), dn, bd, 0, st, down, hbuf, topk_ids, P, E, (int)H, (int)F,
-                               ypair, sd);
-        else
-            hipLaunchKernelGGL((moe_down_kernel<1, 4>), dn, bd, 0, st, down, hbuf, topk_ids, P, E, (int)H, (int)F,
-                               ypair, sd);
+        if (few) Q4MI_MOE_DOWN((moe_down_kernel<1, 1>));
+        else Q4MI_MOE_DOWN((moe_down_kernel<1, 4>));
     }
+#undef Q4MI_MOE_UP
+#undef Q4MI_MOE_DOWN
     if (launch_status() != Q4MI_OK) return Q4MI_E_LAUNCH;
     if (fin) {
         const dim3 grid((unsigned)ceil_div(H / 4, 256), (unsigned)T);
