@@ -18,6 +18,7 @@ torch's current stream of the tensors' device.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
 import warnings
 from dataclasses import dataclass, field
@@ -54,7 +55,18 @@ def _device(dev=None) -> torch.device:
 
 
 def _stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    """The handle of torch's current stream on dev. The raw getter, as torch.cuda.current_stream
+    builds a Stream object first (1.9 us against 0.1, twice per call with a cached workspace)."""
+    return torch._C._cuda_getCurrentRawStream(dev.index)
+
+
+_HERE = contextlib.nullcontext()
+
+
+def _on(dev: torch.device):
+    """A context in which dev is the current device: torch.cuda.device(dev) only where it is
+    not already (that guard costs 1.4 us, the question 0.3)."""
+    return _HERE if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
 
 
 def _to_dev(a, dev: torch.device, dtype=None) -> torch.Tensor:
@@ -175,7 +187,7 @@ def pack_q4_1(blocks, device=None, out: torch.Tensor | None = None, scales: str 
     out = _buf(out, "out", torch.uint8, (nbytes,), dev)
     if scales == "fp16" and w != 20:
         raise ValueError("fp16 scales are a Q4_1 mode (Q4_0 has the exact mx0 layout: pack_q4_0_native)")
-    with torch.cuda.device(dev):
+    with _on(dev):
         check("q4_repack", _lib_handle().q4_repack(_ptr(src), w, _ptr(out), n, k, int(scales == "fp16"),
                                                    _stream(dev)))
     return PackedQ4(out[:nbytes], n, k, scales=scales)
@@ -190,7 +202,7 @@ def pack_q4_1_pool(pool, n: int, k: int, rs: int, device=None) -> PackedQ4:
         raise ValueError(f"pool holds {src.numel()} bytes, [{n}, {k}] needs {n * k * 5 // 8}")
     nbytes = packed_bytes(n, k)
     out = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         check("q4_repack_pool", _lib_handle().q4_repack_pool(_ptr(src), rs, _ptr(out), n, k, _stream(dev)))
     return PackedQ4(out, n, k)
 
@@ -209,7 +221,7 @@ def pack_q4_k(blocks, device=None) -> PackedQ4:
     n, nsb, _ = src.shape
     k = nsb * 256
     out = torch.empty(packed_bytes(n, k), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         check("q4_repack_q4k", _lib_handle().q4_repack_q4k(_ptr(src), _ptr(out), n, k, _stream(dev)))
     return PackedQ4(out, n, k)
 
@@ -224,7 +236,7 @@ def pack_q4_k_chunks(chunks, n: int, k: int, rs: int = 1, device=None) -> Packed
     if src.numel() != want:
         raise ValueError(f"Q4_K chunks hold {src.numel()} bytes, [{n}, {k}] needs {want} (4736 B per 32 x 256)")
     out = torch.empty(packed_bytes(n, k), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         check("q4_repack_q4k_chunks",
               _lib_handle().q4_repack_q4k_chunks(_ptr(src), rs, _ptr(out), n, k, _stream(dev)))
     return PackedQ4(out, n, k)
@@ -275,7 +287,7 @@ def pack_q4_k_native(blocks, device=None) -> PackedQ4K:
     n, nsb, _ = src.shape
     k = nsb * 256
     out = torch.empty(q4k_packed_bytes(n, k), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         check("q4_repack_q4k_native", _lib_handle().q4_repack_q4k_native(_ptr(src), _ptr(out), n, k, _stream(dev)))
     return PackedQ4K(out, n, k)
 
@@ -290,7 +302,7 @@ def pack_q4_k_chunks_native(chunks, n: int, k: int, rs: int = 1, device=None) ->
     if src.numel() != want:
         raise ValueError(f"Q4_K chunks hold {src.numel()} bytes, [{n}, {k}] needs {want} (4736 B per 32 x 256)")
     out = torch.empty(q4k_packed_bytes(n, k), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         check("q4_repack_q4k_chunks_native",
               _lib_handle().q4_repack_q4k_chunks_native(_ptr(src), rs, _ptr(out), n, k, _stream(dev)))
     return PackedQ4K(out, n, k)
@@ -300,7 +312,7 @@ def dequant_q4k(w: PackedQ4K, out: torch.Tensor | None = None) -> torch.Tensor:
     """Native Q4_K layout -> f32[n, k], w = fl32(q (d sc) + m mn), bit-exact."""
     dev = w.device
     out = _buf(out, "out", torch.float32, (w.n, w.k), dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         check("q4_dequant_q4k", _lib_handle().q4_dequant_q4k(_ptr(w.data), _ptr(out), w.n, w.k, _stream(dev)))
     return out
 
@@ -323,7 +335,7 @@ def gemm_q4k(w: PackedQ4K, x, y: torch.Tensor | None = None, workspace: torch.Te
                                  or residual.numel() != M * w.n or residual.device != dev):
         raise ValueError(f"residual must be a contiguous float32 [{M}, {w.n}] tensor on {dev}")
     lib = _lib_handle()
-    with torch.cuda.device(dev):
+    with _on(dev):
         wp, wn = _ws_arg(dev, lib.q4_gemv_q4k_workspace_bytes(M, w.n, w.k), "gemv", workspace)
         check("q4_gemv_q4k", lib.q4_gemv_q4k(_ptr(w.data), _ptr(xt), _x_dtype(xt),
                                              None if residual is None else _ptr(residual), _ptr(y), M, w.n, w.k,
@@ -375,7 +387,7 @@ def pack_q8(src, n: int, k: int, fmt: str = "chunks", rs: int = 1, device=None) 
     if t.numel() != want:
         raise ValueError(f"{fmt} source holds {t.numel()} bytes, [{n}, {k}] needs {want}")
     planes = []
-    with torch.cuda.device(dev):
+    with _on(dev):
         for part in (0, 1):
             out = torch.empty(packed_bytes(n, k), dtype=torch.uint8, device=dev)
             check("q4_repack_q8_split", _lib_handle().q4_repack_q8_split(_ptr(t), {"chunks": 0, "q8_0": 1,
@@ -424,7 +436,7 @@ def pack_q8_native(src, n: int, k: int, fmt: str = "chunks", rs: int = 1, device
     if nbytes < 0:
         raise ValueError(f"[{n}, {k}] does not fit the mx8 layout (n % 64 == 0, k % 32 == 0)")
     out = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         check("q4_repack_q8_native", lib.q4_repack_q8_native(_ptr(t), {"chunks": 0, "q8_0": 1, "chunks_f32": 2}[fmt],
                                                              rs, _ptr(out), n, k, _stream(dev)))
     return PackedQ8N(out, n, k)
@@ -434,7 +446,7 @@ def dequant_q8_native(w: PackedQ8N, out: torch.Tensor | None = None) -> torch.Te
     """mx8 -> f32[n, k], w = s * q (exact)."""
     dev = w.device
     out = _buf(out, "out", torch.float32, (w.n, w.k), dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         check("q4_dequant_q8_native", _lib_handle().q4_dequant_q8_native(_ptr(w.data), _ptr(out), w.n, w.k,
                                                                          _stream(dev)))
     return out
@@ -458,7 +470,7 @@ def gemm_q8_native(w: PackedQ8N, x, y: torch.Tensor | None = None, workspace: to
                                  or residual.numel() != M * w.n or residual.device != dev):
         raise ValueError(f"residual must be a contiguous float32 [{M}, {w.n}] tensor on {dev}")
     lib = _lib_handle()
-    with torch.cuda.device(dev):
+    with _on(dev):
         wp, wn = _ws_arg(dev, lib.q4_gemv_q8_native_workspace_bytes(M, w.n, w.k), "gemv", workspace)
         check("q4_gemv_q8_native", lib.q4_gemv_q8_native(_ptr(w.data), _ptr(xt), _x_dtype(xt),
                                                          None if residual is None else _ptr(residual), _ptr(y),
@@ -508,7 +520,7 @@ def pack_q4_0_native(src, n: int, k: int, fmt: str = "q4_0", rs: int = 1, device
     if nbytes < 0:
         raise ValueError(f"[{n}, {k}] does not fit the mx0 layout (n % 64 == 0, k % 32 == 0)")
     out = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         check("q4_repack_q40", lib.q4_repack_q40(_ptr(t), 0 if fmt == "q4_0" else 1, rs, _ptr(out), n, k,
                                                  _stream(dev)))
     return PackedQ40(out, n, k)
@@ -518,7 +530,7 @@ def dequant_q4_0_native(w: PackedQ40, out: torch.Tensor | None = None) -> torch.
     """mx0 -> f32[n, k], w = fl32(q d - 8 d), bit-exact."""
     dev = w.device
     out = _buf(out, "out", torch.float32, (w.n, w.k), dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         check("q4_dequant_q40", _lib_handle().q4_dequant_q40(_ptr(w.data), _ptr(out), w.n, w.k, _stream(dev)))
     return out
 
@@ -542,7 +554,7 @@ def gemm_q4_0_native(w: PackedQ40, x, y: torch.Tensor | None = None, workspace: 
                                  or residual.numel() != M * w.n or residual.device != dev):
         raise ValueError(f"residual must be a contiguous float32 [{M}, {w.n}] tensor on {dev}")
     lib = _lib_handle()
-    with torch.cuda.device(dev):
+    with _on(dev):
         wp, wn = _ws_arg(dev, lib.q4_gemv_workspace_bytes(M, w.n, w.k), "gemv", workspace)
         check("q4_gemv_q40", lib.q4_gemv_q40(_ptr(w.data), _ptr(xt), _x_dtype(xt),
                                              None if residual is None else _ptr(residual), _ptr(y),
@@ -574,7 +586,7 @@ def pack_chunks(chunks, fmt: str, n: int, k: int, rs: int = 1, device=None) -> P
     if src.numel() != want:
         raise ValueError(f"{fmt} chunks hold {src.numel()} bytes, [{n}, {k}] needs {want} ({cb} B per 32 x 256)")
     out = torch.empty(packed_bytes(n, k), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         check(entry, getattr(_lib_handle(), entry)(_ptr(src), rs, _ptr(out), n, k, _stream(dev)))
     return PackedQ4(out, n, k)
 
@@ -584,7 +596,7 @@ def dequant(w: PackedQ4, out: torch.Tensor | None = None) -> torch.Tensor:
     dev = w.device
     out = _buf(out, "out", torch.float32, (w.n, w.k), dev)
     fn = "q4_dequant_fp16s" if w.scales == "fp16" else "q4_dequant"
-    with torch.cuda.device(dev):
+    with _on(dev):
         check(fn, getattr(_lib_handle(), fn)(_ptr(w.data), _ptr(out), w.n, w.k, _stream(dev)))
     return out
 
@@ -608,7 +620,7 @@ def _workspace(dev: torch.device, nbytes: int, op: str) -> torch.Tensor | None:
     (never allocated by the C library itself)."""
     if nbytes == 0:
         return None
-    key = (op, dev.index, torch.cuda.current_stream(dev).cuda_stream)
+    key = (op, dev.index, _stream(dev))
     ws = _WS.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev)
@@ -697,13 +709,13 @@ def gemm_q4(w: PackedQ4, x, y: torch.Tensor | None = None, workspace: torch.Tens
         if residual is not None and (residual.dtype != torch.float32 or not residual.is_contiguous()
                                      or residual.numel() != M * w.n or residual.device != dev):
             raise ValueError(f"residual must be a contiguous float32 [{M}, {w.n}] tensor on {dev}")
-        with torch.cuda.device(dev):
+        with _on(dev):
             wp, wn = _ws_arg(dev, lib.q4_gemv_workspace_bytes(M, w.n, w.k), "gemv", workspace)
             check("q4_gemv_fp16s", lib.q4_gemv_fp16s(_ptr(w.data), _ptr(xt), _x_dtype(xt),
                                                      None if residual is None else _ptr(residual), _ptr(y), M, w.n,
                                                      w.k, wp, wn, _stream(dev)))
         return y
-    with torch.cuda.device(dev):
+    with _on(dev):
         wp, wn = _ws_arg(dev, lib.q4_gemv_workspace_bytes(M, w.n, w.k), "gemv", workspace)
         if residual is None:
             check("q4_gemv", lib.q4_gemv(_ptr(w.data), _ptr(xt), _x_dtype(xt), _ptr(y), M, w.n, w.k, wp, wn,
@@ -735,7 +747,7 @@ def gemm_q8(w: PackedQ8, x, y: torch.Tensor | None = None, workspace: torch.Tens
                                  or residual.numel() != M * w.n or residual.device != dev):
         raise ValueError(f"residual must be a contiguous float32 [{M}, {w.n}] tensor on {dev}")
     lib = _lib_handle()
-    with torch.cuda.device(dev):
+    with _on(dev):
         wp, wn = _ws_arg(dev, lib.q4_gemv_workspace_bytes(M, w.n, w.k), "gemv", workspace)
         check("q4_gemv_q8", lib.q4_gemv_q8(_ptr(w.hi.data), _ptr(w.lo.data), _ptr(xt), _x_dtype(xt),
                                            None if residual is None else _ptr(residual), _ptr(y), M, w.n, w.k,
@@ -786,7 +798,7 @@ def gemm_q4_rmsnorm(w: PackedQ4, x: torch.Tensor, norm_w: torch.Tensor, eps: flo
     wt, wd = _norm_w(norm_w, w.k, dev)
     y = _buf(y, "y", torch.float32, (M, w.n), dev)
     lib = _lib_handle()
-    with torch.cuda.device(dev):
+    with _on(dev):
         wp, wn = _ws_arg(dev, _norm_ws_bytes(lib, M, w, workspace), "gemv", workspace)
         check("q4_gemv_rmsnorm", lib.q4_gemv_rmsnorm(_ptr(w.data), _ptr(xt), _ptr(wt), wd, float(eps), _ptr(y),
                                                      M, w.n, w.k, wp, wn, _stream(dev)))
@@ -820,7 +832,7 @@ def gemm_q4_partials(w: PackedQ4, x, splits: int | None = None, part: torch.Tens
         raise ValueError(f"splits must be 1..{min(16, w.k // 32)}, got {S}")
     part = _buf(part, "part", torch.float32, (S, M, w.n), dev)
     lib = _lib_handle()
-    with torch.cuda.device(dev):
+    with _on(dev):
         check("q4_gemv_partials", lib.q4_gemv_partials(_ptr(w.data), _ptr(xt), _x_dtype(xt), _ptr(part), S, M, w.n,
                                                        w.k, _stream(dev)))
     return part
@@ -861,7 +873,7 @@ def gemm_q4_rmsnorm_acc(w: PackedQ4, res: torch.Tensor, partials: torch.Tensor |
     wt, wd = _norm_w(norm_w, w.k, dev)
     y = _buf(y, "y", torch.float32, (M, w.n), dev)
     lib = _lib_handle()
-    with torch.cuda.device(dev):
+    with _on(dev):
         wp, wn = _ws_arg(dev, _norm_ws_bytes(lib, M, w, workspace), "gemv", workspace)
         check("q4_gemv_rmsnorm_acc", lib.q4_gemv_rmsnorm_acc(_ptr(w.data), _ptr(xt), pp, S, _ptr(wt), wd, float(eps),
                                                              _ptr(x_out), _ptr(y), M, w.n, w.k, wp, wn,
@@ -886,7 +898,7 @@ def swiglu_q4_acc(gate: PackedQ4, up: PackedQ4, res: torch.Tensor, partials: tor
     wt, wd = _norm_w(norm_w, gate.k, dev)
     h = _buf(h, "h", out_dtype, (M, gate.n), dev)
     lib = _lib_handle()
-    with torch.cuda.device(dev):
+    with _on(dev):
         wp, wn = _ws_arg(dev, lib.q4_gemv_swiglu_workspace_bytes(M, gate.n, gate.k), "swiglu", workspace)
         check("q4_gemv_swiglu_rmsnorm_acc", lib.q4_gemv_swiglu_rmsnorm_acc(
             _ptr(gate.data), _ptr(up.data), _ptr(xt), pp, S, _ptr(wt), wd, float(eps), _ptr(x_out), _ptr(h),
@@ -916,7 +928,7 @@ def swiglu_q4(gate: PackedQ4, up: PackedQ4, x, out_dtype=torch.float32, h: torch
             raise TypeError("out_dtype must be float32 or bfloat16")
         h = _buf(h, "h", out_dtype, (M, gate.n), dev)
         lib = _lib_handle()
-        with torch.cuda.device(dev):
+        with _on(dev):
             wp, wn = _ws_arg(dev, lib.q4_gemv_swiglu_workspace_bytes(M, gate.n, gate.k), "swiglu", workspace)
             check("q4_gemv_swiglu_rmsnorm", lib.q4_gemv_swiglu_rmsnorm(
                 _ptr(gate.data), _ptr(up.data), _ptr(xt), _ptr(wt), wd, float(eps), _ptr(h),
@@ -932,7 +944,7 @@ def swiglu_q4(gate: PackedQ4, up: PackedQ4, x, out_dtype=torch.float32, h: torch
         raise TypeError("out_dtype must be float32 or bfloat16")
     h = _buf(h, "h", out_dtype, (M, gate.n), dev)
     lib = _lib_handle()
-    with torch.cuda.device(dev):
+    with _on(dev):
         wp, wn = _ws_arg(dev, lib.q4_gemv_swiglu_workspace_bytes(M, gate.n, gate.k), "swiglu", workspace)
         check("q4_gemv_swiglu", lib.q4_gemv_swiglu(_ptr(gate.data), _ptr(up.data), _ptr(xt), _x_dtype(xt), _ptr(h),
                                                    Q4MI_BF16 if out_dtype == torch.bfloat16 else Q4MI_F32, M,
@@ -1010,7 +1022,7 @@ def decode_segment(o: PackedQ4, gate: PackedQ4, up: PackedQ4, down: PackedQ4, qk
     if workspace is None:
         workspace = decode_segment_workspace(H, F, NQ, dev)
     lib = _lib_handle()
-    with torch.cuda.device(dev):
+    with _on(dev):
         wp, wn = _ws_arg(dev, lib.q4_decode_segment_workspace_bytes(H, F, NQ), "decode_segment", workspace)
         opt = lambda t: None if t is None else _ptr(t)
         check("q4_decode_segment", lib.q4_decode_segment(
@@ -1044,7 +1056,7 @@ def rmsnorm_add(x: torch.Tensor, w: torch.Tensor, add: torch.Tensor | None = Non
     xn = _buf(xn, "xn", out_dtype if xn is None else xn.dtype, tuple(x.shape), dev)
     if xn.dtype not in (torch.float32, torch.bfloat16):
         raise TypeError(f"xn must be float32 or bfloat16, got {xn.dtype}")
-    with torch.cuda.device(dev):
+    with _on(dev):
         check("q4_rmsnorm_add", _lib_handle().q4_rmsnorm_add(
             _ptr(x), None if add is None else _ptr(add), _ptr(wt), Q4MI_BF16 if wt.dtype == torch.bfloat16 else Q4MI_F32,
             None if y is None else _ptr(y), _ptr(xn), Q4MI_BF16 if xn.dtype == torch.bfloat16 else Q4MI_F32, M, N,
@@ -1104,7 +1116,7 @@ def logits_topk(logits: torch.Tensor, k: int = 1, mode: str = "sampler", n_valid
     dev = lg.device
     ids, vals = _topk_outputs(M, k, dev, ids, vals)
     lib = _lib_handle()
-    with torch.cuda.device(dev):
+    with _on(dev):
         wp, wn = _ws_arg(dev, lib.q4_topk_workspace_bytes(M, n, k), "topk", workspace)
         check("q4_logits_topk", lib.q4_logits_topk(_ptr(lg), lg.stride(0), M, n, k, _topk_mode(mode),
                                                    _ptr(ids), _ptr(vals), wp, wn, _stream(dev)))
@@ -1131,7 +1143,7 @@ def lm_head_topk(w: PackedQ4, x, k: int = 1, mode: str = "sampler", n_valid: int
     logits = _buf(logits, "logits", torch.float32, (M, w.n), dev)
     ids, vals = _topk_outputs(M, k, dev, ids, vals)
     lib = _lib_handle()
-    with torch.cuda.device(dev):
+    with _on(dev):
         wp, wn = _ws_arg(dev, lib.q4_lm_head_workspace_bytes(M, w.n, w.k, k), "lm_head", workspace)
         check("q4_lm_head_topk", lib.q4_lm_head_topk(_ptr(w.data), _ptr(xt), _x_dtype(xt), _ptr(logits), M, w.n,
                                                      w.k, n, k, _topk_mode(mode), _ptr(ids), _ptr(vals), wp, wn,
@@ -1189,7 +1201,7 @@ class GemvGroup:
 
     def run(self) -> None:
         fn = "q4_gemv_grouped_fp16s" if self.scales == "fp16" else "q4_gemv_grouped"
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             check(fn, getattr(_lib_handle(), fn)(
                 _ptr(self.table), self.count, self.total_items, self.M, self.x_dtype, _stream(self.device)))
 
@@ -1213,7 +1225,7 @@ def prefill_scales(w) -> torch.Tensor:
         n = w.n * w.experts if isinstance(w, PackedExperts) else w.n
         lib = _lib_handle()
         t = torch.empty(int(lib.q4_prefill_scales_bytes(n, w.k)), dtype=torch.uint8, device=dev)
-        with torch.cuda.device(dev):
+        with _on(dev):
             check("q4_prefill_scales", lib.q4_prefill_scales(_ptr(w.data), n, w.k, _ptr(t), t.numel(), _stream(dev)))
         w.prefill_scales = t
     return w.prefill_scales
@@ -1247,7 +1259,7 @@ def prefill_prepare(x, precision: str = "fp16", out: torch.Tensor | None = None)
         raise ValueError(f"[{T}, {K}] cannot be prepared (K % 32 == 0)")
     data = _buf(out, "out", torch.uint8, (nbytes,), dev)
     if T:
-        with torch.cuda.device(dev):
+        with _on(dev):
             check("q4_prefill_prepare", lib.q4_prefill_prepare(_ptr(xt), _x_dtype(xt), T, K, _PRECISION[precision],
                                                                _ptr(data), nbytes, _stream(dev)))
     return PreparedActs(data, T, K, _x_dtype(xt), precision)
@@ -1287,7 +1299,7 @@ def rmsnorm_prepare(x: torch.Tensor, w: torch.Tensor, add: torch.Tensor | None =
     nbytes = int(lib.q4_prefill_prepared_bytes(T, K, Q4MI_BF16, _PRECISION[precision])) if T else 0
     data = _buf(out, "out", torch.uint8, (nbytes,), dev)
     if T:
-        with torch.cuda.device(dev):
+        with _on(dev):
             check("q4_rmsnorm_prepare", lib.q4_rmsnorm_prepare(
                 _ptr(x), None if add is None else _ptr(add), planes, _ptr(wt),
                 Q4MI_BF16 if wt.dtype == torch.bfloat16 else Q4MI_F32, None if y is None else _ptr(y), T, K,
@@ -1326,7 +1338,7 @@ def swiglu_prepare(g: torch.Tensor, u: torch.Tensor | None = None, precision: st
     nbytes = int(lib.q4_prefill_prepared_bytes(T, F, Q4MI_BF16, _PRECISION[precision])) if T else 0
     data = _buf(out, "out", torch.uint8, (nbytes,), dev)
     if T:
-        with torch.cuda.device(dev):
+        with _on(dev):
             check("q4_swiglu_prepare", lib.q4_swiglu_prepare(
                 _ptr(g), _ptr(u), g.stride(0), u.stride(0), T, F, _PRECISION[precision],
                 None if h is None else _ptr(h), _ptr(data), nbytes, _stream(dev)))
@@ -1373,7 +1385,7 @@ def gemm_q4_prefill_swiglu(gate_up: PackedQ4, x, h: torch.Tensor | None = None,
     h = _buf(h, "h", torch.bfloat16, (T, F), dev)
     sc = prefill_scales(gate_up) if precision == "fp16" else None
     if T:
-        with torch.cuda.device(dev):
+        with _on(dev):
             check("q4_gemm_prefill_swiglu", _lib_handle().q4_gemm_prefill_swiglu(
                 _ptr(gate_up.data), None if sc is None else _ptr(sc), _ptr(prep.data), prep.x_dtype, _ptr(h), T, F,
                 gate_up.k, _PRECISION[precision], _stream(dev)))
@@ -1398,7 +1410,7 @@ def gemm_q4_prefill_partials(w: PackedQ4, x: PreparedActs, part: torch.Tensor | 
     part = _buf(part, "part", torch.float32, (S, x.t, w.n), dev)
     sc = prefill_scales(w) if x.precision == "fp16" else None
     if x.t:
-        with torch.cuda.device(dev):
+        with _on(dev):
             check("q4_gemm_prefill_prepared_partials", lib.q4_gemm_prefill_prepared_partials(
                 _ptr(w.data), None if sc is None else _ptr(sc), _ptr(x.data), x.x_dtype, _ptr(part),
                 part.numel() * 4, x.t, w.n, w.k, _PRECISION[x.precision], _stream(dev)))
@@ -1426,7 +1438,7 @@ def gemm_q4_prefill(w: PackedQ4, x, y: torch.Tensor | None = None, precision: st
             return y
         lib = _lib_handle()
         sc = prefill_scales(w) if x.precision == "fp16" else None
-        with torch.cuda.device(dev):
+        with _on(dev):
             wp, wn = _ws_arg(dev, lib.q4_gemm_prefill_prepared_workspace_bytes(T, w.n, w.k), "prefill", workspace)
             check("q4_gemm_prefill_prepared", lib.q4_gemm_prefill_prepared(
                 _ptr(w.data), None if sc is None else _ptr(sc), _ptr(x.data), x.x_dtype, _ptr(y), T, w.n, w.k, prec,
@@ -1442,12 +1454,12 @@ def gemm_q4_prefill(w: PackedQ4, x, y: torch.Tensor | None = None, precision: st
     lib = _lib_handle()
     if precision == "fp16" and T > 0 and w.n > 0:
         sc = prefill_scales(w)
-        with torch.cuda.device(dev):
+        with _on(dev):
             wp, wn = _ws_arg(dev, lib.q4_gemm_prefill_scaled_workspace_bytes(T, w.n, w.k), "prefill", workspace)
             check("q4_gemm_prefill_scaled", lib.q4_gemm_prefill_scaled(
                 _ptr(w.data), _ptr(sc), _ptr(xt), _x_dtype(xt), _ptr(y), T, w.n, w.k, wp, wn, _stream(dev)))
         return y
-    with torch.cuda.device(dev):
+    with _on(dev):
         wp, wn = _ws_arg(dev, lib.q4_gemm_prefill_workspace_bytes(T, w.n, w.k), "prefill", workspace)
         check("q4_gemm_prefill", lib.q4_gemm_prefill(
             _ptr(w.data), _ptr(xt), _x_dtype(xt), _ptr(y), T, w.n, w.k, _PRECISION[precision], wp, wn,
@@ -1579,7 +1591,7 @@ def moe_batch(gate_up: PackedExperts, down: PackedExperts, x, topk_ids, topk_w,
         if T == 0:
             return out
         sc = (prefill_scales(gate_up), prefill_scales(down)) if precision == "fp16" else (None, None)
-        with torch.cuda.device(dev):
+        with _on(dev):
             wp, wn = _ws_arg(dev, lib.q4_moe_prefill_workspace_bytes(T, E, topk, H, F), "moe_prefill", workspace)
             check("q4_moe_prefill", lib.q4_moe_prefill(
                 _ptr(gate_up.data), _ptr(down.data), None if sc[0] is None else _ptr(sc[0]),
@@ -1590,14 +1602,14 @@ def moe_batch(gate_up: PackedExperts, down: PackedExperts, x, topk_ids, topk_w,
     if shared_expert is not None:
         sgu, sdn = shared_expert
         Fs = sgu.n // 2
-        with torch.cuda.device(dev):
+        with _on(dev):
             wp, wn = _ws_arg(dev, lib.q4_moe_shared_workspace_bytes(T, E, topk, H, F, Fs), "moe", workspace)
             check("q4_moe_gemv_shared", lib.q4_moe_gemv_shared(
                 _ptr(gate_up.data), _ptr(down.data), _ptr(sgu.data), _ptr(sdn.data), Fs, _ptr(sgw), _ptr(xt),
                 _x_dtype(xt), _ptr(ids), _ptr(wts), None if residual is None else _ptr(residual), _ptr(out),
                 T, E, topk, H, F, wp, wn, _stream(dev)))
         return out
-    with torch.cuda.device(dev):
+    with _on(dev):
         wp, wn = _ws_arg(dev, lib.q4_moe_workspace_bytes(T, E, topk, H, F), "moe", workspace)
         if residual is None and shared is None:
             check("q4_moe_gemv", lib.q4_moe_gemv(
