@@ -631,6 +631,31 @@ __global__ __launch_bounds__(512) void prefill_dma_kernel(const uint8_t* __restr
                                          : wide + xcd_group((int)blockIdx.x - wide, G - wide);
     if (!MIXED || b < wide_wgs) {
         const int tile = b / splits;
+        dma_tile<PREC, 2, 8, 4>(lds, packed, x16, texp, wexp, s16, y, T, N, K, (tile / tiles_t) * 256,
+                                (tile % tiles_t) * 256, b % splits, splits, accum);
+    } else {
+        const int i = b - wide_wgs, tile = i / splits;
+        dma_tile<PREC, 2, 6, 4>(lds, packed, x16, texp, wexp, s16, y, T, N, K, narrow_row0 + (tile / tiles_t) * 192,
+                                (tile % tiles_t) * 256, i % splits, splits, accum);
+    }
+}
+
+// prefill_dma_kernel for a last token tile of at most 192 tokens: each tile runs the instance
+// for its valid 64-token groups.
+template <int PREC, bool MIXED>
+__global__ __launch_bounds__(512) void prefill_ragged_kernel(const uint8_t* __restrict__ packed,
+                                                             const uint16_t* __restrict__ x16,
+                                                             const int* __restrict__ texp,
+                                                             const int* __restrict__ wexp,
+                                                             const uint32_t* __restrict__ s16, float* __restrict__ y,
+                                                             int T, int N, int K, int tiles_t, int splits,
+                                                             int wide_wgs, int narrow_row0, int accum) {
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[5 * kTileB];
+    const int G = (int)gridDim.x, wide = MIXED ? wide_wgs : G;
+    const int b = (int)blockIdx.x < wide ? xcd_group((int)blockIdx.x, wide)
+                                         : wide + xcd_group((int)blockIdx.x - wide, G - wide);
+    if (!MIXED || b < wide_wgs) {
+        const int tile = b / splits;
         dma_tile_valid<PREC, 2, 8, 4>(lds, packed, x16, texp, wexp, s16, y, T, N, K, (tile / tiles_t) * 256,
                                       (tile % tiles_t) * 256, b % splits, splits, accum);
     } else {
@@ -660,10 +685,9 @@ __global__ __launch_bounds__(512) void prefill_dma128_kernel(const uint8_t* __re
                                   (tile % tiles_t) * 128, b % splits, splits, accum);
 }
 
-// The gate/up GEMM with the SwiGLU epilogue: workgroup b takes the row tile of pair rows
-// (b / tiles_t) and token tile b % tiles_t over all of K (no split), writing h. KBS = 2: 256 x
-// 256 tiles, KBS = 4: 128 x 128.
-template <int PREC, int KBS>
+// The gate/up GEMM with the SwiGLU epilogue: workgroup b takes the 256-row tile of pair rows
+// (b / tiles_t) * 256 and token tile b % tiles_t over all of K (no split), writing h.
+template <int PREC>
 __global__ __launch_bounds__(512) void prefill_swiglu_kernel(const uint8_t* __restrict__ packed,
                                                              const uint16_t* __restrict__ x16,
                                                              const int* __restrict__ texp,
@@ -673,10 +697,28 @@ __global__ __launch_bounds__(512) void prefill_swiglu_kernel(const uint8_t* __re
                                                              int tiles_t) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[5 * kTileB];
     const int b = xcd_group((int)blockIdx.x, (int)gridDim.x);
+    dma_tile<PREC, 2, 8, 4, true>(lds, packed, x16, texp, wexp, s16, (float*)h, T, N, K, (b / tiles_t) * 256,
+                                  (b % tiles_t) * 256, 0, 1, 0);
+}
+
+// The same for a last token tile of at most 192 tokens (KBS = 2), or in 128 x 128 tiles (KBS = 4).
+template <int PREC, int KBS>
+__global__ __launch_bounds__(512) void prefill_swiglu_ragged_kernel(const uint8_t* __restrict__ packed,
+                                                                    const uint16_t* __restrict__ x16,
+                                                                    const int* __restrict__ texp,
+                                                                    const int* __restrict__ wexp,
+                                                                    const uint32_t* __restrict__ s16,
+                                                                    uint16_t* __restrict__ h, int T, int N, int K,
+                                                                    int tiles_t) {
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[5 * kTileB];
+    const int b = xcd_group((int)blockIdx.x, (int)gridDim.x);
     constexpr int R = 512 / KBS;
     dma_tile_valid<PREC, KBS, 16 / KBS, 8 / KBS, true>(lds, packed, x16, texp, wexp, s16, (float*)h, T, N, K,
                                                        (b / tiles_t) * R, (b % tiles_t) * R, 0, 1, 0);
 }
+
+// Whether the last 256-token tile leaves a 64-token group or more over.
+bool ragged_tokens(int T) { return T % 256 != 0 && T % 256 <= 192; }
 
 // The exponent that puts a positive finite magnitude v in [2^14, 2^15) after scaling by
 // 2^-e: v in [2^(x-1), 2^x) -> e = x - 15. 0 for zero, inf and NaN (those are passed
@@ -1097,12 +1139,17 @@ void launch_prefill(int cfg, int64_t grid, hipStream_t st, const uint8_t* w, con
                                s16, y, T, N, K, tiles_t, splits, accum);
             break;
         default:
-            if (wide_wgs < grid)
-                hipLaunchKernelGGL((prefill_dma_kernel<PREC, true>), dim3((unsigned)grid), dim3(512), 0, st, w, x16, te,
-                                   we, s16, y, T, N, K, tiles_t, splits, wide_wgs, narrow_row0, accum);
-            else
-                hipLaunchKernelGGL((prefill_dma_kernel<PREC, false>), dim3((unsigned)grid), dim3(512), 0, st, w, x16, te,
-                                   we, s16, y, T, N, K, tiles_t, splits, wide_wgs, narrow_row0, accum);
+#define Q4MI_DMA(KERN)                                                                                              \
+    hipLaunchKernelGGL(KERN, dim3((unsigned)grid), dim3(512), 0, st, w, x16, te, we, s16, y, T, N, K, tiles_t, splits, \
+                       wide_wgs, narrow_row0, accum)
+            if (ragged_tokens(T)) {
+                if (wide_wgs < grid) Q4MI_DMA((prefill_ragged_kernel<PREC, true>));
+                else Q4MI_DMA((prefill_ragged_kernel<PREC, false>));
+            } else {
+                if (wide_wgs < grid) Q4MI_DMA((prefill_dma_kernel<PREC, true>));
+                else Q4MI_DMA((prefill_dma_kernel<PREC, false>));
+            }
+#undef Q4MI_DMA
             break;
     }
 }
@@ -1608,11 +1655,18 @@ extern "C" int q4_gemm_prefill_swiglu(const uint8_t* gate_up, const void* scales
     const int tile = t128 ? 128 : 256, tiles_t = (int)ceil_div(T, tile);
     const dim3 grid((unsigned)((N / tile) * tiles_t)), block(512);
     const hipStream_t st = (hipStream_t)stream;
-#define Q4MI_SG(PR, KBS)                                                                                              \
-    hipLaunchKernelGGL((prefill_swiglu_kernel<PR, KBS>), grid, block, 0, st, gate_up, (const uint16_t*)prepared, te, we, \
-                       s16, (uint16_t*)h, T, (int)N, (int)K, tiles_t)
-    if (precision == 0) { if (t128) Q4MI_SG(0, 4); else Q4MI_SG(0, 2); }
-    else { if (t128) Q4MI_SG(1, 4); else Q4MI_SG(1, 2); }
+#define Q4MI_SG(KERN)                                                                                            \
+    hipLaunchKernelGGL(KERN, grid, block, 0, st, gate_up, (const uint16_t*)prepared, te, we, s16, (uint16_t*)h, T, \
+                       (int)N, (int)K, tiles_t)
+#define Q4MI_SG_FORM(PR)                                                    \
+    do {                                                                    \
+        if (t128) Q4MI_SG((prefill_swiglu_ragged_kernel<PR, 4>));           \
+        else if (ragged_tokens(T)) Q4MI_SG((prefill_swiglu_ragged_kernel<PR, 2>)); \
+        else Q4MI_SG((prefill_swiglu_kernel<PR>));                          \
+    } while (0)
+    if (precision == 0) Q4MI_SG_FORM(0);
+    else Q4MI_SG_FORM(1);
+#undef Q4MI_SG_FORM
 #undef Q4MI_SG
     return launch_status();
 }
@@ -1963,21 +2017,57 @@ __global__ __launch_bounds__(256) void moe_h16prep_kernel(const uint16_t* __rest
 // is row-major ([rows][K]), slot s's row gmap[s] (gmap null: row s).
 template <int PREC, bool SWI = false, bool GATHER = false>
 __global__ __launch_bounds__(512) void moe_dma_kernel(const uint8_t* __restrict__ packed, int64_t ebytes,
-                                                      const uint16_t* __restrict__ x16,
-                                                      const int* __restrict__ texp, const int* __restrict__ wexp,
-                                                      const uint32_t* __restrict__ s16, int64_t s16_words,
-                                                      float* __restrict__ y, const int* __restrict__ tile_e,
-                                                      const int* __restrict__ tile_end, const int* __restrict__ meta,
-                                                      int N, int K, int tiles_n, int accum,
-                                                      const int* __restrict__ gmap = nullptr) {
+                                                      const uint16_t* __restrict__ x16, const int* __restrict__ texp,
+                                                      const int* __restrict__ wexp, const uint32_t* __restrict__ s16,
+                                                      int64_t s16_words, float* __restrict__ y,
+                                                      const int* __restrict__ tile_e, const int* __restrict__ tile_end,
+                                                      const int* __restrict__ meta, int N, int K, int tiles_n, int accum,
+                                                      const int* __restrict__ gmap) {
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[5 * kTileB];
+    const int b = blockIdx.x, tt = b / tiles_n, rt = b % tiles_n;
+    if (tt >= meta[0]) return;
+    const int e = tile_e[tt];
+    dma_tile<PREC, 2, 8, 4, SWI, GATHER>(lds, packed + e * ebytes, x16, texp,
+                                 PREC == 0 ? wexp + (int64_t)e * N : nullptr,
+                                 PREC == 0 ? s16 + e * s16_words : nullptr, y, tile_end[tt], N, K, rt * 256, tt * 256,
+                                 0, 1, accum, gmap);
+}
+
+// The same with each tile's work sized by its valid 64-slot groups.
+template <int PREC, bool SWI = false, bool GATHER = false>
+__global__ __launch_bounds__(512) void moe_ragged_kernel(const uint8_t* __restrict__ packed, int64_t ebytes,
+                                                         const uint16_t* __restrict__ x16, const int* __restrict__ texp,
+                                                         const int* __restrict__ wexp, const uint32_t* __restrict__ s16,
+                                                         int64_t s16_words, float* __restrict__ y,
+                                                         const int* __restrict__ tile_e, const int* __restrict__ tile_end,
+                                                         const int* __restrict__ meta, int N, int K, int tiles_n, int accum,
+                                                         const int* __restrict__ gmap) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[5 * kTileB];
     const int b = blockIdx.x, tt = b / tiles_n, rt = b % tiles_n;
     if (tt >= meta[0]) return;
     const int e = tile_e[tt];
     dma_tile_valid<PREC, 2, 8, 4, SWI, GATHER>(lds, packed + e * ebytes, x16, texp,
-                                               PREC == 0 ? wexp + (int64_t)e * N : nullptr,
-                                               PREC == 0 ? s16 + e * s16_words : nullptr, y, tile_end[tt], N, K,
-                                               rt * 256, tt * 256, 0, 1, accum, gmap);
+                                 PREC == 0 ? wexp + (int64_t)e * N : nullptr,
+                                 PREC == 0 ? s16 + e * s16_words : nullptr, y, tile_end[tt], N, K, rt * 256, tt * 256,
+                                 0, 1, accum, gmap);
+}
+
+// The grouped expert GEMM of a launch: one ragged tile per expert, so up to kMoeFullTiles tiles per
+// expert on average the kernel whose tiles follow their valid slots (128 experts, top-8 of
+// 2048 tokens, 128 of a tile's 256 slots valid: gate/up 191 -> 165 us, down 147 -> 118), beyond
+// that the one-body kernel, where at most 1 / kMoeFullTiles of the tiles could gain.
+constexpr int kMoeFullTiles = 16;
+template <int PREC, bool SWI = false, bool GATHER = false>
+void launch_moe_dma(bool ragged, unsigned grid, hipStream_t st, const uint8_t* packed, int64_t ebytes,
+                    const uint16_t* x16, const int* texp, const int* wexp, const uint32_t* s16, int64_t s16_words,
+                    float* y, const int* tile_e, const int* tile_end, const int* meta, int N, int K, int tiles_n,
+                    int accum, const int* gmap = nullptr) {
+    if (ragged)
+        hipLaunchKernelGGL((moe_ragged_kernel<PREC, SWI, GATHER>), dim3(grid), dim3(512), 0, st, packed, ebytes, x16,
+                           texp, wexp, s16, s16_words, y, tile_e, tile_end, meta, N, K, tiles_n, accum, gmap);
+    else
+        hipLaunchKernelGGL((moe_dma_kernel<PREC, SWI, GATHER>), dim3(grid), dim3(512), 0, st, packed, ebytes, x16,
+                           texp, wexp, s16, s16_words, y, tile_e, tile_end, meta, N, K, tiles_n, accum, gmap);
 }
 
 // out[t][n..n+3] = sum_j w[t][j] Y[slot(t, j)][n..n+3], slot order j.
@@ -2091,6 +2181,7 @@ extern "C" int q4_moe_prefill(const uint8_t* gate_up, const uint8_t* down, const
     const hipStream_t st = (hipStream_t)stream;
     const unsigned S = (unsigned)(w.tiles_max * 256), SP = S / 4;
     const bool xf32 = x_dtype == Q4MI_F32;
+    const bool ragged = P < (int64_t)256 * kMoeFullTiles * E;
 
     hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(1024), 0, st, topk_ids, P, E, cnt, off, tile_e, tile_end, meta);
     if (launch_status() != Q4MI_OK) return Q4MI_E_LAUNCH;
@@ -2117,11 +2208,11 @@ extern "C" int q4_moe_prefill(const uint8_t* gate_up, const uint8_t* down, const
     const bool gather = precision == 1 && !xf32 && (uint64_t)T * H * 2 <= 0xffffffffull &&
                         (uint64_t)S * F * 2 <= 0xffffffffull;
     if (gather) {
-        hipLaunchKernelGGL((moe_dma_kernel<1, true, true>), dim3(g1), dim3(512), 0, st, gate_up, eb1,
+        launch_moe_dma<1, true, true>(ragged, g1, st, gate_up, eb1,
                            (const uint16_t*)x, texp, we1, s1, sw1, (float*)x16, tile_e, tile_end, meta, (int)N1,
                            (int)H, (int)(N1 / 256), 0, (const int*)rowmap);
         if (launch_status() != Q4MI_OK) return Q4MI_E_LAUNCH;
-        hipLaunchKernelGGL((moe_dma_kernel<1, false, true>), dim3(g2), dim3(512), 0, st, down, eb2, x16, texp, we2, s2,
+        launch_moe_dma<1, false, true>(ragged, g2, st, down, eb2, x16, texp, we2, s2,
                            sw2, gy, tile_e, tile_end, meta, (int)N2, (int)F, (int)(N2 / 256), 0, (const int*)nullptr);
         if (launch_status() != Q4MI_OK) return Q4MI_E_LAUNCH;
         hipLaunchKernelGGL(moe_prefill_combine_kernel, dim3((unsigned)ceil_div(H / 4, 256), (unsigned)T), dim3(256), 0,
@@ -2157,24 +2248,24 @@ extern "C" int q4_moe_prefill(const uint8_t* gate_up, const uint8_t* down, const
         // bf16 h from one activation pass: SwiGLU in the gate/up epilogue, h [S][F] bf16 in
         // the G/Y buffer (G itself is never written)
         if (swi && gx)
-            hipLaunchKernelGGL((moe_dma_kernel<0, true, true>), dim3(g1), dim3(512), 0, st, gate_up, eb1, x16, texp,
+            launch_moe_dma<0, true, true>(ragged, g1, st, gate_up, eb1, x16, texp,
                                we1, s1, sw1, gy, tile_e, tile_end, meta, (int)N1, (int)H, (int)(N1 / 256), 0,
                                (const int*)rowmap);
         else if (swi && precision == 0)
-            hipLaunchKernelGGL((moe_dma_kernel<0, true>), dim3(g1), dim3(512), 0, st, gate_up, eb1, x16, texp, we1, s1,
+            launch_moe_dma<0, true>(ragged, g1, st, gate_up, eb1, x16, texp, we1, s1,
                                sw1, gy, tile_e, tile_end, meta, (int)N1, (int)H, (int)(N1 / 256), 0);
         else if (swi)
-            hipLaunchKernelGGL((moe_dma_kernel<1, true>), dim3(g1), dim3(512), 0, st, gate_up, eb1, x16, texp, we1, s1,
+            launch_moe_dma<1, true>(ragged, g1, st, gate_up, eb1, x16, texp, we1, s1,
                                sw1, gy, tile_e, tile_end, meta, (int)N1, (int)H, (int)(N1 / 256), 0);
         else if (gx)
-            hipLaunchKernelGGL((moe_dma_kernel<0, false, true>), dim3(g1), dim3(512), 0, st, gate_up, eb1, x16, texp,
+            launch_moe_dma<0, false, true>(ragged, g1, st, gate_up, eb1, x16, texp,
                                we1, s1, sw1, gy, tile_e, tile_end, meta, (int)N1, (int)H, (int)(N1 / 256), pass,
                                (const int*)rowmap);
         else if (precision == 0)
-            hipLaunchKernelGGL((moe_dma_kernel<0>), dim3(g1), dim3(512), 0, st, gate_up, eb1, x16, texp, we1, s1, sw1,
+            launch_moe_dma<0>(ragged, g1, st, gate_up, eb1, x16, texp, we1, s1, sw1,
                                gy, tile_e, tile_end, meta, (int)N1, (int)H, (int)(N1 / 256), pass);
         else
-            hipLaunchKernelGGL((moe_dma_kernel<1>), dim3(g1), dim3(512), 0, st, gate_up, eb1, x16, texp, we1, s1, sw1,
+            launch_moe_dma<1>(ragged, g1, st, gate_up, eb1, x16, texp, we1, s1, sw1,
                                gy, tile_e, tile_end, meta, (int)N1, (int)H, (int)(N1 / 256), 0);
         if (launch_status() != Q4MI_OK) return Q4MI_E_LAUNCH;
     }
@@ -2202,10 +2293,10 @@ extern "C" int q4_moe_prefill(const uint8_t* gate_up, const uint8_t* down, const
     }
     for (int pass = 0; pass < hpasses; ++pass) {
         if (precision == 0)
-            hipLaunchKernelGGL((moe_dma_kernel<0>), dim3(g2), dim3(512), 0, st, down, eb2, h16[pass], texp, we2, s2,
+            launch_moe_dma<0>(ragged, g2, st, down, eb2, h16[pass], texp, we2, s2,
                                sw2, gy, tile_e, tile_end, meta, (int)N2, (int)F, (int)(N2 / 256), pass);
         else
-            hipLaunchKernelGGL((moe_dma_kernel<1>), dim3(g2), dim3(512), 0, st, down, eb2, h16[pass], texp, we2, s2,
+            launch_moe_dma<1>(ragged, g2, st, down, eb2, h16[pass], texp, we2, s2,
                                sw2, gy, tile_e, tile_end, meta, (int)N2, (int)F, (int)(N2 / 256), 0);
         if (launch_status() != Q4MI_OK) return Q4MI_E_LAUNCH;
     }
