@@ -525,8 +525,7 @@ int q4_gemm_prefill_scaled(const uint8_t* packed, const void* scales, const void
  * output is converted once and read by several projections (gate and up of an FFN; Q, K
  * and V), or written in this layout by the producer itself. The buffer holds the GEMM's
  * 16-bit activation planes (one; two for f32 x in precision 0: value and fp16 remainder) in
- * the pipelined kernel's tiled image (K % 64 == 0; rows [T][K] otherwise), then the
- * per-token exponents (precision 0). The reference's prefill design likewise takes X
+ * the pipelined kernel's tiled image, then the per-token exponents (precision 0). The reference's prefill design likewise takes X
  * pre-tiled for its B operand, the tiling being the host's job (gemm_q4_prefill.py:19-22,
  * :68-70). Bytes, or 0 for bad arguments: */
 size_t q4_prefill_prepared_bytes(int T, int64_t K, int x_dtype, int precision);

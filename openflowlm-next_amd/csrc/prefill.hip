@@ -28,15 +28,11 @@
 // output per block, i.e. twice the MFMA time of the same block at
 // 512 MAC/clk vs 16 FMA/clk per SIMD, so it cannot reach the MFMA roofline.
 //
-// Tiling: a workgroup computes BN weight rows x BT tokens with WGN x WGT
-// waves. Per LDS stage (KS blocks of 32 K) the waves turn the stage's mx
-// tiles (one 64-row group x 32 K each) into 16-bit weights in LDS and copy
-// the activations to LDS; stages are double buffered so the global loads and
-// the dequant of stage s+1 overlap the MFMAs of stage s, with one barrier per
-// stage. The default variant runs 8 waves (two per SIMD, 128x64 wave tiles),
-// so one wave's dequant and LDS traffic hide behind the other's MFMAs. LDS
-// rows are padded by 8 halves so a 16-lane ds_read_b128 phase hits distinct
-// banks.
+// Tiling: a workgroup computes 256 weight rows x 256 tokens, or 128 x 128, in 8 waves (two per
+// SIMD). Per LDS stage the waves turn eight mx tiles (64 rows x 32 K each) into 16-bit weights
+// in LDS and copy the activations to LDS; the loads and the dequant of later stages overlap
+// the MFMAs of stage s, with one barrier per stage, and one wave's dequant and LDS traffic
+// hide behind the other's MFMAs.
 #include <stdlib.h>
 
 #include "norm_core.h"
@@ -94,15 +90,15 @@ __device__ __forceinline__ u32x4 dequant8(uint32_t w, uint32_t s, uint32_t nib2,
 // 2^(s_t + e_n) when the operands were scaled (texp / wexp not null), exactly; accum adds
 // the result to what y holds (the second pass of f32 activations). tmap: token t's exponent
 // is texp[tmap[t]] (activations gathered from another row order), else texp[t].
-// Token fragment j starts TS * j tokens after wt0.
-template <int FN, int FT, int TS, bool SCALED>
+// Token fragment j starts 64 j tokens after wt0.
+template <int FN, int FT, bool SCALED>
 __device__ __forceinline__ void store_tile(const f32x4 (&acc)[FN][FT], float* __restrict__ y,
                                            const int* __restrict__ texp, const int* __restrict__ wexp, int T, int N,
                                            int wt0, int wn0, int accum, const int* __restrict__ tmap = nullptr) {
     const int lane = threadIdx.x & 63, i16 = lane & 15, kg = lane >> 4;
 #pragma unroll
     for (int j = 0; j < FT; ++j) {
-        const int t = wt0 + j * TS + i16;
+        const int t = wt0 + j * 64 + i16;
         if (t >= T) continue;
         const int st = SCALED ? texp[tmap ? max(tmap[t], 0) : t] : 0;
 #pragma unroll
@@ -164,138 +160,8 @@ __device__ __forceinline__ void store_swiglu(const f32x4 (&acc)[FN][FT], uint16_
     }
 }
 
-// BN x BT workgroup tile, WGN x WGT waves (wave tile BN/WGN x BT/WGT), KS
-// 32-K blocks per LDS stage.
-template <int BN, int BT, int WGN, int WGT, int KS, int PREC>
-__global__ __launch_bounds__(64 * WGN * WGT) void prefill_kernel(const uint8_t* __restrict__ packed,
-                                                                 const uint16_t* __restrict__ x16,
-                                                                 const int* __restrict__ texp,
-                                                                 const int* __restrict__ wexp,
-                                                                 const uint32_t* __restrict__ s16,
-                                                                 float* __restrict__ y, int T, int N, int K,
-                                                                 int tiles_t, int accum) {
-    constexpr int NT = 64 * WGN * WGT, NW = WGN * WGT;
-    constexpr int WN = BN / WGN, WT = BT / WGT;      // wave tile
-    constexpr int FN = WN / 16, FT = WT / 16;        // 16-wide fragments per wave
-    constexpr int RG = BN / 64;                      // mx row groups per workgroup tile
-    constexpr int WTILES = RG * KS;                  // mx tiles per stage
-    constexpr int WPW = (WTILES + NW - 1) / NW;      // mx tiles per wave per stage
-    constexpr int BK = 32 * KS;
-    constexpr int STR = BK + 8;                      // halves per LDS row (pad: conflict-free b128 reads)
-    constexpr int XCH = BT * KS * 4 / NT;            // 16-byte activation chunks per thread per stage
-    static_assert(XCH * NT == BT * KS * 4, "activation chunks must divide evenly");
-    typedef typename std::conditional<PREC == 0, f16x8, bf16x8>::type frag_t;
-
-    __shared__ __attribute__((aligned(16))) uint16_t wl[2][BN * STR];
-    __shared__ __attribute__((aligned(16))) uint16_t xl[2][BT * STR];
-
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wn = wave % WGN, wt = wave / WGN;
-    const int bt = blockIdx.x % tiles_t, bn = blockIdx.x / tiles_t;
-    const int n0 = bn * BN, t0 = bt * BT;
-    const int KB = K >> 5, NSTAGE = KB / KS;
-    const int G = N >> 6;
-    const int i16 = lane & 15, kg = lane >> 4;
-
-    // This wave's mx tiles: tile u = wave + NW*i -> (row group u % RG, block u / RG of the
-    // stage). Tile bases are wave-uniform and advance by a uniform stride per stage, and
-    // the per-lane offsets are fixed 32-bit values, so no address register is rewritten
-    // inside the K loop (rewriting one that a pending load targets forces a vmcnt wait).
-    const uint8_t* wbase[WPW];
-    const uint8_t* sbase[WPW];
-    int wrow[WPW], wcol[WPW];
-    bool wown[WPW];
-#pragma unroll
-    for (int i = 0; i < WPW; ++i) {
-        const int u = wave + NW * i;
-        wown[i] = u < WTILES;
-        const int rgl = u % RG, kbl = u / RG;
-        const int rg = min(n0 / 64 + rgl, G - 1);                       // clamp ragged N
-        wbase[i] = packed + ((int64_t)rg * KB + kbl) * kTileBytes;
-        sbase[i] = PREC == 0 ? (const uint8_t*)s16 + ((int64_t)rg * KB + kbl) * 256 : wbase[i] + kCodeBytes;
-        wrow[i] = rgl * 64 + i16;
-        wcol[i] = kbl * 32 + kg * 8;
-    }
-    const uint32_t coff = lane * 16, soff = i16 * 16;
-    constexpr int SSTR = PREC == 0 ? 256 : kTileBytes;               // scale block stride per 32-K block
-    const uint16_t* xbase = x16 + (int64_t)t0 * K;                    // workgroup-uniform
-    int xoff[XCH], xdst[XCH];
-#pragma unroll
-    for (int c = 0; c < XCH; ++c) {
-        const int ch = tid + NT * c, tok = ch / (KS * 4), part = ch % (KS * 4);
-        xoff[c] = (min(t0 + tok, T - 1) - t0) * K + part * 8;            // halves, fits 32 bits
-        xdst[c] = tok * STR + part * 8;
-    }
-    const uint32_t nib2 = vgpr_const(kNib2);
-    const uint32_t magic = vgpr_const(PREC == 0 ? kMagic1024 : kMagic128);
-
-    f32x4 acc[FN][FT];
-#pragma unroll
-    for (int i = 0; i < FN; ++i)
-#pragma unroll
-        for (int j = 0; j < FT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    u32x4 wc[WPW], wsc[WPW];
-    u32x4 xr[XCH];
-    auto gload = [&](int st) {
-        const uint16_t* xs = xbase + st * BK;                            // uniform
-#pragma unroll
-        for (int c = 0; c < XCH; ++c) xr[c] = *(const u32x4*)(xs + xoff[c]);
-#pragma unroll
-        for (int i = 0; i < WPW; ++i) {
-            if (wown[i]) {
-                const uint8_t* tp = wbase[i] + st * (KS * kTileBytes);  // uniform
-                wc[i] = load_nt_u32x4(tp + coff);
-                wsc[i] = load_nt_u32x4(sbase[i] + st * (KS * SSTR) + soff);
-            }
-        }
-    };
-    auto lstore = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < WPW; ++i) {
-            if (wown[i]) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const u32x4 v = dequant8<PREC>(wc[i][r], wsc[i][r], nib2, magic);
-                    *(u32x4*)&wl[buf][(wrow[i] + r * 16) * STR + wcol[i]] = v;
-                }
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < XCH; ++c) *(u32x4*)&xl[buf][xdst[c]] = xr[c];
-    };
-
-    gload(0);
-    lstore(0);
-    __syncthreads();
-    for (int st = 0; st < NSTAGE; ++st) {
-        const int buf = st & 1;
-        const bool more = st + 1 < NSTAGE;
-        if (more) gload(st + 1);
-#pragma unroll
-        for (int kk = 0; kk < KS; ++kk) {
-            frag_t a[FN], b[FT];
-#pragma unroll
-            for (int i = 0; i < FN; ++i)
-                a[i] = *(const frag_t*)&wl[buf][(wn * WN + i * 16 + i16) * STR + kk * 32 + kg * 8];
-#pragma unroll
-            for (int j = 0; j < FT; ++j)
-                b[j] = *(const frag_t*)&xl[buf][(wt * WT + j * 16 + i16) * STR + kk * 32 + kg * 8];
-#pragma unroll
-            for (int i = 0; i < FN; ++i)
-#pragma unroll
-                for (int j = 0; j < FT; ++j) acc[i][j] = mfma16(a[i], b[j], acc[i][j]);
-        }
-        if (more) lstore(buf ^ 1);
-        __syncthreads();
-    }
-
-    store_tile<FN, FT, 16, PREC == 0>(acc, y, texp, wexp, T, N, t0 + wt * WT, n0 + wn * WN, accum);
-}
-
 // ---------------------------------------------------------------------------
-// The pipelined variant (default for K % 64 == 0): 256 x 256 workgroup tile,
+// The pipelined kernel: 256 x 256 workgroup tile,
 // 8 waves (2 along N x 4 along T, 128 x 64 wave tiles), 64-K stages.
 //   * weights: each wave loads one mx tile (64 rows x 32 K) per stage into
 //     registers three stages ahead (three register sets) and dequantizes
@@ -393,10 +259,14 @@ __device__ __forceinline__ void vgpr_landed(u32x4& v) { asm volatile("" : "+v"(v
 // fetches the 16-byte chunk that its LDS slot holds under the swizzle, so the LDS image is
 // the pre-tiled one's. The token exponents (PREC 0) are then indexed by source row too:
 // texp[gmap[s]].
+// TAIL: K / 32 is not a multiple of KBS; the last stage's planes past K are zeros on both sides (so
+// an infinity or NaN in the data meets no made-up factor): their weight words are masked (the
+// loads re-read the row group's last tile) and their activations DMA'd from past a buffer
+// resource's range.
 // SWI: the matrix alternates 64 gate and 64 up rows. A 256-row tile's wave holds one such pair
 // as fragments 0..3 and 4..7; in a 128-row tile (one pair) wave wn holds the pair's gate rows
 // [32 wn, +32) as fragments 0, 1 and the same up rows as fragments 2, 3.
-template <int PREC, int KBS, int FN, int FT, bool SWI = false, bool GATHER = false>
+template <int PREC, int KBS, int FN, int FT, bool SWI = false, bool GATHER = false, bool TAIL = false>
 __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict__ packed,
                                          const uint16_t* __restrict__ x16, const int* __restrict__ texp,
                                          const int* __restrict__ wexp, const uint32_t* __restrict__ s16,
@@ -405,6 +275,7 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
     static_assert((KBS == 2 && (FN == 8 || FN == 6)) || (KBS == 4 && FN == 4), "256-, 192- or 128-row tiles");
     static_assert(FT >= 1 && FT * KBS <= 8, "a ring slot holds 32 KB of activations");
     static_assert(!SWI || FN != 6, "the SwiGLU epilogue pairs gate and up rows");
+    static_assert(!TAIL || (!GATHER && FN != 6), "one DMA source, whole row tiles");
     constexpr int WN = 16 * FN, RGS = 8 / KBS, RG = FN / 2;
     constexpr int WPB = RGS * 64 * 64;               // one 32-K plane of the weight buffer
     constexpr int XPB = FT * 64 * 64;                // one 32-K plane of an activation slot
@@ -414,7 +285,7 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn = wave & 1, wt = wave >> 1;
-    const int KB = K >> 5, NSTK = KB / KBS;
+    const int KB = K >> 5, NSTK = TAIL ? (KB + KBS - 1) / KBS : KB / KBS;
     const int st0 = (int)((int64_t)split * NSTK / splits), NST = (int)((int64_t)(split + 1) * NSTK / splits) - st0;
     y += (int64_t)split * T * N;
     const int G = N >> 6;
@@ -477,18 +348,30 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
             const uint32_t dst = xdst + slot * kTileB + plane * XPB + unit * 1024;
             if constexpr (GATHER)
                 lds_dma16_buf(xrs, goff[q / GQ], (uint32_t)(KBS * (st0 + st) + plane) * 64, dst);
+            else if constexpr (TAIL)
+                lds_dma16_buf(__builtin_amdgcn_make_buffer_rsrc((void*)(xsrc + (int64_t)KBS * st * kPlaneB), 0,
+                                                                (int)(kPadOffset - 1), kBufferWord3),
+                              KBS * (st0 + st) + plane < KB ? xoff : kPadOffset, plane * kPlaneB + unit * 1024, dst);
             else
                 lds_dma16(xsrc + ((int64_t)(KBS * st + plane) * kPlaneB + unit * 1024), xoff, dst);
         }
     };
     auto issue_w = [&](int st, u32x4& c, u32x4& sc) {
+        if constexpr (TAIL) {                        // tiles past the row group's last: that one again
+            const int back = max(KBS * (st0 + st) + kbl - (KB - 1), 0);
+            load16_async(c, wsrc + (int64_t)(KBS * st - back) * kTileBytes, coff);
+            load16_async(sc, ssrc + (int64_t)(KBS * st - back) * SSTR, soff);
+            return;
+        }
         load16_async(c, wsrc + st * (KBS * kTileBytes), coff);         // uniform bases
         load16_async(sc, ssrc + st * (KBS * SSTR), soff);
     };
-    auto store_w = [&](int buf, const u32x4& c, const u32x4& sc, int r0, int r1) {
+    auto store_w = [&](int st, int buf, const u32x4& c, const u32x4& sc, int r0, int r1) {
+        const uint32_t in = !TAIL || KBS * (st0 + st) + kbl < KB ? ~0u : 0u;       // uniform
 #pragma unroll
         for (int r = r0; r < r1; ++r)
-            *(u32x4*)(lds + wst + buf * kTileB + r * 1024) = dequant8<PREC>(c[r], sc[r], nib2, magic);
+            *(u32x4*)(lds + wst + buf * kTileB + r * 1024) =
+                TAIL ? dequant8<PREC>(c[r] & in, sc[r] & in, nib2, magic) : dequant8<PREC>(c[r], sc[r], nib2, magic);
     };
     auto read_frags = [&](int buf, int slot, int kk, frag_t (&a)[FN], frag_t (&b)[FT]) {
         const uint8_t* xp = lds + (slot == 2 ? bbase2 : bbase + slot * kTileB) + kk * XPB;
@@ -517,7 +400,7 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
     else __builtin_amdgcn_s_waitcnt(kWaitVm0);
     vgpr_landed(wc[0]);
     vgpr_landed(ws[0]);
-    store_w(0, wc[0], ws[0], 0, 4);
+    store_w(0, 0, wc[0], ws[0], 0, 4);
     __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
     asm volatile("s_barrier" ::: "memory");
 
@@ -546,7 +429,7 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
         for (int kk = 0; kk < KBS; ++kk) {
             frag_t a[FN], b[FT];
             read_frags(cur, slot, kk, a, b);
-            store_w(cur ^ 1, wc[nset], ws[nset], DW * kk, DW * kk + DW);
+            store_w(st + 1, cur ^ 1, wc[nset], ws[nset], DW * kk, DW * kk + DW);
             mfmas(a, b);
             __builtin_amdgcn_sched_group_barrier(0x100, FN + FT, 0);
 #pragma unroll
@@ -595,22 +478,23 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
         store_swiglu<FN, FT, PREC == 0>(acc, (uint16_t*)y, texp, wexp, T, N, t0 + wt * 16,
                                         n0 + (kPair ? wn * 32 : wn * WN), tmap);
     else
-        store_tile<FN, FT, 64, PREC == 0>(acc, y, texp, wexp, T, N, t0 + wt * 16, n0 + wn * WN, accum, tmap);
+        store_tile<FN, FT, PREC == 0>(acc, y, texp, wexp, T, N, t0 + wt * 16, n0 + wn * WN, accum, tmap);
 }
 
 // dma_tile with the smallest token tile that covers the valid tokens [t0, T) of a tile of
 // 64 * FTMAX (workgroup-uniform). A 256-row stage takes ~0.55, 0.68, 0.85 and 1.0 us with 1 to 4
 // groups of 64 tokens: the dequantization and the LDS traffic of the weights remain.
-template <int PREC, int KBS, int FN, int FTMAX, bool SWI = false, bool GATHER = false, class... A>
+template <int PREC, int KBS, int FN, int FTMAX, bool SWI = false, bool GATHER = false, bool TAIL = false, class... A>
 __device__ __forceinline__ void dma_tile_valid(uint8_t* lds, const uint8_t* packed, const uint16_t* x16,
                                                const int* texp, const int* wexp, const uint32_t* s16, float* y, int T,
                                                int N, int K, int n0, int t0, A... rest) {
     const int groups = (T - t0 + 63) >> 6;
     if (groups >= FTMAX)
-        dma_tile<PREC, KBS, FN, FTMAX, SWI, GATHER>(lds, packed, x16, texp, wexp, s16, y, T, N, K, n0, t0, rest...);
+        dma_tile<PREC, KBS, FN, FTMAX, SWI, GATHER, TAIL>(lds, packed, x16, texp, wexp, s16, y, T, N, K, n0, t0,
+                                                          rest...);
     else if constexpr (FTMAX > 1)
-        dma_tile_valid<PREC, KBS, FN, FTMAX - 1, SWI, GATHER>(lds, packed, x16, texp, wexp, s16, y, T, N, K, n0, t0,
-                                                              rest...);
+        dma_tile_valid<PREC, KBS, FN, FTMAX - 1, SWI, GATHER, TAIL>(lds, packed, x16, texp, wexp, s16, y, T, N, K, n0,
+                                                                    t0, rest...);
 }
 
 // Workgroups [0, wide_wgs) take the 256-row tiles of rows [0, narrow_row0), the rest the
@@ -685,6 +569,24 @@ __global__ __launch_bounds__(512) void prefill_dma128_kernel(const uint8_t* __re
                                   (tile % tiles_t) * 128, b % splits, splits, accum);
 }
 
+// Either form for a K that ends inside a stage (KBS = 2: K % 64 == 32, KBS = 4: K % 128 != 0), the rest of
+// the last stage zeros. An unpipelined kernel without K splits took such shapes before:
+// 147 f32 tokens on 1600 x 10656 798 -> 61 us, 89 on 5376 x 2656 109 -> 22, 2048 on 8192 x 2080 106
+// -> 78; and K % 128 == 64 had 256 x 256 tiles only: 260 on 4096 x 2752 38 -> 32.
+template <int PREC, int KBS>
+__global__ __launch_bounds__(512) void prefill_tail_kernel(const uint8_t* __restrict__ packed,
+                                                           const uint16_t* __restrict__ x16,
+                                                           const int* __restrict__ texp, const int* __restrict__ wexp,
+                                                           const uint32_t* __restrict__ s16, float* __restrict__ y,
+                                                           int T, int N, int K, int tiles_t, int splits, int accum) {
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[5 * kTileB];
+    const int b = xcd_group((int)blockIdx.x, (int)gridDim.x), tile = b / splits;
+    constexpr int R = 512 / KBS;
+    dma_tile_valid<PREC, KBS, 16 / KBS, 8 / KBS, false, false, true>(lds, packed, x16, texp, wexp, s16, y, T, N, K,
+                                                                     (tile / tiles_t) * R, (tile % tiles_t) * R,
+                                                                     b % splits, splits, accum);
+}
+
 // The gate/up GEMM with the SwiGLU epilogue: workgroup b takes the 256-row tile of pair rows
 // (b / tiles_t) * 256 and token tile b % tiles_t over all of K (no split), writing h.
 template <int PREC>
@@ -734,12 +636,12 @@ __device__ __forceinline__ int fp16_fit_exponent(float v) {
 // token tiles). PREC 0: fp16, token row t scaled by 2^-s_t with s_t = fp16_fit_exponent(max
 // |x_t|), and texp[t] = s_t. PREC 1: bf16 (RNE from f32), no exponents.
 // TILED: the 16-byte chunk i (k = 8i..8i+7) of token t goes to its place in the LDS image
-// of the pipelined kernel's activation tiles: [token tile][64-K stage][32-K plane][256 rows]
-// [4 chunks], chunk c of row r at slot c ^ ((r >> 1) & 3). Each stage of a token tile is then
+// of the pipelined kernel's activation tiles: [token tile][32-K plane][256 rows][4 chunks],
+// chunk c of row r at slot c ^ ((r >> 1) & 3). Each stage of a token tile is then
 // one contiguous 32 KB block, copied to LDS verbatim. Otherwise rows stay [T][K].
 __device__ __forceinline__ int64_t xchunk_dst(int t, int i, int K) {
-    const int r = t & 255, st = i >> 3, kk = (i >> 2) & 1, c = i & 3;
-    return ((((int64_t)(t >> 8) * (K >> 6) + st) * 2 + kk) * 256 + r) * 4 + (c ^ ((r >> 1) & 3));
+    const int r = t & 255, plane = i >> 2, c = i & 3;
+    return (((int64_t)(t >> 8) * (K >> 5) + plane) * 256 + r) * 4 + (c ^ ((r >> 1) & 3));
 }
 
 // Block-wide max of a non-negative value over 256 threads (result in every thread).
@@ -930,7 +832,7 @@ __global__ __launch_bounds__(256) void prefill_xprep(const void* __restrict__ x,
 // last, took 29.7 us at five planes, this 14.7 (4.3 TB/s). The row also goes to LDS, from which thread
 // tid sums the squares of elements tid + 256 j, j ascending, as rmsnorm_add_kernel does (values
 // past K are zeros there and are skipped here: the fp64 sum is the same).
-template <int PER, int PREC, bool TILED>
+template <int PER, int PREC>
 __global__ __launch_bounds__(256) void rmsnorm_prepare_kernel(const float* x, const float* __restrict__ add,
                                                               int add_planes, const void* __restrict__ w, int w_bf16,
                                                               int vec, float* y, uint16_t* __restrict__ x16,
@@ -1026,7 +928,7 @@ __global__ __launch_bounds__(256) void rmsnorm_prepare_kernel(const float* x, co
         }
         __syncthreads();
     }
-    xprep_row<false, PREC, TILED, 0>(            // the row sits in LDS: read it there twice
+    xprep_row<false, PREC, true, 0>(            // the row sits in LDS: read it there twice
         [&](int i, float (&o)[8]) {
             const u32x4 wd = *(const u32x4*)(xs + 8 * i);
 #pragma unroll
@@ -1041,7 +943,7 @@ __global__ __launch_bounds__(256) void rmsnorm_prepare_kernel(const float* x, co
 // in LDS and converted as prefill_xprep converts a bf16 row; h is also stored [T][F] when
 // h_out is given. g and u are f32 rows with strides ldg / ldu (one fused gate/up output:
 // u = g + F, both strides 2F). Rows past T are the tile padding (zeros).
-template <int PREC, bool TILED>
+template <int PREC>
 __global__ __launch_bounds__(256) void swiglu_prepare_kernel(const float* __restrict__ g, const float* __restrict__ u,
                                                              int64_t ldg, int64_t ldu, uint16_t* __restrict__ h_out,
                                                              uint16_t* __restrict__ x16, int* __restrict__ texp,
@@ -1065,7 +967,7 @@ __global__ __launch_bounds__(256) void swiglu_prepare_kernel(const float* __rest
         }
         __syncthreads();
     }
-    xprep_row<false, PREC, TILED, 0>(
+    xprep_row<false, PREC, true, 0>(
         [&](int i, float (&o)[8]) {
             const u32x4 wd = *(const u32x4*)(hs + 8 * i);
 #pragma unroll
@@ -1074,84 +976,27 @@ __global__ __launch_bounds__(256) void swiglu_prepare_kernel(const float* __rest
         t >= T, x16, texp, t, F, 0);
 }
 
-// Kernel variants: (BN, BT, waves along N, waves along T, 32-K blocks per stage).
-struct TileCfg {
-    int bn, bt, wgn, wgt, ks;
-};
-constexpr TileCfg kCfgs[] = {
-    {256, 256, 2, 4, 2},     // 8 waves, 128x64 wave tiles, 64-K stages
-    {256, 128, 2, 4, 2},     // 8 waves, 128x32
-    {128, 256, 2, 4, 2},     // 8 waves, 64x64
-    {128, 128, 2, 4, 2},     // 8 waves, 64x32
-    {256, 256, 2, 2, 1},     // 4 waves, 128x128 wave tiles, 32-K stages
-    {256, 256, 2, 4, 2},     // the LDS-DMA pipelined kernel (prefill_dma_kernel)
-    {128, 128, 2, 4, 4},     // its 128 x 128 form (prefill_dma128_kernel)
-};
-constexpr int kDmaCfg = 5, kDma128Cfg = 6;
-constexpr bool dma_cfg(int cfg) { return cfg >= kDmaCfg; }   // reads the tiled activation image
-
-// Kernel variant: the pipelined kernel whenever K % 64 == 0 (K splits keep small grids
-// busy); otherwise the generic variant with the fewest rounds of 256 workgroups
-// (Q4MI_PREFILL_CFG overrides).
-int choose_cfg(int T, int N, int K) {
-    static int forced = [] {
-        const char* e = getenv("Q4MI_PREFILL_CFG");
-        return e ? atoi(e) : -1;
-    }();
-    if (forced >= 0 && forced < kDmaCfg && K % (32 * kCfgs[forced].ks) == 0) return forced;
-    if (K % 64 == 0) return kDmaCfg;
-    const double eff[] = {1.0, 0.9, 0.9, 0.75, 0.8};   // relative per-workgroup efficiency
-    double best = 1e300;
-    int pick = 4;
-    for (int i = 0; i < kDmaCfg; ++i) {
-        if (K % (32 * kCfgs[i].ks)) continue;
-        const int64_t wgs = ceil_div(N, kCfgs[i].bn) * ceil_div(T, kCfgs[i].bt);
-        const int64_t rounds = ceil_div(wgs, 256);
-        const double cost = (double)rounds * kCfgs[i].bn * kCfgs[i].bt / eff[i];
-        if (cost < best) {
-            best = cost;
-            pick = i;
-        }
-    }
-    return pick;
-}
-
-template <int C, int PREC>
-void launch_cfg(int64_t grid, hipStream_t st, const uint8_t* w, const uint16_t* x16, const int* te, const int* we,
-                const uint32_t* s16, float* y, int T, int N, int K, int tiles_t, int accum) {
-    constexpr TileCfg c = kCfgs[C];
-    hipLaunchKernelGGL((prefill_kernel<c.bn, c.bt, c.wgn, c.wgt, c.ks, PREC>), dim3((unsigned)grid),
-                       dim3(64 * c.wgn * c.wgt), 0, st, w, x16, te, we, s16, y, T, N, K, tiles_t, accum);
-}
-
+// One GEMM launch of the plan's form: tile 256 or 128 (see PrefillPlan).
 template <int PREC>
-void launch_prefill(int cfg, int64_t grid, hipStream_t st, const uint8_t* w, const uint16_t* x16, const int* te,
+void launch_prefill(int tile, int64_t grid, hipStream_t st, const uint8_t* w, const uint16_t* x16, const int* te,
                     const int* we, const uint32_t* s16, float* y, int T, int N, int K, int tiles_t, int splits,
                     int wide_wgs, int narrow_row0, int accum) {
-    switch (cfg) {
-        case 0: launch_cfg<0, PREC>(grid, st, w, x16, te, we, s16, y, T, N, K, tiles_t, accum); break;
-        case 1: launch_cfg<1, PREC>(grid, st, w, x16, te, we, s16, y, T, N, K, tiles_t, accum); break;
-        case 2: launch_cfg<2, PREC>(grid, st, w, x16, te, we, s16, y, T, N, K, tiles_t, accum); break;
-        case 3: launch_cfg<3, PREC>(grid, st, w, x16, te, we, s16, y, T, N, K, tiles_t, accum); break;
-        case 4: launch_cfg<4, PREC>(grid, st, w, x16, te, we, s16, y, T, N, K, tiles_t, accum); break;
-        case kDma128Cfg:
-            hipLaunchKernelGGL((prefill_dma128_kernel<PREC>), dim3((unsigned)grid), dim3(512), 0, st, w, x16, te, we,
-                               s16, y, T, N, K, tiles_t, splits, accum);
-            break;
-        default:
-#define Q4MI_DMA(KERN)                                                                                              \
+#define Q4MI_DMA(KERN, ...)                                                                                         \
     hipLaunchKernelGGL(KERN, dim3((unsigned)grid), dim3(512), 0, st, w, x16, te, we, s16, y, T, N, K, tiles_t, splits, \
-                       wide_wgs, narrow_row0, accum)
-            if (ragged_tokens(T)) {
-                if (wide_wgs < grid) Q4MI_DMA((prefill_ragged_kernel<PREC, true>));
-                else Q4MI_DMA((prefill_ragged_kernel<PREC, false>));
-            } else {
-                if (wide_wgs < grid) Q4MI_DMA((prefill_dma_kernel<PREC, true>));
-                else Q4MI_DMA((prefill_dma_kernel<PREC, false>));
-            }
-#undef Q4MI_DMA
-            break;
+                       ##__VA_ARGS__, accum)
+    if (tile == 128) {
+        if (K % 128) Q4MI_DMA((prefill_tail_kernel<PREC, 4>));
+        else Q4MI_DMA((prefill_dma128_kernel<PREC>));
+    } else if (K % 64) {
+        Q4MI_DMA((prefill_tail_kernel<PREC, 2>));
+    } else if (ragged_tokens(T)) {
+        if (wide_wgs < grid) Q4MI_DMA((prefill_ragged_kernel<PREC, true>), wide_wgs, narrow_row0);
+        else Q4MI_DMA((prefill_ragged_kernel<PREC, false>), wide_wgs, narrow_row0);
+    } else {
+        if (wide_wgs < grid) Q4MI_DMA((prefill_dma_kernel<PREC, true>), wide_wgs, narrow_row0);
+        else Q4MI_DMA((prefill_dma_kernel<PREC, false>), wide_wgs, narrow_row0);
     }
+#undef Q4MI_DMA
 }
 
 // y = sum of the S partials in split order (deterministic), 4 floats per thread; accum adds
@@ -1189,12 +1034,12 @@ int device_cus() {
     return cus;
 }
 
-// Launch plan of one prefill GEMM: the kernel variant, its token tiles and K splits, and for
-// the 256-row form of the pipelined kernel the rows covered by 256-row tiles ([0,
-// narrow_row0), wide_wgs workgroups) and by 192-row tiles (the rest). Both forms hold one
-// workgroup per CU (160 KB of LDS). Three levers fit the work to the CUs: the tile (256 x 256,
-// or 128 x 128 when K % 128 == 0: four times the tiles, so small grids need fewer K splits
-// and their partial traffic, at two thirds of the MFMA rate), a K split (partial sums
+// Launch plan of one prefill GEMM: its tile (256 x 256 or 128 x 128), token tiles and K splits,
+// and for the 256-row form the rows covered by 256-row tiles ([0, narrow_row0), wide_wgs
+// workgroups) and by 192-row tiles (the rest; K % 64 == 0). Both forms hold one workgroup per
+// CU (160 KB of LDS). Three levers fit the work to the CUs: the tile (128 x 128: four times
+// the tiles, so small grids need fewer K splits and their partial traffic, at two thirds
+// of the MFMA rate), a K split (partial sums
 // reduced in order afterwards) and 192-row tiles, which fill the CUs the last round of 256-row
 // tiles leaves idle without any partial traffic (Llama-3-8B gate_up at T = 2048: 448 tiles of
 // 256 rows run in 2 rounds of 256 CUs; 256 of 256 rows + 256 of 192 rows in 1 + 3/4).
@@ -1202,7 +1047,7 @@ int device_cus() {
 // Q4MI_PREFILL_SPLITS and Q4MI_PREFILL_NARROW (the count of 192-row strips) override (256-row
 // tiles only).
 struct PrefillPlan {
-    int cfg, tiles_t, splits, wide_wgs, narrow_row0;
+    int tile, tiles_t, splits, wide_wgs, narrow_row0;
     int64_t grid;
 };
 
@@ -1239,81 +1084,79 @@ double makespan(int64_t A, int64_t B, int64_t C, double cw, double cn) {
 
 PrefillPlan make_plan_uncached(int T, int64_t N, int64_t K) {
     PrefillPlan p;
-    p.cfg = choose_cfg(T, (int)N, (int)K);
-    p.tiles_t = (int)ceil_div(T, kCfgs[p.cfg].bt);
-    int64_t tiles = ceil_div(N, kCfgs[p.cfg].bn) * p.tiles_t;
+    p.tile = 256;
+    p.tiles_t = (int)ceil_div(T, 256);
+    int64_t tiles = ceil_div(N, 256) * p.tiles_t;
     p.splits = 1;
     p.wide_wgs = (int)tiles;
     p.narrow_row0 = (int)N;
-    if (p.cfg == kDmaCfg) {
-        static const int forced = [] {
-            const char* e = getenv("Q4MI_PREFILL_SPLITS");
-            return e ? atoi(e) : 0;
-        }();
-        static const int forced_narrow = [] {
-            const char* e = getenv("Q4MI_PREFILL_NARROW");
-            return e ? atoi(e) : -1;
-        }();
-        const int nst = (int)(K / 64), cap = nst < 16 ? nst : 16;
-        const int64_t G = N / 64, tt = p.tiles_t;
-        const int cus = device_cus();
-        const int ftl = (int)ceil_div(T - (tt - 1) * 256, 64);         // 64-token groups of the last token tile
-        // the split reduce: a launch and its traffic
-        auto reduce_us = [&](int S) { return S > 1 ? 3.0 + (double)(S + 1) * T * N * 4 / 5.0e6 : 0.0; };
-        // a forced strip count is used only where it fits: 3b <= G and 4 | G - 3b
-        const int64_t fb = forced_narrow > 0 && 3 * (int64_t)forced_narrow <= G &&
-                                   (G - 3 * (int64_t)forced_narrow) % 4 == 0
-                               ? forced_narrow
-                               : forced_narrow == 0 ? 0 : -1;
-        double best = 1e300;
-        // b 192-row strips and a 256-row strips with 4a + 3b = G (b = 0: 256-row strips only,
-        // the last one clamped when G % 4 != 0). 192-row tiles only fill the last round of
-        // 256-row ones, so at most two rounds of them are considered.
-        for (int64_t b = 0; 3 * b <= G && (b * tt <= 2 * cus || b == fb); ++b) {
-            if (b > 0 && (G - 3 * b) % 4) continue;
-            if (fb >= 0 && b != fb) continue;
-            const int64_t a = b > 0 ? (G - 3 * b) / 4 : ceil_div(G, 4);
-            for (int S = 1; S <= cap; ++S) {
-                if (forced > 0 && S != (forced < cap ? forced : cap)) continue;
-                if (b > 0 && b != fb && b * tt * S > 2 * cus) break;
-                const int ns = (int)ceil_div(nst, S);
-                const double full = tile_us(256, 4, ns, 4), last = tile_us(256, ftl, ns, 4);
-                double cost;
-                if (b > 0) {        // every tile at the mean of the full and the ragged token tiles
-                    const double mean = ((double)(tt - 1) + last / full) / (double)tt;
-                    cost = makespan(a * tt * S, b * tt * S, cus, mean * full, mean * tile_us(192, 4, ns, 4));
-                } else {
-                    cost = makespan(a * (tt - 1) * S, a * S, cus, full, last);
-                }
-                // ties: fewer rows computed (a clamped last 256-row strip repeats rows)
-                cost += reduce_us(S) + 1e-6 * (double)(256 * a + 192 * b);
-                if (cost < best) {
-                    best = cost;
-                    p.splits = S;
-                    p.wide_wgs = (int)(a * tt * S);
-                    p.narrow_row0 = b > 0 ? (int)(256 * a) : (int)N;
-                    tiles = (a + b) * tt;
-                }
+    static const int forced = [] {
+        const char* e = getenv("Q4MI_PREFILL_SPLITS");
+        return e ? atoi(e) : 0;
+    }();
+    static const int forced_narrow = [] {
+        const char* e = getenv("Q4MI_PREFILL_NARROW");
+        return e ? atoi(e) : -1;
+    }();
+    const int nst = (int)ceil_div(K, 64), cap = nst < 16 ? nst : 16;
+    const int64_t G = N / 64, tt = p.tiles_t;
+    const int cus = device_cus();
+    const int ftl = (int)ceil_div(T - (tt - 1) * 256, 64);         // 64-token groups of the last token tile
+    // the split reduce: a launch and its traffic
+    auto reduce_us = [&](int S) { return S > 1 ? 3.0 + (double)(S + 1) * T * N * 4 / 5.0e6 : 0.0; };
+    // a forced strip count is used only where it fits: 3b <= G and 4 | G - 3b
+    const int64_t fb = forced_narrow > 0 && 3 * (int64_t)forced_narrow <= G &&
+                               (G - 3 * (int64_t)forced_narrow) % 4 == 0
+                           ? forced_narrow
+                           : forced_narrow == 0 ? 0 : -1;
+    double best = 1e300;
+    // b 192-row strips and a 256-row strips with 4a + 3b = G (b = 0: 256-row strips only,
+    // the last one clamped when G % 4 != 0). 192-row tiles only fill the last round of
+    // 256-row ones, so at most two rounds of them are considered.
+    for (int64_t b = 0; 3 * b <= G && (b * tt <= 2 * cus || b == fb); ++b) {
+        if (b > 0 && ((G - 3 * b) % 4 || K % 64)) continue;
+        if (fb >= 0 && b != fb) continue;
+        const int64_t a = b > 0 ? (G - 3 * b) / 4 : ceil_div(G, 4);
+        for (int S = 1; S <= cap; ++S) {
+            if (forced > 0 && S != (forced < cap ? forced : cap)) continue;
+            if (b > 0 && b != fb && b * tt * S > 2 * cus) break;
+            const int ns = (int)ceil_div(nst, S);
+            const double full = tile_us(256, 4, ns, 4), last = tile_us(256, ftl, ns, 4);
+            double cost;
+            if (b > 0) {        // every tile at the mean of the full and the ragged token tiles
+                const double mean = ((double)(tt - 1) + last / full) / (double)tt;
+                cost = makespan(a * tt * S, b * tt * S, cus, mean * full, mean * tile_us(192, 4, ns, 4));
+            } else {
+                cost = makespan(a * (tt - 1) * S, a * S, cus, full, last);
+            }
+            // ties: fewer rows computed (a clamped last 256-row strip repeats rows)
+            cost += reduce_us(S) + 1e-6 * (double)(256 * a + 192 * b);
+            if (cost < best) {
+                best = cost;
+                p.splits = S;
+                p.wide_wgs = (int)(a * tt * S);
+                p.narrow_row0 = b > 0 ? (int)(256 * a) : (int)N;
+                tiles = (a + b) * tt;
             }
         }
-        // 128 x 128 tiles, 128-K stages
-        if (K % 128 == 0 && forced <= 0 && forced_narrow < 0) {
-            const int64_t r2 = ceil_div(G, 2), t2 = ceil_div(T, 128);
-            const int nst2 = (int)(K / 128), cap2 = nst2 < 16 ? nst2 : 16;
-            const int ftl2 = (int)ceil_div(T - (t2 - 1) * 128, 64);
-            for (int S = 1; S <= cap2; ++S) {
-                const int ns = (int)ceil_div(nst2, S);
-                const double cost = makespan(r2 * (t2 - 1) * S, r2 * S, cus, tile_us(128, 2, ns, 4),
-                                             tile_us(128, ftl2, ns, 4)) + reduce_us(S);
-                if (cost < best) {
-                    best = cost;
-                    p.cfg = kDma128Cfg;
-                    p.tiles_t = (int)t2;
-                    p.splits = S;
-                    p.wide_wgs = 0;
-                    p.narrow_row0 = (int)N;
-                    tiles = r2 * t2;
-                }
+    }
+    // 128 x 128 tiles, 128-K stages
+    if (forced <= 0 && forced_narrow < 0) {
+        const int64_t r2 = ceil_div(G, 2), t2 = ceil_div(T, 128);
+        const int nst2 = (int)ceil_div(K, 128), cap2 = nst2 < 16 ? nst2 : 16;
+        const int ftl2 = (int)ceil_div(T - (t2 - 1) * 128, 64);
+        for (int S = 1; S <= cap2; ++S) {
+            const int ns = (int)ceil_div(nst2, S);
+            const double cost = makespan(r2 * (t2 - 1) * S, r2 * S, cus, tile_us(128, 2, ns, 4),
+                                         tile_us(128, ftl2, ns, 4)) + reduce_us(S);
+            if (cost < best) {
+                best = cost;
+                p.tile = 128;
+                p.tiles_t = (int)t2;
+                p.splits = S;
+                p.wide_wgs = 0;
+                p.narrow_row0 = (int)N;
+                tiles = r2 * t2;
             }
         }
     }
@@ -1442,10 +1285,10 @@ int gemm_pass(const uint8_t* packed, const void* scales, const uint16_t* x16, co
     float* out = plan.splits > 1 ? part : y;
     const int accum = plan.splits > 1 ? 0 : pass;
     if (precision == 0)
-        launch_prefill<0>(plan.cfg, plan.grid, st, packed, x16, te, we, s16, out, T, (int)N, (int)K, plan.tiles_t,
+        launch_prefill<0>(plan.tile, plan.grid, st, packed, x16, te, we, s16, out, T, (int)N, (int)K, plan.tiles_t,
                           plan.splits, plan.wide_wgs, plan.narrow_row0, accum);
     else
-        launch_prefill<1>(plan.cfg, plan.grid, st, packed, x16, nullptr, nullptr, nullptr, out, T, (int)N, (int)K,
+        launch_prefill<1>(plan.tile, plan.grid, st, packed, x16, nullptr, nullptr, nullptr, out, T, (int)N, (int)K,
                           plan.tiles_t, plan.splits, plan.wide_wgs, plan.narrow_row0, accum);
     if (launch_status() != Q4MI_OK) return Q4MI_E_LAUNCH;
     if (plan.splits > 1) {
@@ -1468,10 +1311,9 @@ int prefill_impl(const uint8_t* packed, const void* scales, const void* x, int x
     uint16_t* x16 = (uint16_t*)workspace;
     int* te = (int*)((char*)workspace + x16_bytes(T, K));
     float* part = (float*)((char*)workspace + xprep_bytes(T, K));
-    const bool tiled = dma_cfg(make_plan(T, N, K).cfg);
     for (int pass = 0; pass < activation_passes(x_dtype, precision); ++pass) {
         // rows up to whole 64-token groups: the kernels read no others
-        launch_xprep(x_dtype == Q4MI_F32, precision, tiled, dim3((unsigned)(ceil_div(T, 64) * 64)), st, x, x16, te, T,
+        launch_xprep(x_dtype == Q4MI_F32, precision, true, dim3((unsigned)(ceil_div(T, 64) * 64)), st, x, x16, te, T,
                      (int)K, pass);
         if (launch_status() != Q4MI_OK) return Q4MI_E_LAUNCH;
         const int rc = gemm_pass(packed, scales, x16, te, y, T, N, K, precision, part, pass, st);
@@ -1523,7 +1365,6 @@ extern "C" int q4_gemm_prefill_scaled(const uint8_t* packed, const void* scales,
 // and read by several projections (gate and up of an FFN, Q, K and V), or written in this
 // layout by the producer itself. Layout: the activation planes of the GEMM's passes (two for
 // f32 x in precision 0: value and remainder), each x16_bytes(T, K), then the token exponents.
-// The pipelined kernel's tiled image when K % 64 == 0, else rows [T][K].
 // ---------------------------------------------------------------------------
 namespace {
 size_t prepared_bytes(int T, int64_t K, int x_dtype, int precision) {
@@ -1549,7 +1390,7 @@ extern "C" int q4_prefill_prepare(const void* x, int x_dtype, int T, int64_t K, 
     const int passes = activation_passes(x_dtype, precision);
     int* te = (int*)((char*)prepared + passes * x16_bytes(T, K));
     for (int pass = 0; pass < passes; ++pass) {
-        launch_xprep(x_dtype == Q4MI_F32, precision, K % 64 == 0, dim3((unsigned)padded_tokens(T)),
+        launch_xprep(x_dtype == Q4MI_F32, precision, true, dim3((unsigned)padded_tokens(T)),
                      (hipStream_t)stream, x, (uint16_t*)((char*)prepared + pass * x16_bytes(T, K)), te, T, (int)K,
                      pass);
         if (launch_status() != Q4MI_OK) return Q4MI_E_LAUNCH;
@@ -1586,19 +1427,18 @@ extern "C" int q4_rmsnorm_prepare(const float* x, const float* add, int add_plan
     const dim3 grid((unsigned)padded_tokens(T)), block(256);
     const hipStream_t st = (hipStream_t)stream;
     const int wb = w_dtype == Q4MI_BF16;
-    const bool tiled = K % 64 == 0;
     const int vec = !misaligned16(x) && !misaligned16(add) && !misaligned16(w) && !misaligned16(y);
-#define Q4MI_RP(PER, PR, TL)                                                                                   \
-    hipLaunchKernelGGL((rmsnorm_prepare_kernel<PER, PR, TL>), grid, block, 0, st, x, add, add_planes, w, wb, vec, y, \
-                       x16, te, T, (int)K, eps)
-#define Q4MI_RP_K(PR, TL)                                                                            \
-    do {                                                                                             \
-        if (K <= 256 * 16) Q4MI_RP(16, PR, TL);                                                      \
-        else if (K <= 256 * 32) Q4MI_RP(32, PR, TL);                                                 \
-        else Q4MI_RP(64, PR, TL);                                                                    \
+#define Q4MI_RP(PER, PR)                                                                                            \
+    hipLaunchKernelGGL((rmsnorm_prepare_kernel<PER, PR>), grid, block, 0, st, x, add, add_planes, w, wb, vec, y, x16, \
+                       te, T, (int)K, eps)
+#define Q4MI_RP_K(PR)                               \
+    do {                                            \
+        if (K <= 256 * 16) Q4MI_RP(16, PR);         \
+        else if (K <= 256 * 32) Q4MI_RP(32, PR);    \
+        else Q4MI_RP(64, PR);                       \
     } while (0)
-    if (precision == 0) { if (tiled) Q4MI_RP_K(0, true); else Q4MI_RP_K(0, false); }
-    else { if (tiled) Q4MI_RP_K(1, true); else Q4MI_RP_K(1, false); }
+    if (precision == 0) Q4MI_RP_K(0);
+    else Q4MI_RP_K(1);
 #undef Q4MI_RP_K
 #undef Q4MI_RP
     return launch_status();
@@ -1626,12 +1466,10 @@ extern "C" int q4_swiglu_prepare(const float* g, const float* u, int64_t ldg, in
     int* te = (int*)((char*)prepared + x16_bytes(T, F));
     const dim3 grid((unsigned)padded_tokens(T)), block(256);
     const hipStream_t st = (hipStream_t)stream;
-    const bool tiled = F % 64 == 0;
-#define Q4MI_SP(PR, TL)                                                                                          \
-    hipLaunchKernelGGL((swiglu_prepare_kernel<PR, TL>), grid, block, 0, st, g, u, ldg, ldu, (uint16_t*)h, x16, te, \
-                       T, (int)F)
-    if (precision == 0) { if (tiled) Q4MI_SP(0, true); else Q4MI_SP(0, false); }
-    else { if (tiled) Q4MI_SP(1, true); else Q4MI_SP(1, false); }
+#define Q4MI_SP(PR)                                                                                               \
+    hipLaunchKernelGGL((swiglu_prepare_kernel<PR>), grid, block, 0, st, g, u, ldg, ldu, (uint16_t*)h, x16, te, T, (int)F)
+    if (precision == 0) Q4MI_SP(0);
+    else Q4MI_SP(1);
 #undef Q4MI_SP
     return launch_status();
 }
@@ -1685,7 +1523,6 @@ extern "C" int q4_gemm_prefill_prepared(const uint8_t* packed, const void* scale
     if (a != Q4MI_OK) return a > 0 ? Q4MI_OK : a;
     if (precision == 0 && (!scales || misaligned16(scales))) return Q4MI_E_ARG;
     const PrefillPlan plan = make_plan(T, N, K);
-    if (dma_cfg(plan.cfg) != (K % 64 == 0)) return Q4MI_E_ARG;   // a forced generic variant reads rows
     if (plan.splits > 1 && (!workspace || workspace_bytes < q4_gemm_prefill_prepared_workspace_bytes(T, N, K)))
         return Q4MI_E_WORKSPACE;
     const int passes = activation_passes(x_dtype, precision);
@@ -1713,7 +1550,6 @@ extern "C" int q4_gemm_prefill_prepared_partials(const uint8_t* packed, const vo
     if (a != Q4MI_OK) return a > 0 ? Q4MI_OK : a;
     if (precision == 0 && (!scales || misaligned16(scales))) return Q4MI_E_ARG;
     const PrefillPlan plan = make_plan(T, N, K);
-    if (dma_cfg(plan.cfg) != (K % 64 == 0)) return Q4MI_E_ARG;
     // the planes this call writes follow this process's plan, not a count queried elsewhere
     if (part_bytes < (size_t)plan.splits * T * N * sizeof(float)) return Q4MI_E_WORKSPACE;
     const int* te = (const int*)((const char*)prepared + x16_bytes(T, K));
@@ -1722,10 +1558,10 @@ extern "C" int q4_gemm_prefill_prepared_partials(const uint8_t* packed, const vo
     const hipStream_t st = (hipStream_t)stream;
     // plane s of the K split at part + s T N (one plane, the whole product, when unsplit)
     if (precision == 0)
-        launch_prefill<0>(plan.cfg, plan.grid, st, packed, (const uint16_t*)prepared, te, we, s16, part, T, (int)N,
+        launch_prefill<0>(plan.tile, plan.grid, st, packed, (const uint16_t*)prepared, te, we, s16, part, T, (int)N,
                           (int)K, plan.tiles_t, plan.splits, plan.wide_wgs, plan.narrow_row0, 0);
     else
-        launch_prefill<1>(plan.cfg, plan.grid, st, packed, (const uint16_t*)prepared, nullptr, nullptr, nullptr, part, T,
+        launch_prefill<1>(plan.tile, plan.grid, st, packed, (const uint16_t*)prepared, nullptr, nullptr, nullptr, part, T,
                           (int)N, (int)K, plan.tiles_t, plan.splits, plan.wide_wgs, plan.narrow_row0, 0);
     return launch_status();
 }
