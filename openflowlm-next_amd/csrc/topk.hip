@@ -18,9 +18,9 @@
 // Padding slots are key 0, below every real key. Each lane holds 4 keys. For k <= 8 a
 // block of 4 waves takes 1024 logits: each lane sorts its 4 keys in registers, each
 // wave pops its k largest with k pairs of DPP wave reductions, and wave 0 merges the
-// four wave lists the same way. For larger k a block of 16 waves takes 4096: each wave
-// runs a bitonic network over its 256 keys and the top-64 lists merge 16 -> 4 -> 1 with
-// the network's last two stages. Blocks emit k keys each; the same kernel then runs over those keys
+// four wave lists the same way. For larger k a block of 16 waves takes up to 4096: the keys
+// that reach a bound that 64 of them reach are ranked by counting (or, when too many do,
+// sorted). Blocks emit k (64 for the larger k) keys each; the same kernel then runs over those keys
 // until one block per token remains, which writes ids and values.
 #include "q4mi_device.h"
 #include "q4mi_internal.h"
@@ -171,14 +171,27 @@ __device__ __forceinline__ void bitonic256(uint64_t (&a)[4], int lane) {
     if constexpr (S0 < 256) bitonic256<S0 * 2>(a, lane);
 }
 
-// The k > 8 block: 16 waves over 4096 inputs. Each wave brings its 256 keys to a
-// descending order -- logits with the full network; keys of an earlier pass, which
-// arrive as sorted runs of 64, with only the last two stages (odd runs read reversed,
-// so each pair of runs is a bitonic 128-run). The waves' top-64 lists are merged four
-// at a time with the same two stages: 16 -> 4 -> 1. Non-final passes write their
-// sorted top 64 (a superset of the top k); the final pass writes the first k as ids and
-// values. Cost does not depend on k.
+// The k > 8 block: 16 waves over up to 4096 inputs, 4 per lane, its top 64 found by
+// filtering and counting. The lanes' quads are 256 groups of up to 16 keys; a value (a key's
+// high word) that 64 of the groups' maxima reach is a bound that at least 64 keys reach, so
+// only the keys that reach it can be among the top 64. The largest such value, to its top
+// kBoundBits, is found bit by bit with ballots: 70 to 90 of a full block's keys reach it in
+// any order that does not depend on the position. They are compacted into LDS (in any order)
+// and each one's rank is the number of larger ones, counted by 1024 / slots threads per key;
+// keys are distinct, so the ranks are too. Keys of an earlier pass arrive as sorted runs of
+// 64: quad q of a wave takes a run's places q mod 16, so the groups' maxima are the runs'
+// leading keys. A block with more than kSurvivors (positions in descending order, many equal
+// values) sorts: each wave runs the bitonic network over its 256 keys and the top-64 lists
+// merge four at a time, 16 -> 4 -> 1, with the network's last two stages. That sort alone was
+// bound by its ~1440 VALU instructions a wave with 4 waves on a SIMD. The smallest of 64
+// groups' maxima as the bound leaves 300 keys, more than 512 in 1 % of the blocks, and the
+// slowest block sets the time: no gain (15.3 us). Non-final passes write their top 64 (a
+// superset of the top k); the final pass writes the first k as ids and values. Cost does
+// not depend on k. 8 rows of 128256 f32 logits, k = 40, first and last pass:
+// 15.1 + 8.3 us sorted, 6.8 + 5.9 filtered.
 constexpr int kSortWaves = 16, kSortThreads = kSortWaves * kLanes, kSortChunk = kSortThreads * kPerLane;
+constexpr int kSurvivors = 512, kGroups = kSortThreads / 4, kBoundBits = 18;
+static_assert(kGroups == 4 * kLanes, "four groups per lane");
 
 __device__ __forceinline__ void merge4(uint64_t (&a)[4], const uint64_t (*lists)[kLanes], int lane) {
 #pragma unroll
@@ -199,53 +212,122 @@ __device__ __forceinline__ void put_top64(const uint64_t (&a)[4], uint64_t* list
     }
 }
 
+// The largest value over each quad of lanes, in all of them.
+__device__ __forceinline__ uint32_t quad_max_u32(uint32_t v) {
+    v = dpp_step<true>(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0xB1, 0xF, 0xF, false));
+    return dpp_step<true>(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x4E, 0xF, 0xF, false));
+}
+
+// Block s: inputs [s * chunk, min(n, (s + 1) * chunk)) of token row m, chunk <= kSortChunk.
 template <bool KEYS, bool FINAL>
 __global__ __launch_bounds__(kSortThreads) void topk_sort_kernel(const void* __restrict__ in, int64_t ld, int64_t n,
-                                                                 int k, int mode, uint64_t* __restrict__ out_keys,
+                                                                 int chunk, int k, int mode,
+                                                                 uint64_t* __restrict__ out_keys,
                                                                  int32_t* __restrict__ ids,
                                                                  float* __restrict__ vals) {
-    __shared__ uint64_t l1[kSortWaves][kLanes], l2[4][kLanes];
-    const int lane = threadIdx.x & (kLanes - 1), wave = threadIdx.x / kLanes;
-    const int64_t s = blockIdx.x, m = blockIdx.y;
-    const int64_t base = s * kSortChunk + wave * (kLanes * kPerLane);
+    __shared__ uint64_t l1[kSortWaves][kLanes], l2[4][kLanes], top[kLanes];
+    __shared__ __attribute__((aligned(16))) uint64_t surv[kSurvivors];
+    __shared__ int rank[kSurvivors];
+    __shared__ __attribute__((aligned(16))) uint32_t group_max[kGroups];
+    __shared__ int count;
+    const int tid = threadIdx.x, lane = tid & (kLanes - 1), wave = tid / kLanes;
+    const int64_t s = blockIdx.x, m = blockIdx.y, base = s * chunk;
+    const int at = wave * kLanes + (KEYS ? (lane >> 2) + 16 * (lane & 3) : lane);
     uint64_t a[kPerLane];
-    if constexpr (KEYS) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int e = 4 * lane + r;                      // run e >> 6 of this wave, odd runs reversed
-            const int64_t i = base + (e & ~63) + (((e >> 6) & 1) ? 63 - (e & 63) : (e & 63));
-            a[r] = i < n ? ((const uint64_t*)in)[m * ld + i] : 0;
+    for (int j = 0; j < kPerLane; ++j) {
+        const int o = j * kSortThreads + at;
+        const int64_t i = base + o;
+        if (o < chunk && i < n) {
+            if constexpr (KEYS)
+                a[j] = ((const uint64_t*)in)[m * ld + i];
+            else
+                a[j] = logit_key(((const float*)in)[m * ld + i], (uint32_t)i, mode);
+        } else {
+            a[j] = 0;
         }
-        bitonic256<128>(a, lane);
-    } else {
-#pragma unroll
-        for (int j = 0; j < kPerLane; ++j) {
-            const int64_t i = base + j * kLanes + lane;      // coalesced
-            a[j] = i < n ? logit_key(((const float*)in)[m * ld + i], (uint32_t)i, mode) : 0;
-        }
-        bitonic256<2>(a, lane);
     }
-    put_top64(a, l1[wave], wave & 1, lane);
+    if (tid < kSurvivors) surv[tid] = 0, rank[tid] = 0;
+    if (tid < kLanes) top[tid] = 0;
+    if (tid == 0) count = 0;
+    uint32_t big = 0;
+#pragma unroll
+    for (int j = 0; j < kPerLane; ++j) big = dpp_step<true>(big, (uint32_t)(a[j] >> 32));
+    big = quad_max_u32(big);
+    if ((lane & 3) == 0) group_max[tid >> 2] = big;
     __syncthreads();
-    if (wave < 4) {
-        merge4(a, l1 + 4 * wave, lane);
-        put_top64(a, l2[wave], wave & 1, lane);
+    const uint4 g = *(const uint4*)(group_max + 4 * lane);
+    uint32_t bound = 0;
+#pragma unroll
+    for (int b = 31; b > 31 - kBoundBits; --b) {
+        const uint32_t v = bound | 1u << b;
+        const int reach = __popcll(__ballot(g.x >= v)) + __popcll(__ballot(g.y >= v)) + __popcll(__ballot(g.z >= v)) +
+                          __popcll(__ballot(g.w >= v));
+        if (reach >= kLanes) bound = v;
+    }
+    // the keys that reach the bound (padding, key 0, never does)
+    uint64_t hit[kPerLane];
+    int c = 0;
+#pragma unroll
+    for (int j = 0; j < kPerLane; ++j) {
+        hit[j] = __ballot(a[j] != 0 && (uint32_t)(a[j] >> 32) >= bound);
+        c += __popcll(hit[j]);
+    }
+    int o = 0;
+    if (lane == 0 && c) o = atomicAdd(&count, c);
+    o = __builtin_amdgcn_readfirstlane(o);
+#pragma unroll
+    for (int j = 0; j < kPerLane; ++j) {
+        const int to = o + __popcll(hit[j] & ((1ull << lane) - 1ull));
+        if ((hit[j] >> lane & 1) && to < kSurvivors) surv[to] = a[j];
+        o += __popcll(hit[j]);
+    }
+    __syncthreads();
+    const int total = count;
+    if (total <= kSurvivors) {
+        // thread (slot, part): the larger keys among part's share of the survivors (an even
+        // number from an even place; the zeros behind the last one count for none)
+        const int slots = total <= kSurvivors / 4 ? kSurvivors / 4 : total <= kSurvivors / 2 ? kSurvivors / 2 : kSurvivors;
+        const int parts = kSortThreads / slots;
+        const int slot = tid & (slots - 1), part = tid / slots;
+        const int share = ((total + parts - 1) / parts + 1) & ~1;
+        const int j0 = min(part * share, total), j1 = min(j0 + share, total);
+        const uint64_t key = surv[slot];
+        int larger = 0;
+        if ((slot & ~(kLanes - 1)) < total) {                 // wave-uniform
+#pragma unroll 4
+            for (int j = j0; j < j1; j += 2) {
+                const ulonglong2 v = *(const ulonglong2*)(surv + j);
+                larger += (v.x > key) + (v.y > key);
+            }
+            atomicAdd(&rank[slot], larger);
+        }
+        __syncthreads();
+        if (tid < total && rank[tid] < kLanes) top[rank[tid]] = surv[tid];
+    } else {
+        bitonic256<2>(a, lane);
+        put_top64(a, l1[wave], wave & 1, lane);
+        __syncthreads();
+        if (wave < 4) {
+            merge4(a, l1 + 4 * wave, lane);
+            put_top64(a, l2[wave], wave & 1, lane);
+        }
+        __syncthreads();
+        if (wave == 0) {
+            merge4(a, l2, lane);
+            put_top64(a, top, false, lane);
+        }
     }
     __syncthreads();
     if (wave != 0) return;
-    merge4(a, l2, lane);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int e = 4 * lane + r;
-        const uint64_t key = a[r];
-        if constexpr (FINAL) {
-            if (e < k) {
-                ids[m * k + e] = key ? (int32_t)~(uint32_t)key : -1;
-                if (vals) vals[m * k + e] = key ? from_monotone((uint32_t)(key >> 32)) : -__builtin_inff();
-            }
-        } else if (e < 64) {
-            out_keys[(m * gridDim.x + s) * 64 + e] = key;
+    const uint64_t key = top[lane];
+    if constexpr (FINAL) {
+        if (lane < k) {
+            ids[m * k + lane] = key ? (int32_t)~(uint32_t)key : -1;
+            if (vals) vals[m * k + lane] = key ? from_monotone((uint32_t)(key >> 32)) : -__builtin_inff();
         }
+    } else {
+        out_keys[(m * gridDim.x + s) * kLanes + lane] = key;
     }
 }
 
@@ -316,11 +398,13 @@ void launch_topk(const TopkPlan& p, bool final_pass, dim3 grid, hipStream_t st, 
             hipLaunchKernelGGL((topk_kernel<KEYS, false>), grid, dim3(kThreads), 0, st, in, ld, n, k, mode,
                                out_keys, ids, vals);
     } else {
+        // even chunks, whole runs of 64: a short last block would pass its group bound too easily
+        const int chunk = (int)(ceil_div(ceil_div(n, (int64_t)grid.x), (int64_t)kLanes) * kLanes);
         if (final_pass)
-            hipLaunchKernelGGL((topk_sort_kernel<KEYS, true>), grid, dim3(kSortThreads), 0, st, in, ld, n, k, mode,
-                               out_keys, ids, vals);
+            hipLaunchKernelGGL((topk_sort_kernel<KEYS, true>), grid, dim3(kSortThreads), 0, st, in, ld, n, chunk, k,
+                               mode, out_keys, ids, vals);
         else
-            hipLaunchKernelGGL((topk_sort_kernel<KEYS, false>), grid, dim3(kSortThreads), 0, st, in, ld, n, k,
+            hipLaunchKernelGGL((topk_sort_kernel<KEYS, false>), grid, dim3(kSortThreads), 0, st, in, ld, n, chunk, k,
                                mode, out_keys, ids, vals);
     }
 }
