@@ -1955,7 +1955,10 @@ __global__ __launch_bounds__(512) void moe_dma_kernel(const uint8_t* __restrict_
                                  0, 1, accum, gmap);
 }
 
-// The same with each tile's work sized by its valid 64-slot groups.
+// The same with each tile's work sized by its valid 64-slot groups. An XCD takes a contiguous run of
+// the tiles there are (meta[0], not the grid's bound; the last count % 8 stay where they are), so an
+// expert's row tiles fetch its gathered token rows into one L2 instead of each into another's: 128
+// experts, top-8 of 2048 tokens, the block 1.203 -> 1.231 times the speed of the same earlier build.
 template <int PREC, bool SWI = false, bool GATHER = false>
 __global__ __launch_bounds__(512) void moe_ragged_kernel(const uint8_t* __restrict__ packed, int64_t ebytes,
                                                          const uint16_t* __restrict__ x16, const int* __restrict__ texp,
@@ -1965,8 +1968,10 @@ __global__ __launch_bounds__(512) void moe_ragged_kernel(const uint8_t* __restri
                                                          const int* __restrict__ meta, int N, int K, int tiles_n, int accum,
                                                          const int* __restrict__ gmap) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[5 * kTileB];
-    const int b = blockIdx.x, tt = b / tiles_n, rt = b % tiles_n;
-    if (tt >= meta[0]) return;
+    const int count = meta[0] * tiles_n, whole = count & ~7;
+    if ((int)blockIdx.x >= count) return;
+    const int b = (int)blockIdx.x < whole ? xcd_group((int)blockIdx.x, whole) : (int)blockIdx.x;
+    const int tt = b / tiles_n, rt = b % tiles_n;
     const int e = tile_e[tt];
     dma_tile_valid<PREC, 2, 8, 4, SWI, GATHER>(lds, packed + e * ebytes, x16, texp,
                                  PREC == 0 ? wexp + (int64_t)e * N : nullptr,
