@@ -210,6 +210,7 @@ __device__ __forceinline__ void lds_dma16_buf(__amdgpu_buffer_rsrc_t rsrc, uint3
                  : "memory", "m0");
 }
 constexpr uint32_t kPadOffset = 0x80000000u;   // past the gather resource's range: a zero row
+constexpr uint64_t kGatherBytes = kPadOffset - 1;   // the resource's range: a longer matrix is not gathered from
 constexpr int kBufferWord3 = 0x00020000;       // raw buffer resource, 32-bit data format
 
 // 16 bytes per lane into registers (uniform base + 32-bit lane offset). The compiler does not
@@ -313,7 +314,7 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
     // of the group; LDS slot lane & 3 holds chunk (lane & 3) ^ ((lane >> 3) & 3))
     constexpr int GQ = FT % 2 ? 1 : KBS;             // units of a wave that share a row group
     uint32_t goff[XD / GQ];
-    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc((void*)x16, 0, (int)(kPadOffset - 1),
+    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc((void*)x16, 0, (int)kGatherBytes,
                                                                          kBufferWord3);   // GATHER only
     if constexpr (GATHER) {
         const uint32_t chunk = (uint32_t)((lane & 3) ^ ((lane >> 3) & 3)) * 16;
@@ -350,7 +351,7 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
                 lds_dma16_buf(xrs, goff[q / GQ], (uint32_t)(KBS * (st0 + st) + plane) * 64, dst);
             else if constexpr (TAIL)
                 lds_dma16_buf(__builtin_amdgcn_make_buffer_rsrc((void*)(xsrc + (int64_t)KBS * st * kPlaneB), 0,
-                                                                (int)(kPadOffset - 1), kBufferWord3),
+                                                                (int)kGatherBytes, kBufferWord3),
                               KBS * (st0 + st) + plane < KB ? xoff : kPadOffset, plane * kPlaneB + unit * 1024, dst);
             else
                 lds_dma16(xsrc + ((int64_t)(KBS * st + plane) * kPlaneB + unit * 1024), xoff, dst);
@@ -2112,9 +2113,9 @@ extern "C" int q4_moe_prefill(const uint8_t* gate_up, const uint8_t* down, const
 
     hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(1024), 0, st, topk_ids, P, E, cnt, off, tile_e, tile_end, meta);
     if (launch_status() != Q4MI_OK) return Q4MI_E_LAUNCH;
-    // precision 0 with 32-bit gather offsets: the gate/up GEMM gathers its token rows (below), whose
-    // pre-pass rides in the slots' launch
-    const bool gx = precision == 0 && (uint64_t)T * H * 2 <= 0xffffffffull;
+    // precision 0, token rows within a gather resource's range: the gate/up GEMM gathers them
+    // (below), and their pre-pass rides in the slots' launch
+    const bool gx = precision == 0 && (uint64_t)T * H * 2 <= kGatherBytes;
     if (gx && xf32)
         hipLaunchKernelGGL((moe_slots_xprep_kernel<true>), dim3((unsigned)(E + T)), dim3(256), 0, st, topk_ids, P,
                            topk, E, cnt, off, sop, rowmap, x, x16, texp, (int)H);
@@ -2141,10 +2142,10 @@ extern "C" int q4_moe_prefill(const uint8_t* gate_up, const uint8_t* down, const
 
     // precision 1 on bf16 x: the expert GEMMs DMA their token rows straight from x (gate/up,
     // slot s <- token rowmap[s]) and from h (down, slot s <- h row s): no per-slot activation
-    // images. h [S][F] bf16 from the gate/up epilogue goes to the x16 region, Y to gy. The DMA
-    // offsets are 32-bit.
-    const bool gather = precision == 1 && !xf32 && (uint64_t)T * H * 2 <= 0xffffffffull &&
-                        (uint64_t)S * F * 2 <= 0xffffffffull;
+    // images. h [S][F] bf16 from the gate/up epilogue goes to the x16 region, Y to gy. Rows past
+    // a gather resource's range would read as zeros, so longer x or h take the images.
+    const bool gather = precision == 1 && !xf32 && (uint64_t)T * H * 2 <= kGatherBytes &&
+                        (uint64_t)S * F * 2 <= kGatherBytes;
     if (gather) {
         launch_moe_dma<1, true, true>(ragged, g1, st, gate_up, eb1,
                            (const uint16_t*)x, texp, we1, s1, sw1, (float*)x16, tile_e, tile_end, meta, (int)N1,
