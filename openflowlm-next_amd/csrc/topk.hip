@@ -19,9 +19,9 @@
 // block of 4 waves takes 1024 logits: each lane sorts its 4 keys in registers, each
 // wave pops its k largest with k pairs of DPP wave reductions, and wave 0 merges the
 // four wave lists the same way. For larger k a block of 16 waves takes up to 4096: the keys
-// that reach a bound that 64 of them reach are ranked by counting (or, when too many do,
-// sorted). Blocks emit k (64 for the larger k) keys each; the same kernel then runs over those keys
-// until one block per token remains, which writes ids and values.
+// that reach a bound that 64 of them reach are ranked by counting. Blocks emit k (64 for the
+// larger k) keys each; the same kernel then runs over those keys until one block per token
+// remains, which writes ids and values.
 #include "q4mi_device.h"
 #include "q4mi_internal.h"
 
@@ -114,103 +114,28 @@ __device__ __forceinline__ uint64_t wave_pop(uint64_t (&a)[N], int k, int lane) 
     return mine;
 }
 
-// Exchange a 32-bit value with lane ^ M (M = 1, 2: DPP quad permutes; 4..16: ds_swizzle's
-// xor mode; 32: ds_bpermute).
-template <int M>
-__device__ __forceinline__ uint32_t xchg(uint32_t v, int lane) {
-    if constexpr (M == 1)
-        return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0xB1, 0xF, 0xF, false);
-    else if constexpr (M == 2)
-        return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x4E, 0xF, 0xF, false);
-    else if constexpr (M < 32)
-        return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, (M << 10) | 0x1F);
-    else
-        return (uint32_t)__builtin_amdgcn_ds_bpermute((lane ^ 32) << 2, (int)v);
-}
-
-// One stage (size S, distance J) of the bitonic network over the wave's 256 keys, key e
-// = 4 lane + r held in a[r]: position e keeps the larger of (e, e ^ J) when it is the
-// lower of the pair and its S-run sorts descending ((e & S) == 0), else the smaller.
-template <int S, int J>
-__device__ __forceinline__ void bitonic_stage(uint64_t (&a)[4], int lane) {
-    if constexpr (J >= 4) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const uint64_t o = ((uint64_t)xchg<J / 4>((uint32_t)(a[r] >> 32), lane) << 32) |
-                               xchg<J / 4>((uint32_t)a[r], lane);
-            const int e = 4 * lane + r;
-            const bool keep_max = ((e & J) == 0) == ((e & S) == 0);
-            const uint64_t hi = o > a[r] ? o : a[r], lo = o > a[r] ? a[r] : o;
-            a[r] = keep_max ? hi : lo;
-        }
-    } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            if ((r & J) == 0) {
-                const bool desc = ((4 * lane + r) & S) == 0;
-                const uint64_t x = a[r], y = a[r ^ J];
-                const bool swap = desc ? (x < y) : (x > y);
-                a[r] = swap ? y : x;
-                a[r ^ J] = swap ? x : y;
-            }
-        }
-    }
-}
-
-template <int S, int J>
-__device__ __forceinline__ void bitonic_merge(uint64_t (&a)[4], int lane) {
-    bitonic_stage<S, J>(a, lane);
-    if constexpr (J > 1) bitonic_merge<S, J / 2>(a, lane);
-}
-
-// Stages S0, 2 S0, ..., 256: with S0 = 2 a full descending sort of the wave's 256 keys;
-// with S0 = 128 the merge of two bitonic 128-runs (desc then asc halves) into one.
-template <int S0>
-__device__ __forceinline__ void bitonic256(uint64_t (&a)[4], int lane) {
-    bitonic_merge<S0, S0 / 2>(a, lane);
-    if constexpr (S0 < 256) bitonic256<S0 * 2>(a, lane);
-}
-
 // The k > 8 block: 16 waves over up to 4096 inputs, 4 per lane, its top 64 found by
-// filtering and counting. The lanes' quads are 256 groups of up to 16 keys; a value (a key's
-// high word) that 64 of the groups' maxima reach is a bound that at least 64 keys reach, so
-// only the keys that reach it can be among the top 64. The largest such value, to its top
-// kBoundBits, is found bit by bit with ballots: 70 to 90 of a full block's keys reach it in
-// any order that does not depend on the position. They are compacted into LDS (in any order)
-// and each one's rank is the number of larger ones, counted by 1024 / slots threads per key;
-// keys are distinct, so the ranks are too. Keys of an earlier pass arrive as sorted runs of
-// 64: quad q of a wave takes a run's places q mod 16, so the groups' maxima are the runs'
-// leading keys. A block with more than kSurvivors (positions in descending order, many equal
-// values) sorts: each wave runs the bitonic network over its 256 keys and the top-64 lists
-// merge four at a time, 16 -> 4 -> 1, with the network's last two stages. That sort alone was
-// bound by its ~1440 VALU instructions a wave with 4 waves on a SIMD. The smallest of 64
-// groups' maxima as the bound leaves 300 keys, more than 512 in 1 % of the blocks, and the
-// slowest block sets the time: no gain (15.3 us). Non-final passes write their top 64 (a
-// superset of the top k); the final pass writes the first k as ids and values. Cost does
-// not depend on k. 8 rows of 128256 f32 logits, k = 40, first and last pass:
-// 15.1 + 8.3 us sorted, 6.8 + 5.9 filtered.
-constexpr int kSortWaves = 16, kSortThreads = kSortWaves * kLanes, kSortChunk = kSortThreads * kPerLane;
-constexpr int kSurvivors = 512, kGroups = kSortThreads / 4, kBoundBits = 18;
+// filtering and counting. The lanes' quads are 256 groups of up to 16 keys; a bound that 64 of
+// the groups' maxima reach is one that at least 64 keys reach, so only the keys that reach it
+// can be among the top 64. The largest value (a key's high word) that serves, to its top
+// kBoundBits, is found bit by bit with ballots (by one wave: the counting is scalar work, and a
+// CU has one scalar unit for its 16 waves): 70 to 90 of a full block's keys reach it in any
+// order that does not depend on the position. They are compacted into LDS (in any order) and
+// each one's rank is the number of larger ones, counted by 1024 / slots threads per key; keys
+// are distinct, so the ranks are too. Keys of an earlier pass arrive as sorted runs of 64: quad
+// q of a wave takes a run's places q mod 16, so the groups' maxima are the runs' leading keys.
+// Where more than kRanked keys reach the bound (a masked row: most logits one value) it is found
+// again to the last bit of the key, value and id: then exactly 64 groups reach it, which hold at
+// most 1024 keys. (Ranking costs 1.7 us for 256 keys, 2.9 for 260 and 7 for 500; finding the
+// bound again and ranking what is left about 4.) Where more than kRanked of those do, they are
+// one per lane, so quads of them are groups of 4 and the same bound over these leaves at most
+// 256. Non-final passes write their top 64 (a superset of the top k); the final pass writes the
+// first k as ids and values. Cost does not depend on k. 8 rows of 128256 f32 logits, k = 40,
+// both passes: a bitonic sort of the block's keys 21.4 us for any values; this 10.3 (N(0, 1)),
+// 18.3 (all but 50 logits -inf) and 21.3 (values that repeat every 256 logits, filtered twice).
+constexpr int kFilterWaves = 16, kFilterThreads = kFilterWaves * kLanes, kFilterChunk = kFilterThreads * kPerLane;
+constexpr int kRanked = 320, kSlots = 512, kGroups = kFilterThreads / 4, kBoundBits = 18;
 static_assert(kGroups == 4 * kLanes, "four groups per lane");
-
-__device__ __forceinline__ void merge4(uint64_t (&a)[4], const uint64_t (*lists)[kLanes], int lane) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int e = 4 * lane + r;
-        a[r] = lists[e >> 6][e & 63];
-    }
-    bitonic256<128>(a, lane);
-}
-
-__device__ __forceinline__ void put_top64(const uint64_t (&a)[4], uint64_t* list, bool reversed, int lane) {
-    if (lane < 16) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int e = 4 * lane + r;
-            list[reversed ? 63 - e : e] = a[r];
-        }
-    }
-}
 
 // The largest value over each quad of lanes, in all of them.
 __device__ __forceinline__ uint32_t quad_max_u32(uint32_t v) {
@@ -218,25 +143,103 @@ __device__ __forceinline__ uint32_t quad_max_u32(uint32_t v) {
     return dpp_step<true>(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x4E, 0xF, 0xF, false));
 }
 
-// Block s: inputs [s * chunk, min(n, (s + 1) * chunk)) of token row m, chunk <= kSortChunk.
+// One wave, four groups per lane: the largest number that 64 of the groups' reach and that has
+// from's bits above hi and zeros below lo (from itself is reached by 64).
+__device__ __forceinline__ uint32_t reached_by_64(const uint4& g, uint32_t from, int hi, int lo) {
+    for (int b = hi; b >= lo; --b) {
+        const uint32_t v = from | 1u << b;
+        const int reach = __popcll(__ballot(g.x >= v)) + __popcll(__ballot(g.y >= v)) + __popcll(__ballot(g.z >= v)) +
+                          __popcll(__ballot(g.w >= v));
+        if (reach >= kLanes) from = v;
+    }
+    return from;
+}
+
+struct FilterLds {
+    alignas(16) uint64_t found[kFilterThreads];  // the keys that reach the bound, zeros behind them
+    alignas(16) uint32_t high[kGroups], low[kGroups];   // the groups' maxima
+    uint64_t top[kLanes], bound;
+    int rank[kSlots], count[3];
+};
+
+// The largest key that 64 of the groups' maxima reach, the threads' keys a in quads; the `known`
+// leading bits of its value are those of from. found is cleared. Every thread calls it (barriers
+// inside).
+template <int N>
+__device__ __forceinline__ uint64_t exact_bound(const uint64_t (&a)[N], uint32_t from, int known, FilterLds& m) {
+    const int tid = threadIdx.x;
+    uint32_t high = 0, low = 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j) high = dpp_step<true>(high, (uint32_t)(a[j] >> 32));
+    high = quad_max_u32(high);
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+        if ((uint32_t)(a[j] >> 32) == high) low = dpp_step<true>(low, (uint32_t)a[j]);
+    low = quad_max_u32(low);
+    if ((tid & 3) == 0) m.high[tid >> 2] = high, m.low[tid >> 2] = low;
+    __syncthreads();
+    m.found[tid] = 0;
+    if (tid < kLanes) {
+        const uint4 g = *(const uint4*)(m.high + 4 * tid);
+        uint4 l = *(const uint4*)(m.low + 4 * tid);
+        const uint32_t v = reached_by_64(g, from, 31 - known, 0);
+        // fewer than 64 lead with more: the id's word is among those that lead with v, and has the
+        // bits that these share
+        uint32_t most = 0, least = ~0u;
+        auto leading = [&](uint32_t gv, uint32_t& lv) {
+            if (gv == v) most = dpp_step<true>(most, lv), least = dpp_step<false>(least, lv);
+            else lv = gv > v ? ~0u : 0u;
+        };
+        leading(g.x, l.x), leading(g.y, l.y), leading(g.z, l.z), leading(g.w, l.w);
+        most = wave_reduce_u32<true>(most), least = wave_reduce_u32<false>(least);
+        const int hi = 31 - __builtin_clz((most ^ least) | 1u);
+        const uint32_t i = reached_by_64(l, most & ~((2u << hi) - 1u), hi, 0);
+        if (tid == 0) m.bound = (uint64_t)v << 32 | i;
+    }
+    __syncthreads();
+    return m.bound;
+}
+
+// The keys that reach the bound (padding, key 0, never does) into found; their number, counted in
+// count (zero before). Every thread calls it (a barrier inside).
+template <int N>
+__device__ __forceinline__ int collect(const uint64_t (&a)[N], uint64_t bound, FilterLds& m, int* count) {
+    const int lane = threadIdx.x & (kLanes - 1);
+    uint64_t hit[N];
+    int c = 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        hit[j] = __ballot(a[j] != 0 && a[j] >= bound);
+        c += __popcll(hit[j]);
+    }
+    int o = 0;
+    if (lane == 0 && c) o = atomicAdd(count, c);
+    o = __builtin_amdgcn_readfirstlane(o);
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const int to = o + __popcll(hit[j] & ((1ull << lane) - 1ull));
+        if ((hit[j] >> lane & 1) && to < kFilterThreads) m.found[to] = a[j];
+        o += __popcll(hit[j]);
+    }
+    __syncthreads();
+    return *count;
+}
+
+// Block s: inputs [s * chunk, min(n, (s + 1) * chunk)) of token row m, chunk <= kFilterChunk.
 template <bool KEYS, bool FINAL>
-__global__ __launch_bounds__(kSortThreads) void topk_sort_kernel(const void* __restrict__ in, int64_t ld, int64_t n,
-                                                                 int chunk, int k, int mode,
-                                                                 uint64_t* __restrict__ out_keys,
-                                                                 int32_t* __restrict__ ids,
-                                                                 float* __restrict__ vals) {
-    __shared__ uint64_t l1[kSortWaves][kLanes], l2[4][kLanes], top[kLanes];
-    __shared__ __attribute__((aligned(16))) uint64_t surv[kSurvivors];
-    __shared__ int rank[kSurvivors];
-    __shared__ __attribute__((aligned(16))) uint32_t group_max[kGroups];
-    __shared__ int count;
+__global__ __launch_bounds__(kFilterThreads) void topk_filter_kernel(const void* __restrict__ in, int64_t ld,
+                                                                     int64_t n, int chunk, int k, int mode,
+                                                                     uint64_t* __restrict__ out_keys,
+                                                                     int32_t* __restrict__ ids,
+                                                                     float* __restrict__ vals) {
+    __shared__ FilterLds lds;
     const int tid = threadIdx.x, lane = tid & (kLanes - 1), wave = tid / kLanes;
     const int64_t s = blockIdx.x, m = blockIdx.y, base = s * chunk;
     const int at = wave * kLanes + (KEYS ? (lane >> 2) + 16 * (lane & 3) : lane);
     uint64_t a[kPerLane];
 #pragma unroll
     for (int j = 0; j < kPerLane; ++j) {
-        const int o = j * kSortThreads + at;
+        const int o = j * kFilterThreads + at;
         const int64_t i = base + o;
         if (o < chunk && i < n) {
             if constexpr (KEYS)
@@ -247,87 +250,59 @@ __global__ __launch_bounds__(kSortThreads) void topk_sort_kernel(const void* __r
             a[j] = 0;
         }
     }
-    if (tid < kSurvivors) surv[tid] = 0, rank[tid] = 0;
-    if (tid < kLanes) top[tid] = 0;
-    if (tid == 0) count = 0;
-    uint32_t big = 0;
+    lds.found[tid] = 0;
+    if (tid < kSlots) lds.rank[tid] = 0;
+    if (tid < kLanes) lds.top[tid] = 0;
+    if (tid < 3) lds.count[tid] = 0;
+    uint32_t high = 0;
 #pragma unroll
-    for (int j = 0; j < kPerLane; ++j) big = dpp_step<true>(big, (uint32_t)(a[j] >> 32));
-    big = quad_max_u32(big);
-    if ((lane & 3) == 0) group_max[tid >> 2] = big;
+    for (int j = 0; j < kPerLane; ++j) high = dpp_step<true>(high, (uint32_t)(a[j] >> 32));
+    high = quad_max_u32(high);
+    if ((lane & 3) == 0) lds.high[tid >> 2] = high;
     __syncthreads();
-    const uint4 g = *(const uint4*)(group_max + 4 * lane);
-    uint32_t bound = 0;
-#pragma unroll
-    for (int b = 31; b > 31 - kBoundBits; --b) {
-        const uint32_t v = bound | 1u << b;
-        const int reach = __popcll(__ballot(g.x >= v)) + __popcll(__ballot(g.y >= v)) + __popcll(__ballot(g.z >= v)) +
-                          __popcll(__ballot(g.w >= v));
-        if (reach >= kLanes) bound = v;
-    }
-    // the keys that reach the bound (padding, key 0, never does)
-    uint64_t hit[kPerLane];
-    int c = 0;
-#pragma unroll
-    for (int j = 0; j < kPerLane; ++j) {
-        hit[j] = __ballot(a[j] != 0 && (uint32_t)(a[j] >> 32) >= bound);
-        c += __popcll(hit[j]);
-    }
-    int o = 0;
-    if (lane == 0 && c) o = atomicAdd(&count, c);
-    o = __builtin_amdgcn_readfirstlane(o);
-#pragma unroll
-    for (int j = 0; j < kPerLane; ++j) {
-        const int to = o + __popcll(hit[j] & ((1ull << lane) - 1ull));
-        if ((hit[j] >> lane & 1) && to < kSurvivors) surv[to] = a[j];
-        o += __popcll(hit[j]);
+    if (wave == 0) {
+        const uint32_t v = reached_by_64(*(const uint4*)(lds.high + 4 * lane), 0, 31, 32 - kBoundBits);
+        if (lane == 0) lds.bound = (uint64_t)v << 32;
     }
     __syncthreads();
-    const int total = count;
-    if (total <= kSurvivors) {
-        // thread (slot, part): the larger keys among part's share of the survivors (an even
-        // number from an even place; the zeros behind the last one count for none)
-        const int slots = total <= kSurvivors / 4 ? kSurvivors / 4 : total <= kSurvivors / 2 ? kSurvivors / 2 : kSurvivors;
-        const int parts = kSortThreads / slots;
-        const int slot = tid & (slots - 1), part = tid / slots;
-        const int share = ((total + parts - 1) / parts + 1) & ~1;
-        const int j0 = min(part * share, total), j1 = min(j0 + share, total);
-        const uint64_t key = surv[slot];
-        int larger = 0;
-        if ((slot & ~(kLanes - 1)) < total) {                 // wave-uniform
+    const uint64_t bound = lds.bound;
+    int total = collect(a, bound, lds, &lds.count[0]);
+    if (total > kRanked) {
+        total = collect(a, exact_bound(a, (uint32_t)(bound >> 32), kBoundBits, lds), lds, &lds.count[1]);
+        if (total > kRanked) {
+            const uint64_t one[1] = {lds.found[tid]};
+            total = collect(one, exact_bound(one, 0, 0, lds), lds, &lds.count[2]);
+        }
+    }
+    // thread (slot, part): the larger keys among part's share of those found (an even number
+    // from an even place; the zeros behind the last one count for none)
+    const int slots = total <= kSlots / 4 ? kSlots / 4 : total <= kSlots / 2 ? kSlots / 2 : kSlots;
+    const int parts = kFilterThreads / slots;
+    const int slot = tid & (slots - 1), part = tid / slots;
+    const int share = ((total + parts - 1) / parts + 1) & ~1;
+    const int j0 = min(part * share, total), j1 = min(j0 + share, total);
+    const uint64_t key = lds.found[slot];
+    int larger = 0;
+    if ((slot & ~(kLanes - 1)) < total) {                 // wave-uniform
 #pragma unroll 4
-            for (int j = j0; j < j1; j += 2) {
-                const ulonglong2 v = *(const ulonglong2*)(surv + j);
-                larger += (v.x > key) + (v.y > key);
-            }
-            atomicAdd(&rank[slot], larger);
+        for (int j = j0; j < j1; j += 2) {
+            const ulonglong2 v = *(const ulonglong2*)(lds.found + j);
+            larger += (v.x > key) + (v.y > key);
         }
-        __syncthreads();
-        if (tid < total && rank[tid] < kLanes) top[rank[tid]] = surv[tid];
-    } else {
-        bitonic256<2>(a, lane);
-        put_top64(a, l1[wave], wave & 1, lane);
-        __syncthreads();
-        if (wave < 4) {
-            merge4(a, l1 + 4 * wave, lane);
-            put_top64(a, l2[wave], wave & 1, lane);
-        }
-        __syncthreads();
-        if (wave == 0) {
-            merge4(a, l2, lane);
-            put_top64(a, top, false, lane);
-        }
+        atomicAdd(&lds.rank[slot], larger);
     }
+    __syncthreads();
+    if (tid < total && lds.rank[tid] < kLanes) lds.top[lds.rank[tid]] = lds.found[tid];
     __syncthreads();
     if (wave != 0) return;
-    const uint64_t key = top[lane];
+    const uint64_t out = lds.top[lane];
     if constexpr (FINAL) {
         if (lane < k) {
-            ids[m * k + lane] = key ? (int32_t)~(uint32_t)key : -1;
-            if (vals) vals[m * k + lane] = key ? from_monotone((uint32_t)(key >> 32)) : -__builtin_inff();
+            ids[m * k + lane] = out ? (int32_t)~(uint32_t)out : -1;
+            if (vals) vals[m * k + lane] = out ? from_monotone((uint32_t)(out >> 32)) : -__builtin_inff();
         }
     } else {
-        out_keys[(m * gridDim.x + s) * kLanes + lane] = key;
+        out_keys[(m * gridDim.x + s) * kLanes + lane] = out;
     }
 }
 
@@ -374,7 +349,7 @@ __global__ __launch_bounds__(kThreads) void topk_kernel(const void* __restrict__
     }
 }
 
-constexpr int kPopMaxK = 8;     // k above this: the sorting-network block
+constexpr int kPopMaxK = 8;     // k above this: the filtering block
 
 // Pass geometry: inputs per block and keys each non-final block writes.
 struct TopkPlan {
@@ -384,7 +359,7 @@ struct TopkPlan {
 };
 
 inline TopkPlan topk_plan(int k) {
-    return k <= kPopMaxK ? TopkPlan{true, kChunk, k} : TopkPlan{false, kSortChunk, 64};
+    return k <= kPopMaxK ? TopkPlan{true, kChunk, k} : TopkPlan{false, kFilterChunk, 64};
 }
 
 template <bool KEYS>
@@ -401,10 +376,10 @@ void launch_topk(const TopkPlan& p, bool final_pass, dim3 grid, hipStream_t st, 
         // even chunks, whole runs of 64: a short last block would pass its group bound too easily
         const int chunk = (int)(ceil_div(ceil_div(n, (int64_t)grid.x), (int64_t)kLanes) * kLanes);
         if (final_pass)
-            hipLaunchKernelGGL((topk_sort_kernel<KEYS, true>), grid, dim3(kSortThreads), 0, st, in, ld, n, chunk, k,
+            hipLaunchKernelGGL((topk_filter_kernel<KEYS, true>), grid, dim3(kFilterThreads), 0, st, in, ld, n, chunk, k,
                                mode, out_keys, ids, vals);
         else
-            hipLaunchKernelGGL((topk_sort_kernel<KEYS, false>), grid, dim3(kSortThreads), 0, st, in, ld, n, chunk, k,
+            hipLaunchKernelGGL((topk_filter_kernel<KEYS, false>), grid, dim3(kFilterThreads), 0, st, in, ld, n, chunk, k,
                                mode, out_keys, ids, vals);
     }
 }
