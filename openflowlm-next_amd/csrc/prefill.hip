@@ -90,15 +90,15 @@ __device__ __forceinline__ u32x4 dequant8(uint32_t w, uint32_t s, uint32_t nib2,
 // 2^(s_t + e_n) when the operands were scaled (texp / wexp not null), exactly; accum adds
 // the result to what y holds (the second pass of f32 activations). tmap: token t's exponent
 // is texp[tmap[t]] (activations gathered from another row order), else texp[t].
-// Token fragment j starts 64 j tokens after wt0.
-template <int FN, int FT, bool SCALED>
+// Token fragment j starts TS j tokens after wt0.
+template <int FN, int FT, int TS, bool SCALED>
 __device__ __forceinline__ void store_tile(const f32x4 (&acc)[FN][FT], float* __restrict__ y,
                                            const int* __restrict__ texp, const int* __restrict__ wexp, int T, int N,
                                            int wt0, int wn0, int accum, const int* __restrict__ tmap = nullptr) {
     const int lane = threadIdx.x & 63, i16 = lane & 15, kg = lane >> 4;
 #pragma unroll
     for (int j = 0; j < FT; ++j) {
-        const int t = wt0 + j * 64 + i16;
+        const int t = wt0 + j * TS + i16;
         if (t >= T) continue;
         const int st = SCALED ? texp[tmap ? max(tmap[t], 0) : t] : 0;
 #pragma unroll
@@ -125,8 +125,8 @@ __device__ __forceinline__ void store_tile(const f32x4 (&acc)[FN][FT], float* __
 // gate rows (from wn0), the others the up rows 64 further on, at the same lane positions, so
 // h = bf16(silu(g) * u) (q4_swiglu_prepare's arithmetic) is formed from the accumulators and
 // only h [T][F] bf16 is stored: the f32 gate/up output never reaches memory. Token fragment j
-// starts at wt0 + 64 j.
-template <int FN, int FT, bool SCALED>
+// starts at wt0 + TS j.
+template <int FN, int FT, int TS, bool SCALED>
 __device__ __forceinline__ void store_swiglu(const f32x4 (&acc)[FN][FT], uint16_t* __restrict__ h,
                                              const int* __restrict__ texp, const int* __restrict__ wexp, int T, int N,
                                              int wt0, int wn0, const int* __restrict__ tmap = nullptr) {
@@ -134,7 +134,7 @@ __device__ __forceinline__ void store_swiglu(const f32x4 (&acc)[FN][FT], uint16_
     const int F = N >> 1, f0 = (wn0 >> 7) * 64 + (wn0 & 127);   // wn0 = 128 p + c: gate rows from 64 p + c
 #pragma unroll
     for (int j = 0; j < FT; ++j) {
-        const int t = wt0 + j * 64 + i16;
+        const int t = wt0 + j * TS + i16;
         if (t >= T) continue;
         const int st = SCALED ? texp[tmap ? max(tmap[t], 0) : t] : 0;
 #pragma unroll
@@ -238,10 +238,12 @@ __device__ __forceinline__ void vgpr_landed(u32x4& v) { asm volatile("" : "+v"(v
 // writes its partial sums to y + s * T * N; the host sums the splits in order).
 // KBS: 32-K blocks per stage. A stage always holds eight mx tiles, one per wave, so the row
 // tile narrows as the stage deepens: KBS = 2: 256 rows x 64 K, KBS = 4: 128 rows x 128 K.
-// Waves are 2 along N x 4 along T. A wave's weight rows are [16 FN wn, +16 FN), its token
-// fragments the 16-token groups wt, wt + 4, ... (FT of them), so a tile with few valid tokens
-// (the ragged last tile of T, an expert's tokens) runs an instance with a smaller FT in which
-// every wave does the same, smaller share of the MFMAs, fragment reads and DMA.
+// Waves are 2 along N x 4 along T. A wave's weight rows are [16 FN wn, +16 FN), its tokens FT
+// groups of 16: a tile with few valid tokens (the ragged last tile of T, an expert's tokens) runs
+// an instance with a smaller FT in which every wave does the same, smaller share of the MFMAs,
+// fragment reads and DMA. Its groups are wt, wt + 4, ... there, which spreads the valid tokens
+// and their stores over the waves; a full tile's lie together, FT wt, FT wt + 1, ... (64
+// apart, the stores of 512 tokens on 4096 x 14336 made the call 1.09 times as long).
 // KBS = 2, FN = 8: 256 rows. FN = 6: 192 rows, with the 256-row tile's loads, DMA and dequant
 // unchanged: the waves of row group 3 load row group 2's mx tile again and store it to LDS
 // rows 192..255, which no fragment reads, so every wave issues the same loads and the wait
@@ -281,6 +283,8 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
     constexpr int WPB = RGS * 64 * 64;               // one 32-K plane of the weight buffer
     constexpr int XPB = FT * 64 * 64;                // one 32-K plane of an activation slot
     constexpr int XD = FT * KBS / 2;                 // activation DMAs per wave and stage
+    constexpr bool kFull = FT * KBS == 8;
+    constexpr int TS = kFull ? 16 : 64, TW = kFull ? 16 * FT : 16;   // tokens from fragment to fragment, wave to wave
     typedef typename std::conditional<PREC == 0, f16x8, bf16x8>::type frag_t;
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -307,9 +311,11 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
     // activations: pre-tiled as the LDS image of each stage ([256-token tile][32-K plane][256
     // rows], 16 KB per plane, zero-padded to whole 64-token groups); this wave copies the units
     // XD wave .. + XD of the stage, unit u = 16-row group u / KBS of plane u % KBS.
-    const uint8_t* const xsrc = (const uint8_t*)x16 + (((int64_t)(t0 >> 8) * KB + KBS * st0) * kPlaneB + (t0 & 255) * 64);
+    const int unit0 = XD * wave / KBS;
+    const uint8_t* const xsrc = (const uint8_t*)x16 +
+                                (((int64_t)(t0 >> 8) * KB + KBS * st0) * kPlaneB + (t0 & 255) * 64 + unit0 * 1024);
     const uint32_t xoff = lane * 16;
-    const uint32_t xdst = (uint32_t)(uintptr_t)lds + kXRing;            // LDS byte address
+    const uint32_t xdst = (uint32_t)(uintptr_t)lds + kXRing + unit0 * 1024;   // LDS byte address
     // GATHER: the byte offset of this lane's chunk in its token row of each unit (row lane / 4
     // of the group; LDS slot lane & 3 holds chunk (lane & 3) ^ ((lane >> 3) & 3))
     constexpr int GQ = FT % 2 ? 1 : KBS;             // units of a wave that share a row group
@@ -326,10 +332,10 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
         }
     }
 
-    // fragment bases: A = weight rows (frag_row), B = token rows 64 j + 16 wt + i16
+    // fragment bases: A = weight rows, B = token rows TW wt + TS j + i16
     constexpr bool kPair = SWI && KBS == 4;
     const uint32_t abase = (kPair ? wn * 32 : wn * WN) * 64 + lane_row;
-    const uint32_t bbase = kXRing + wt * 1024 + lane_row;
+    const uint32_t bbase = kXRing + wt * TW * 64 + lane_row;
     const uint32_t bbase2 = bbase + 2 * kTileB;                         // ring slot 2 (offset > 64 KB)
     const uint32_t nib2 = vgpr_const(kNib2);
     const uint32_t magic = vgpr_const(PREC == 0 ? kMagic1024 : kMagic128);
@@ -344,8 +350,9 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
     auto issue_x = [&](int st, int slot) {
 #pragma unroll
         for (int q = 0; q < XD; ++q) {
-            const int u = XD * wave + q;                                // uniform
-            const int unit = u / KBS, plane = u % KBS;
+            // the wave's unit q, from the first row group that the wave's units touch
+            const int plane = XD % KBS ? (XD * wave + q) % KBS : q % KBS;
+            const int unit = XD % KBS ? (XD * wave + q) / KBS - XD * wave / KBS : q / KBS;
             const uint32_t dst = xdst + slot * kTileB + plane * XPB + unit * 1024;
             if constexpr (GATHER)
                 lds_dma16_buf(xrs, goff[q / GQ], (uint32_t)(KBS * (st0 + st) + plane) * 64, dst);
@@ -354,7 +361,7 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
                                                                 (int)kGatherBytes, kBufferWord3),
                               KBS * (st0 + st) + plane < KB ? xoff : kPadOffset, plane * kPlaneB + unit * 1024, dst);
             else
-                lds_dma16(xsrc + ((int64_t)(KBS * st + plane) * kPlaneB + unit * 1024), xoff, dst);
+                lds_dma16(xsrc + (int64_t)st * (KBS * kPlaneB) + (plane * kPlaneB + unit * 1024), xoff, dst);
         }
     };
     auto issue_w = [&](int st, u32x4& c, u32x4& sc) {
@@ -378,7 +385,7 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
         const uint8_t* xp = lds + (slot == 2 ? bbase2 : bbase + slot * kTileB) + kk * XPB;
         const uint8_t* wp = lds + abase + buf * kTileB + kk * WPB;
 #pragma unroll
-        for (int j = 0; j < FT; ++j) b[j] = *(const frag_t*)(xp + j * 4096);
+        for (int j = 0; j < FT; ++j) b[j] = *(const frag_t*)(xp + j * TS * 64);
 #pragma unroll
         for (int i = 0; i < FN; ++i) a[i] = *(const frag_t*)(wp + (kPair ? (i >> 1) * 4096 + (i & 1) * 1024 : i * 1024));
     };
@@ -476,10 +483,10 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
     // gathered activations carry their exponents by source row
     const int* tmap = GATHER ? gmap : nullptr;
     if constexpr (SWI)
-        store_swiglu<FN, FT, PREC == 0>(acc, (uint16_t*)y, texp, wexp, T, N, t0 + wt * 16,
+        store_swiglu<FN, FT, TS, PREC == 0>(acc, (uint16_t*)y, texp, wexp, T, N, t0 + wt * TW,
                                         n0 + (kPair ? wn * 32 : wn * WN), tmap);
     else
-        store_tile<FN, FT, PREC == 0>(acc, y, texp, wexp, T, N, t0 + wt * 16, n0 + wn * WN, accum, tmap);
+        store_tile<FN, FT, TS, PREC == 0>(acc, y, texp, wexp, T, N, t0 + wt * TW, n0 + wn * WN, accum, tmap);
 }
 
 // dma_tile with the smallest token tile that covers the valid tokens [t0, T) of a tile of
