@@ -1008,23 +1008,45 @@ void launch_prefill(int tile, int64_t grid, hipStream_t st, const uint8_t* w, co
 }
 
 // y = sum of the S partials in split order (deterministic), 4 floats per thread; accum adds
-// it to what y holds. Eight planes' loads go out together: one load behind the other took 0.5
-// to 0.9 us longer per call (T = 64, N = 2048, 8 planes: 4.3 -> 3.4 us).
+// it to what y holds. S > 0: all planes' loads go out together; S = 0: `splits` of them, one
+// behind the other.
+template <int S>
 __global__ __launch_bounds__(256) void prefill_reduce_kernel(const f32x4* __restrict__ part, f32x4* __restrict__ y,
-                                                             int64_t MN4, int S, int accum) {
+                                                             int64_t MN4, int splits, int accum) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= MN4) return;
-    constexpr int B = 8;
     f32x4 s;
-    for (int q = 0; q < S; q += B) {
-        f32x4 t[B];
+    if constexpr (S > 0) {
+        f32x4 t[S];
 #pragma unroll
-        for (int u = 0; u < B; ++u) t[u] = part[(int64_t)min(q + u, S - 1) * MN4 + i];
+        for (int q = 0; q < S; ++q) t[q] = part[(int64_t)q * MN4 + i];
+        s = t[0];
 #pragma unroll
-        for (int u = 0; u < B; ++u)
-            if (q + u < S) s = q + u == 0 ? t[u] : s + t[u];
+        for (int q = 1; q < S; ++q) s += t[q];
+    } else {
+        s = part[i];
+        for (int q = 1; q < splits; ++q) s += part[(int64_t)q * MN4 + i];
     }
     y[i] = accum ? y[i] + s : s;
+}
+
+constexpr int kMaxSplits = 16;
+
+// Whether a thread's loads of all planes go out together. Small planes wait for latency (16 of
+// 25 x 4096 f32: 4.9 us one behind the other, 2.9 together; 8 of 300 x 4096, 39 MB: 7.2 and 5.9),
+// planes past the caches for memory, which many open streams slow down (8 of 512 x 4096,
+// 67 MB: 11.5 and 14.4; 5 of 640 x 4096, 52 MB: 10.0 and 10.1).
+bool planes_together(int planes, int64_t TN) { return planes * TN * 4 <= (int64_t)48 << 20; }
+
+template <int S = kMaxSplits>
+void launch_reduce(int splits, hipStream_t st, const float* part, float* y, int64_t TN, int accum) {
+    auto launch = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(TN / 4, 256)), dim3(256), 0, st, (const f32x4*)part,
+                           (f32x4*)y, TN / 4, splits, accum);
+    };
+    if (!planes_together(splits, TN)) launch(prefill_reduce_kernel<0>);
+    else if (splits == S) launch(prefill_reduce_kernel<S>);
+    else if constexpr (S > 2) launch_reduce<S - 1>(splits, st, part, y, TN, accum);
 }
 
 // CUs of the current device (the MI355X's 256 when no device is visible, e.g. for a
@@ -1300,9 +1322,7 @@ int gemm_pass(const uint8_t* packed, const void* scales, const uint16_t* x16, co
                           plan.tiles_t, plan.splits, plan.wide_wgs, plan.narrow_row0, accum);
     if (launch_status() != Q4MI_OK) return Q4MI_E_LAUNCH;
     if (plan.splits > 1) {
-        const int64_t MN4 = (int64_t)T * N / 4;
-        hipLaunchKernelGGL(prefill_reduce_kernel, dim3((unsigned)ceil_div(MN4, 256)), dim3(256), 0, st,
-                           (const f32x4*)out, (f32x4*)y, MN4, plan.splits, pass);
+        launch_reduce(plan.splits, st, out, y, (int64_t)T * N, pass);
         if (launch_status() != Q4MI_OK) return Q4MI_E_LAUNCH;
     }
     return Q4MI_OK;
