@@ -837,15 +837,18 @@ __global__ __launch_bounds__(256) void prefill_xprep(const void* __restrict__ x,
 // 8 MB each), so a thread takes PER / 4 groups of four neighbouring values and issues all of a
 // row's loads, PB planes at a time, before the first is used (16 bytes each; vec 0: some pointer
 // is not 16-byte aligned, four 4-byte loads). One plane and one value at a time, each behind the
-// last, took 29.7 us at five planes, this 14.7 (4.3 TB/s). The row also goes to LDS, from which thread
+// last, took 29.4 us at five planes, this 13.3; K = 14336 with two planes 55.4 and 34.7. PER fits K, and
+// PB is 1 for one plane or planes past the caches: registers and loads of values that are not
+// there cost a wave more than they hide (T = 2048, K = 1024, one plane: 9.6 us before, 11.5 with PER =
+// 16 and PB = 4 for it too, 7.3 now; K = 4096 20.2, 21.6 and 20.3). The row also goes to LDS, from which thread
 // tid sums the squares of elements tid + 256 j, j ascending, as rmsnorm_add_kernel does (values
 // past K are zeros there and are skipped here: the fp64 sum is the same).
-template <int PER, int PREC>
+template <int PER, int PREC, int PB>
 __global__ __launch_bounds__(256) void rmsnorm_prepare_kernel(const float* x, const float* __restrict__ add,
                                                               int add_planes, const void* __restrict__ w, int w_bf16,
                                                               int vec, float* y, uint16_t* __restrict__ x16,
                                                               int* __restrict__ texp, int T, int K, float eps) {
-    constexpr int C = PER / 4, PB = PER <= 16 ? 4 : PER <= 32 ? 2 : 1;
+    constexpr int C = PER / 4;
     __shared__ double part[4];
     __shared__ __attribute__((aligned(16))) float row[256 * PER];   // f32 x, then the bf16 xn
     uint16_t* const xs = (uint16_t*)row;
@@ -881,10 +884,11 @@ __global__ __launch_bounds__(256) void rmsnorm_prepare_kernel(const float* x, co
                 f32x4 a[PB][C];
 #pragma unroll
                 for (int u = 0; u < PB; ++u)
+                    if (q0 + u < add_planes) {
 #pragma unroll
-                    for (int c = 0; c < C; ++c)
-                        a[u][c] = ld4(ar + (int64_t)min(q0 + u, add_planes - 1) * pstride +
-                                      min(4 * (tid + 256 * c), K - 4));
+                        for (int c = 0; c < C; ++c)
+                            a[u][c] = ld4(ar + (int64_t)(q0 + u) * pstride + min(4 * (tid + 256 * c), K - 4));
+                    }
 #pragma unroll
                 for (int u = 0; u < PB; ++u)
                     if (q0 + u < add_planes) {
@@ -1455,19 +1459,28 @@ extern "C" int q4_rmsnorm_prepare(const float* x, const float* add, int add_plan
     const dim3 grid((unsigned)padded_tokens(T)), block(256);
     const hipStream_t st = (hipStream_t)stream;
     const int wb = w_dtype == Q4MI_BF16;
+    const bool one = !add || add_planes == 1 || !planes_together(add_planes, (int64_t)T * K);
     const int vec = !misaligned16(x) && !misaligned16(add) && !misaligned16(w) && !misaligned16(y);
-#define Q4MI_RP(PER, PR)                                                                                            \
-    hipLaunchKernelGGL((rmsnorm_prepare_kernel<PER, PR>), grid, block, 0, st, x, add, add_planes, w, wb, vec, y, x16, \
+#define Q4MI_RP(PER, PR, PB)                                                                                           \
+    hipLaunchKernelGGL((rmsnorm_prepare_kernel<PER, PR, PB>), grid, block, 0, st, x, add, add_planes, w, wb, vec, y, x16, \
                        te, T, (int)K, eps)
-#define Q4MI_RP_K(PR)                               \
-    do {                                            \
-        if (K <= 256 * 16) Q4MI_RP(16, PR);         \
-        else if (K <= 256 * 32) Q4MI_RP(32, PR);    \
-        else Q4MI_RP(64, PR);                       \
+#define Q4MI_RP_P(PER, PR, PB)                                                    \
+    {                                                                             \
+        if (one) Q4MI_RP(PER, PR, 1);                                             \
+        else Q4MI_RP(PER, PR, PB);                                                \
+    }
+#define Q4MI_RP_K(PR)                                       \
+    do {                                                    \
+        if (K <= 256 * 4) Q4MI_RP_P(4, PR, 4)               \
+        else if (K <= 256 * 8) Q4MI_RP_P(8, PR, 4)          \
+        else if (K <= 256 * 16) Q4MI_RP_P(16, PR, 4)        \
+        else if (K <= 256 * 32) Q4MI_RP_P(32, PR, 2)        \
+        else Q4MI_RP(64, PR, 1);                            \
     } while (0)
     if (precision == 0) Q4MI_RP_K(0);
     else Q4MI_RP_K(1);
 #undef Q4MI_RP_K
+#undef Q4MI_RP_P
 #undef Q4MI_RP
     return launch_status();
 }

@@ -18,13 +18,7 @@ def _rows(gpu, T, K, shift, seed):
     return buf[shift:shift + T * K].view(T, K)
 
 
-@pytest.mark.parametrize("shift", [0, 1])
-@pytest.mark.parametrize("K", [32, 992, 4096, 4128, 8192, 8224, 16384])
-@pytest.mark.parametrize("planes", [0, 1, 2, 4, 5, 9])
-@pytest.mark.parametrize("wdt", [torch.bfloat16, torch.float32])
-def test_planes_and_alignment(gpu, pkg, K, planes, shift, wdt):
-    say(f"rmsnorm_prepare loads K={K} planes={planes} shift={shift} {wdt}")
-    T = 3
+def _check(gpu, pkg, T, K, planes, shift, wdt):
     x = _rows(gpu, T, K, shift, 1)
     add = _rows(gpu, planes * T, K, shift, 2).view(planes, T, K) if planes else None
     w = _rows(gpu, 1, K, shift, 3).view(-1).to(wdt)
@@ -45,3 +39,21 @@ def test_planes_and_alignment(gpu, pkg, K, planes, shift, wdt):
     torch.cuda.synchronize()
     assert torch.equal(got_y, ref_y)
     assert torch.equal(got.data, ref.data)
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("K", [32, 992, 1024, 1056, 2048, 2080, 4096, 4128, 8192, 8224, 16384])
+@pytest.mark.parametrize("planes", [0, 1, 2, 4, 5, 9])
+@pytest.mark.parametrize("wdt", [torch.bfloat16, torch.float32])
+def test_planes_and_alignment(gpu, pkg, K, planes, shift, wdt):
+    say(f"rmsnorm_prepare loads K={K} planes={planes} shift={shift} {wdt}")
+    _check(gpu, pkg, 3, K, planes, shift, wdt)
+
+
+# 48 MiB of planes and one row more: loaded together, then one behind the other
+@pytest.mark.parametrize("K,planes", [(1024, 6), (2048, 3), (4096, 2), (8192, 3), (16384, 2)])
+@pytest.mark.parametrize("more", [0, 1])
+def test_planes_past_the_caches(gpu, pkg, K, planes, more):
+    T = (48 << 20) // (planes * K * 4) + more
+    say(f"rmsnorm_prepare loads T={T} K={K} planes={planes}")
+    _check(gpu, pkg, T, K, planes, 0, torch.bfloat16)
