@@ -551,6 +551,11 @@ int q4_rmsnorm_prepare(const float* x, const float* add, int add_planes, const v
 /* The K splits the prefill GEMM's plan takes for (T, N, K) (1: unsplit), 0 for bad shapes. */
 int q4_prefill_split_count(int T, int64_t N, int64_t K);
 
+/* The rows of the tiles that plan takes: 128, 256, or 192 (192-row tiles beside any 256-row
+ * ones); swiglu != 0: of q4_gemm_prefill_swiglu's over its N = 2F rows (128 or 256). 0 for bad
+ * shapes. */
+int q4_prefill_tile_rows(int T, int64_t N, int64_t K, int swiglu);
+
 /* q4_gemm_prefill_prepared without the split reduce: plane s of the plan's S K-splits at
  * part + s T N (f32 [S][T][N]; S = q4_prefill_split_count; the whole product when S = 1). The
  * planes summed in order are the prepared GEMM's Y bit for bit; q4_rmsnorm_prepare takes them
@@ -580,7 +585,7 @@ int q4_swiglu_prepare(const float* g, const float* u, int64_t ldg, int64_t ldu, 
  * (the q4_moe_gemv expert layout), with its prefill scales for precision 0 (q4_prefill_scales
  * of that matrix). Each h is what q4_swiglu_prepare forms from the plain GEMM's f32 gate and
  * up outputs (the same GEMM bits where that GEMM's plan is unsplit), without the f32 output
- * in memory. 256-row tiles, no K split. F % 128 == 0, K % 64 == 0. Replaces the reference's
+ * in memory. No K split. F % 128 == 0, K % 64 == 0. Replaces the reference's
  * gate/up prefill dispatches and the bf16 SwiGLU after them (moe_batch.h:181-202). */
 int q4_gemm_prefill_swiglu(const uint8_t* gate_up, const void* scales, const void* prepared, int x_dtype, void* h,
                            int T, int64_t F, int64_t K, int precision, void* stream);

@@ -1085,17 +1085,26 @@ struct PrefillPlan {
     int64_t grid;
 };
 
-// Microseconds of one workgroup of the pipelined kernel: nst stages of a tile of `rows` rows x
-// 64 ft tokens, a start-up and the store of its tile (out_bytes per row and token, at a CU's
-// share of ~4.5 TB/s). Per-stage times measured by varying the K split at T = 64 .. 256 on
-// 14336 x 4096, 4096 x 14336 and 4096 x 4096 (a stage holds eight mx tiles in either form, so
-// its dequantization is the same; the MFMAs grow with ft). 192-row tiles take 0.9 of a
-// 256-row tile's stage (gate_up at T = 2048: 236.6 us as 2 rounds of 256-row tiles, 224.9 as
-// 1 round of each).
-double tile_us(int rows, int ft, int nst, double out_bytes) {
-    static constexpr double s256[5] = {0, 0.55, 0.68, 0.85, 1.0}, s128[3] = {0, 0.66, 0.95};
-    const double stage = rows == 128 ? s128[ft] : rows == 192 ? 0.9 * s256[ft] : s256[ft];
-    return nst * stage + 4.0 + rows * 64.0 * ft * out_bytes / 17600.0;
+// Microseconds of one workgroup of the pipelined kernel while `busy` (0 to 1) of the CUs hold one:
+// nst stages of a tile of `rows` rows x 64 ft tokens and the store of the tile (out_bytes per row
+// and token; the CUs share the memory). Fitted, with the reduce below, to the graph replay times
+// of every sensible plan of 906 calls (25 to 4096 tokens, N 512 to 28672, K 1024 to 14336; 578 in
+// precision 0, 328 in precision 1, whose dequantization is slower: one plan serves both). The
+// planned form is 0.7 % slower than the call's fastest (geometric mean; 5 % in the slowest
+// twentieth). Stage times taken at 64 to 256 tokens on few CUs have the 128-row form a tenth
+// too fast on a full chip: 148 tokens on 19712 x 2304 took 51 us where the fastest takes 34,
+// 848 on 3136 x 5824 61 where it takes 54, and 2 % were lost on average.
+double tile_us(int rows, int ft, int nst, double out_bytes, double busy) {
+    static constexpr double s256[5] = {0, 0.66, 0.88, 1.05, 1.28};
+    const double stage = rows == 128 ? (ft == 1 ? 0.56 + 0.32 * busy : 1.03 + 0.26 * busy)
+                                     : s256[ft] * (rows == 192 ? 0.89 : 1.0);
+    return nst * stage + 0.5 + rows * ft / 1024.0 * (out_bytes / 4.0) * (4.8 + 4.5 * busy);
+}
+
+// Finish time of n equal workgroups on C CUs: whole rounds, then the rest on fewer of them.
+template <class Cost>
+double rounds_us(int64_t n, int64_t C, Cost cost) {
+    return (double)(n / C) * cost(1.0) + (n % C ? cost((double)(n % C) / (double)C) : 0.0);
 }
 
 // Finish time of A units of cost cw followed by B units of cost cn when each starts on the
@@ -1132,12 +1141,14 @@ PrefillPlan make_plan_uncached(int T, int64_t N, int64_t K) {
         const char* e = getenv("Q4MI_PREFILL_NARROW");
         return e ? atoi(e) : -1;
     }();
-    const int nst = (int)ceil_div(K, 64), cap = nst < 16 ? nst : 16;
+    const int nst = (int)ceil_div(K, 64), cap = nst < kMaxSplits ? nst : kMaxSplits;
     const int64_t G = N / 64, tt = p.tiles_t;
     const int cus = device_cus();
-    const int ftl = (int)ceil_div(T - (tt - 1) * 256, 64);         // 64-token groups of the last token tile
+    // 64-token groups of a token tile: a row tile's token tiles are neighbours in the grid, so a
+    // ragged one lies among the full ones and a round lasts as long as a full one
+    const int ft = tt > 1 ? 4 : (int)ceil_div(T, 64);
     // the split reduce: a launch and its traffic
-    auto reduce_us = [&](int S) { return S > 1 ? 3.0 + (double)(S + 1) * T * N * 4 / 5.0e6 : 0.0; };
+    auto reduce_us = [&](int S) { return S > 1 ? 2.0 + (double)(S + 1) * T * N * 4 / 4.15e6 : 0.0; };
     // a forced strip count is used only where it fits: 3b <= G and 4 | G - 3b
     const int64_t fb = forced_narrow > 0 && 3 * (int64_t)forced_narrow <= G &&
                                (G - 3 * (int64_t)forced_narrow) % 4 == 0
@@ -1155,13 +1166,13 @@ PrefillPlan make_plan_uncached(int T, int64_t N, int64_t K) {
             if (forced > 0 && S != (forced < cap ? forced : cap)) continue;
             if (b > 0 && b != fb && b * tt * S > 2 * cus) break;
             const int ns = (int)ceil_div(nst, S);
-            const double full = tile_us(256, 4, ns, 4), last = tile_us(256, ftl, ns, 4);
             double cost;
-            if (b > 0) {        // every tile at the mean of the full and the ragged token tiles
-                const double mean = ((double)(tt - 1) + last / full) / (double)tt;
-                cost = makespan(a * tt * S, b * tt * S, cus, mean * full, mean * tile_us(192, 4, ns, 4));
+            if (b > 0) {
+                const double busy = (a + b) * tt * S < cus ? (double)((a + b) * tt * S) / cus : 1.0;
+                cost = makespan(a * tt * S, b * tt * S, cus, tile_us(256, ft, ns, 4, busy),
+                                tile_us(192, ft, ns, 4, busy));
             } else {
-                cost = makespan(a * (tt - 1) * S, a * S, cus, full, last);
+                cost = rounds_us(a * tt * S, cus, [&](double busy) { return tile_us(256, ft, ns, 4, busy); });
             }
             // ties: fewer rows computed (a clamped last 256-row strip repeats rows)
             cost += reduce_us(S) + 1e-6 * (double)(256 * a + 192 * b);
@@ -1177,12 +1188,12 @@ PrefillPlan make_plan_uncached(int T, int64_t N, int64_t K) {
     // 128 x 128 tiles, 128-K stages
     if (forced <= 0 && forced_narrow < 0) {
         const int64_t r2 = ceil_div(G, 2), t2 = ceil_div(T, 128);
-        const int nst2 = (int)ceil_div(K, 128), cap2 = nst2 < 16 ? nst2 : 16;
-        const int ftl2 = (int)ceil_div(T - (t2 - 1) * 128, 64);
+        const int nst2 = (int)ceil_div(K, 128), cap2 = nst2 < kMaxSplits ? nst2 : kMaxSplits;
+        const int ft2 = t2 > 1 ? 2 : (int)ceil_div(T, 64);
         for (int S = 1; S <= cap2; ++S) {
             const int ns = (int)ceil_div(nst2, S);
-            const double cost = makespan(r2 * (t2 - 1) * S, r2 * S, cus, tile_us(128, 2, ns, 4),
-                                         tile_us(128, ftl2, ns, 4)) + reduce_us(S);
+            const double cost = rounds_us(r2 * t2 * S, cus,
+                                          [&](double busy) { return tile_us(128, ft2, ns, 4, busy); }) + reduce_us(S);
             if (cost < best) {
                 best = cost;
                 p.tile = 128;
@@ -1204,9 +1215,13 @@ bool swiglu_tile128(int T, int64_t N, int64_t K) {
     if (K % 128) return false;
     const int cus = device_cus();
     auto finish = [&](int tile, int nst) {
-        const int64_t tt = ceil_div(T, tile), rows = N / tile;
-        const int ftl = (int)ceil_div(T - (tt - 1) * tile, 64);
-        return makespan(rows * (tt - 1), rows, cus, tile_us(tile, tile / 64, nst, 1), tile_us(tile, ftl, nst, 1));
+        const int64_t tt = ceil_div(T, tile);
+        const int ft = tt > 1 ? tile / 64 : (int)ceil_div(T, 64);
+        // and the epilogue's expf and divisions, 4 us for a 256 x 256 tile: of 200 shapes in both
+        // precisions the faster form in all but one, which it misses by 0.5 %
+        return rounds_us(N / tile * tt, cus, [&](double busy) {
+            return tile_us(tile, ft, nst, 1, busy) + tile * ft / 1024.0 * 4.0;
+        });
     };
     return finish(128, (int)(K / 128)) < finish(256, (int)(K / 64));
 }
@@ -1580,6 +1595,13 @@ extern "C" int q4_gemm_prefill_prepared(const uint8_t* packed, const void* scale
 extern "C" int q4_prefill_split_count(int T, int64_t N, int64_t K) {
     if (T <= 0 || N <= 0 || K <= 0 || N % 64 || K % 32) return 0;
     return make_plan(T, N, K).splits;
+}
+
+extern "C" int q4_prefill_tile_rows(int T, int64_t N, int64_t K, int swiglu) {
+    if (T <= 0 || N <= 0 || K <= 0 || N % 64 || K % 32 || (swiglu && (N % 256 || K % 64))) return 0;
+    if (swiglu) return swiglu_tile128(T, N, K) ? 128 : 256;
+    const PrefillPlan p = make_plan(T, N, K);
+    return p.tile == 256 && p.wide_wgs < p.grid ? 192 : p.tile;
 }
 
 extern "C" int q4_gemm_prefill_prepared_partials(const uint8_t* packed, const void* scales, const void* prepared,

@@ -384,6 +384,8 @@ def test_prefill_partials_argument_errors(lib):
     """q4_gemm_prefill_prepared_partials refuses two-pass activations and bad shapes before any
     launch; the split count query follows the plan."""
     assert lib.q4_prefill_split_count(2048, 4096, 14336) >= 1
+    assert lib.q4_prefill_tile_rows(2048, 4100, 14336, 0) == lib.q4_prefill_tile_rows(2048, 8192, 4112, 1) == 0
+    assert lib.q4_prefill_tile_rows(2048, 4224, 4096, 1) == lib.q4_prefill_tile_rows(0, 4096, 4096, 0) == 0
     assert lib.q4_prefill_split_count(2048, 4100, 14336) == 0
     w, sc, prep, part = (C.c_void_p(0x10000000 * i) for i in (1, 2, 3, 4))
     big = 1 << 40
