@@ -129,9 +129,9 @@ def test_prefill_split_tiles_are_deterministic(gpu, pkg, oracle, T, N, K):
 
 @pytest.mark.parametrize("T,N,K", [(256, 192, 64), (256, 448, 256), (1000, 704, 512)])
 def test_prefill_192_row_tiles(gpu, pkg, oracle, T, N, K):
-    """Shapes the planner gives 192-row tiles: N = 192 alone (one 192-row tile instead of a
-    clamped 256-row one), 448 = 256 + 192 with a 4-way K split, 704 = 2 x 256 + 192 with a
-    ragged token count. Same bar as the 256-row tiles."""
+    """Row counts that leave 192 over (192, 256 + 192, 2 x 256 + 192), the last with a ragged token
+    count, in the tiles the planner gives such small grids. The 192-row tiles themselves are in
+    test_gpu_prefill_tiles.py. Same bar as the 256-row tiles."""
     say(f"prefill 192-row tiles T={T} N={N} K={K}")
     rng = np.random.default_rng(T + N + K + 1)
     blocks = oracle.baseline_q4_1_blocks(N, K, rng)
@@ -206,8 +206,7 @@ def test_prefill_fp16_range_per_row(gpu, pkg, oracle, T, N, K, xdt):
     ~5e3 (weights past fp16's 65504) and token rows from ~1e-6 to ~1e5 in magnitude, every
     token row and every weight row held to maxrel <= 1e-3 against the fp64 oracle on its own
     (per row, the bar the tiny rows would miss, and the large ones overflow, without their
-    power-of-two scaling). K = 2080 takes the generic kernel (K % 64 != 0), K = 1024 the
-    pipelined one."""
+    power-of-two scaling). K = 2080 ends inside a K stage, K = 1024 does not."""
     say(f"prefill fp16 range T={T} N={N} K={K} {xdt}")
     rng = np.random.default_rng(T + N + K + (xdt == "f32"))
     blocks = _wide_range_blocks(oracle, rng, N, K, -6.0, 3.5)
@@ -291,7 +290,7 @@ def test_prefill_scales_match_numpy_and_paths_agree(gpu, pkg, oracle):
     (300, 256, 512, "bf16", "fp16"),       # one token tile + a ragged one, unsplit
     (300, 256, 512, "f32", "fp16"),        # value and remainder planes
     (512, 4096, 14336, "bf16", "fp16"),    # config 3's down at T = 512: K split and reduce
-    (200, 192, 96, "bf16", "fp16"),        # K % 64 != 0: rows [T][K], the generic kernel
+    (200, 192, 96, "bf16", "fp16"),        # K % 64 != 0: the last K stage is half zeros
     (300, 256, 512, "f32", "bf16"),        # the reference tile
 ])
 def test_prefill_prepared_activations_equal_the_one_call_path(gpu, pkg, oracle, T, N, K, xdt, precision):
