@@ -371,7 +371,7 @@ __global__ __launch_bounds__(64 * kDnWaves) void moe_down_kernel(const uint8_t* 
 }
 
 // ---------------------------------------------------------------------------
-// Many pairs per expert (more than kManyPerExpert on average): work items are (expert, 32 of its
+// Many pairs per expert (many_pairs): work items are (expert, 32 of its
 // pairs), so an expert's pairs run side by side instead of chunk by chunk in one workgroup, and
 // two 16-token blocks share each weight tile's loads and conversion (gemv_rows_pipe_tb2). The up
 // kernel stores h as the two bf16 halves that the down kernel's MFMAs take. Same arithmetic and
@@ -383,8 +383,17 @@ __global__ __launch_bounds__(64 * kDnWaves) void moe_down_kernel(const uint8_t* 
 // resident workgroups walking runs of items (routing once each): 130 to 164 there, slower
 // below; accumulators kept out of the AGPRs: 139.
 // ---------------------------------------------------------------------------
-constexpr int kManyPerExpert = 12;
-constexpr int kManyExperts = kMaxPairs / kManyPerExpert;   // P > kManyPerExpert E: fewer experts than this
+constexpr int kManyPerExpert = 12, kManyPerExpertWide = 14, kWideExperts = 160;
+constexpr int kManyExperts = kMaxPairs / kManyPerExpertWide;   // no more experts than this have many pairs
+static_assert(kWideExperts <= kManyExperts);
+
+// Whether P pairs over E experts take the kernels below. Up to 160 experts from 12 pairs per expert on
+// (128 experts of 2048 x 768: at 8 pairs 91 -> 96 us, at 10 102 -> 101, at 12.5 116 -> 109; of
+// sizes from 1024 x 128 to 4096 x 512 0.67 to 1.03 of the time, single ones with F <= 384 up to
+// 1.10). More experts fill the chip with one workgroup each, so 12 to 13.6 pairs take 0.99 to 1.14
+// of the time over 200 to 300 experts (2048 x 256 over 300: 126 -> 138 us) and the line lies at
+// 14: from there 0.90 to 1.05.
+bool many_pairs(int64_t P, int64_t E) { return P > (E > kWideExperts ? kManyPerExpertWide : kManyPerExpert) * E; }
 constexpr int kChunk = 32;
 constexpr int kManyDnGroups = 2;
 
@@ -727,10 +736,9 @@ static int moe_impl(const uint8_t* gate_up, const uint8_t* down, const void* x, 
     const int64_t routed_max = E < P ? E : P;
     // At most 2 routed pairs per expert on average (decode batches): the one-accumulator
     // instances, whose lower register use keeps more waves per SIMD. Larger batches stream
-    // each expert's rows once per 16 tokens instead of once per 4, from kManyPerExpert pairs
-    // per expert on once per 32, the 32s side by side (at 8 pairs per expert
-    // 91 -> 96 us over 128 experts, at 10 102 -> 101, at 12.5 116 -> 109).
-    const bool few = P <= 2 * E, many = P > kManyPerExpert * E;
+    // each expert's rows once per 16 tokens instead of once per 4, with many pairs per expert
+    // once per 32, the 32s side by side.
+    const bool few = P <= 2 * E, many = many_pairs(P, E);
     const int ng = many ? (H % (64 * kManyDnGroups) == 0 ? kManyDnGroups : 1)
                         : H % (64 * kDnGroups) == 0 ? kDnGroups : 1;
     const int64_t items = many ? routed_max + P / kChunk : routed_max;   // many: chunks, at most one short per expert

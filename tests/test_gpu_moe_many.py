@@ -42,6 +42,24 @@ def test_many_pairs_equal_small_batches(gpu, pkg, oracle, H, F, xdt, counts):
         assert torch.equal(out[t:t + step], ref), f"tokens {t}.. differ from a small batch"
 
 
+# more experts than a wave's threads count (two per thread), as many as can have many pairs (14 x 292 =
+# 4088), and the last counts of the other kernels; some experts empty
+@pytest.mark.parametrize("E,T", [(129, 1549), (160, 1921), (161, 2255), (200, 2801), (200, 2800), (292, 4090), (292, 4088)])
+def test_many_experts(gpu, pkg, oracle, E, T):
+    say(f"moe many E={E} T={T}")
+    H, F = 128, 64
+    rng = np.random.default_rng(E)
+    gu, dn = _experts(pkg, oracle, gpu, E, H, F, rng)
+    live = rng.permutation(E)[:E - E // 5]
+    live = np.union1d(live, [0, E - 1])
+    ids = torch.from_numpy(np.concatenate([live, rng.choice(live, T - len(live))]).astype(np.int32)).view(T, 1).to(gpu)
+    w = torch.rand(T, 1, generator=torch.Generator(gpu).manual_seed(1), device=gpu)
+    x = torch.randn(T, H, generator=torch.Generator(gpu).manual_seed(2), device=gpu).to(torch.bfloat16)
+    out = pkg.moe_batch(gu, dn, x, ids, w, path="decode")
+    for t in range(0, T, 2 * E):
+        assert torch.equal(out[t:t + 2 * E], pkg.moe_batch(gu, dn, x[t:t + 2 * E], ids[t:t + 2 * E], w[t:t + 2 * E], path="decode"))
+
+
 @pytest.mark.parametrize("T", [33, 64, 97])
 def test_many_pairs_with_shared_expert(gpu, pkg, oracle, T):
     say(f"moe many shared T={T}")
