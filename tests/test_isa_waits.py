@@ -67,6 +67,28 @@ def test_prefill_loop_waits_cover_every_asm_load(tmp_path):
             for body in loops:
                 n, bad = early_uses_in(body)
                 assert n >= 6 and not bad, f"{what} precision {prec}: {n} loads, early uses {bad[:3]}"
+    # every kernel of the pipelined tile, one loop per tile instance: a 256-row tile of 1 to 4 groups of 64
+    # tokens (twice with 192-row tiles beside), a 128-row one of 1 or 2. A new one has to be entered here.
+    bools = ("Lb0", "Lb1")
+    want = {}
+    for prec in ("Li0", "Li1"):
+        want |= {f"prefill_dma_kernelI{prec}ELb0": 1, f"prefill_dma_kernelI{prec}ELb1": 2, f"prefill_dma128_kernelI{prec}": 2,
+                 f"prefill_ragged_kernelI{prec}ELb0": 4, f"prefill_ragged_kernelI{prec}ELb1": 8,
+                 f"prefill_tail_kernelI{prec}ELi2": 4, f"prefill_tail_kernelI{prec}ELi4": 2,
+                 f"prefill_swiglu_kernelI{prec}": 1, f"prefill_swiglu_ragged_kernelI{prec}ELi2": 4,
+                 f"prefill_swiglu_ragged_kernelI{prec}ELi4": 2}
+        want |= {f"moe_dma_kernelI{prec}E{a}E{b}": 1 for a in bools for b in bools}
+        want |= {f"moe_ragged_kernelI{prec}E{a}E{b}": 4 for a in bools for b in bools}
+    found = {}
+    for i, l in enumerate(text):
+        m = re.match(r"_ZN12_GLOBAL__N_1\d+?((?:prefill_(?:dma|dma128|ragged|tail|swiglu|swiglu_ragged)|moe_(?:dma|ragged))_kernelI\w+?)EEEv\w*:", l)
+        if not m:
+            continue
+        stop = next(j for j in range(i, len(text)) if text[j].startswith(".Lfunc_end"))
+        results = [early_uses_in(body) for body in inner_loops(text[i:stop])]
+        assert all(n >= 6 and not bad for n, bad in results), f"{m.group(1)}: {results}"
+        found[m.group(1)] = len(results)
+    assert found == want
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="hipcc not available")
@@ -81,8 +103,8 @@ def test_moe_pipelined_loops_wait_for_every_asm_load(tmp_path):
            str(src), "-o", str(out)]
     subprocess.run(cmd, check=True, capture_output=True, timeout=600)
     text = out.read_text().splitlines()
-    kernels = [l.split(":")[0] for l in text if re.match(r"_ZN12_GLOBAL__N_1\w*moe_(up|down)_kernel\w*:", l)]
-    assert len(kernels) == 8
+    kernels = [l.split(":")[0] for l in text if re.match(r"_ZN12_GLOBAL__N_1\w*moe_(up|down)(_many)?_kernel\w*:", l)]
+    assert len(kernels) == 12
     for k in kernels:
         start = next(i for i, l in enumerate(text) if l.startswith(k + ":"))
         stop = next(i for i in range(start, len(text)) if text[i].startswith(".Lfunc_end"))
