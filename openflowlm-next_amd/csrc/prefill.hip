@@ -715,6 +715,32 @@ __global__ __launch_bounds__(256) void prefill_scale_write_kernel(const uint8_t*
     }
 }
 
+// Eight values of a row into the MFMA's 16-bit type. PREC 0: fp16 of v 2^-s, or on the lo pass of
+// an f32 source its remainder; PREC 1: bf16.
+template <bool F32SRC, int PREC>
+__device__ __forceinline__ u32x4 cvt8(const float (&v)[8], int s, int lo_pass) {
+    u32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        uint32_t lo, hi;
+        if constexpr (PREC == 0) {
+            const float a = ldexpf(v[2 * e], -s), b = ldexpf(v[2 * e + 1], -s);
+            _Float16 ha = (_Float16)a, hb = (_Float16)b;
+            if (F32SRC && lo_pass) {
+                ha = (_Float16)(a - (float)ha);
+                hb = (_Float16)(b - (float)hb);
+            }
+            lo = __builtin_bit_cast(uint16_t, ha);
+            hi = __builtin_bit_cast(uint16_t, hb);
+        } else {
+            lo = f32_to_bf16_rne(v[2 * e]);
+            hi = f32_to_bf16_rne(v[2 * e + 1]);
+        }
+        o[e] = lo | (hi << 16);
+    }
+    return o;
+}
+
 // lo_pass (f32 activations, PREC 0): the fp16 remainder x 2^-s - fp16(x 2^-s) instead of the
 // rounded value; the two passes' products add up to the f32 activations' to ~2^-22.
 // One token row of prefill_xprep (all 256 threads): ld8(i, v) loads the row's 8-element
@@ -766,39 +792,17 @@ __device__ __forceinline__ void xprep_row(Load ld8, bool zero, uint16_t* __restr
         s = fp16_fit_exponent(block_max256(mx, red));
         if (threadIdx.x == 0) texp[t] = s;
     }
-    auto cvt8 = [&](const float (&v)[8]) -> u32x4 {
-        u32x4 o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            uint32_t lo, hi;
-            if constexpr (PREC == 0) {
-                const float a = ldexpf(v[2 * e], -s), b = ldexpf(v[2 * e + 1], -s);
-                _Float16 ha = (_Float16)a, hb = (_Float16)b;
-                if (F32SRC && lo_pass) {
-                    ha = (_Float16)(a - (float)ha);
-                    hb = (_Float16)(b - (float)hb);
-                }
-                lo = __builtin_bit_cast(uint16_t, ha);
-                hi = __builtin_bit_cast(uint16_t, hb);
-            } else {
-                lo = f32_to_bf16_rne(v[2 * e]);
-                hi = f32_to_bf16_rne(v[2 * e + 1]);
-            }
-            o[e] = lo | (hi << 16);
-        }
-        return o;
-    };
     if (held) {
 #pragma unroll
         for (int c = 0; c < kHeld; ++c) {
             const int i = threadIdx.x + 256 * c;
-            if (i < n8) out[dst(i)] = cvt8(hv[c]);
+            if (i < n8) out[dst(i)] = cvt8<F32SRC, PREC>(hv[c], s, lo_pass);
         }
     } else {
         for (int i = threadIdx.x; i < n8; i += 256) {
             float v[8];
             ld8(i, v);
-            out[dst(i)] = cvt8(v);
+            out[dst(i)] = cvt8<F32SRC, PREC>(v, s, lo_pass);
         }
     }
 }
@@ -1246,19 +1250,12 @@ PrefillPlan make_plan(int T, int64_t N, int64_t K) {
 
 size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
-template <bool XF, int PR, bool TL>
-void launch_xprep_t(dim3 g, hipStream_t st, const void* x, uint16_t* x16, int* te, int T, int K, int lo_pass) {
-    hipLaunchKernelGGL((prefill_xprep<XF, PR, TL>), g, dim3(256), 0, st, x, x16, te, T, K, lo_pass);
-}
-
-void launch_xprep(bool xf32, int prec, bool tiled, dim3 g, hipStream_t st, const void* x, uint16_t* x16, int* te,
-                  int T, int K, int lo_pass) {
-    typedef void (*fn_t)(dim3, hipStream_t, const void*, uint16_t*, int*, int, int, int);
-    static const fn_t table[8] = {launch_xprep_t<false, 0, false>, launch_xprep_t<false, 0, true>,
-                                  launch_xprep_t<false, 1, false>, launch_xprep_t<false, 1, true>,
-                                  launch_xprep_t<true, 0, false>,  launch_xprep_t<true, 0, true>,
-                                  launch_xprep_t<true, 1, false>,  launch_xprep_t<true, 1, true>};
-    table[(xf32 ? 4 : 0) + (prec ? 2 : 0) + (tiled ? 1 : 0)](g, st, x, x16, te, T, K, lo_pass);
+// The pre-pass of a GEMM's activations into the pipelined kernel's tiled image.
+void launch_xprep(bool xf32, int prec, dim3 g, hipStream_t st, const void* x, uint16_t* x16, int* te, int T, int K,
+                  int lo_pass) {
+    auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, g, dim3(256), 0, st, x, x16, te, T, K, lo_pass); };
+    if (prec == 0) xf32 ? launch(prefill_xprep<true, 0, true>) : launch(prefill_xprep<false, 0, true>);
+    else xf32 ? launch(prefill_xprep<true, 1, true>) : launch(prefill_xprep<false, 1, true>);
 }
 
 }  // namespace
@@ -1360,7 +1357,7 @@ int prefill_impl(const uint8_t* packed, const void* scales, const void* x, int x
     float* part = (float*)((char*)workspace + xprep_bytes(T, K));
     for (int pass = 0; pass < activation_passes(x_dtype, precision); ++pass) {
         // rows up to whole 64-token groups: the kernels read no others
-        launch_xprep(x_dtype == Q4MI_F32, precision, true, dim3((unsigned)(ceil_div(T, 64) * 64)), st, x, x16, te, T,
+        launch_xprep(x_dtype == Q4MI_F32, precision, dim3((unsigned)(ceil_div(T, 64) * 64)), st, x, x16, te, T,
                      (int)K, pass);
         if (launch_status() != Q4MI_OK) return Q4MI_E_LAUNCH;
         const int rc = gemm_pass(packed, scales, x16, te, y, T, N, K, precision, part, pass, st);
@@ -1437,7 +1434,7 @@ extern "C" int q4_prefill_prepare(const void* x, int x_dtype, int T, int64_t K, 
     const int passes = activation_passes(x_dtype, precision);
     int* te = (int*)((char*)prepared + passes * x16_bytes(T, K));
     for (int pass = 0; pass < passes; ++pass) {
-        launch_xprep(x_dtype == Q4MI_F32, precision, true, dim3((unsigned)padded_tokens(T)),
+        launch_xprep(x_dtype == Q4MI_F32, precision, dim3((unsigned)padded_tokens(T)),
                      (hipStream_t)stream, x, (uint16_t*)((char*)prepared + pass * x16_bytes(T, K)), te, T, (int)K,
                      pass);
         if (launch_status() != Q4MI_OK) return Q4MI_E_LAUNCH;
@@ -1800,32 +1797,6 @@ __global__ __launch_bounds__(256) void moe_slots_xprep_kernel(const int32_t* __r
     const int t = (int)blockIdx.x - E;
     const void* xrow = (const uint8_t*)x + (int64_t)t * H * (XF32 ? 4 : 2);
     xprep_row<XF32, 0, false>([&](int i, float (&v)[8]) { load_x8<XF32>(xrow, i, v); }, false, x16, texp, t, H, 0);
-}
-
-// Eight values of a row into the MFMA's 16-bit type. PREC 0: fp16 of v 2^-s, or on the lo pass of
-// an f32 source its remainder; PREC 1: bf16.
-template <bool F32SRC, int PREC>
-__device__ __forceinline__ u32x4 cvt8(const float (&v)[8], int s, int lo_pass) {
-    u32x4 o;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        uint32_t lo, hi;
-        if constexpr (PREC == 0) {
-            const float a = ldexpf(v[2 * e], -s), b = ldexpf(v[2 * e + 1], -s);
-            _Float16 ha = (_Float16)a, hb = (_Float16)b;
-            if (F32SRC && lo_pass) {
-                ha = (_Float16)(a - (float)ha);
-                hb = (_Float16)(b - (float)hb);
-            }
-            lo = __builtin_bit_cast(uint16_t, ha);
-            hi = __builtin_bit_cast(uint16_t, hb);
-        } else {
-            lo = f32_to_bf16_rne(v[2 * e]);
-            hi = f32_to_bf16_rne(v[2 * e + 1]);
-        }
-        o[e] = lo | (hi << 16);
-    }
-    return o;
 }
 
 // One slot row per wave (4 per workgroup) of the MoE activation preps: xprep_row's
@@ -2230,7 +2201,9 @@ extern "C" int q4_moe_prefill(const uint8_t* gate_up, const uint8_t* down, const
         if (gx && pass == 0) {
             // done with the slots
         } else if (gx) {
-            launch_xprep(xf32, 0, false, dim3((unsigned)T), st, x, x16, texp, T, (int)H, pass);
+            // the remainder pass of f32 x, in rows for the gather
+            hipLaunchKernelGGL((prefill_xprep<true, 0, false>), dim3((unsigned)T), dim3(256), 0, st, x, x16, texp, T,
+                               (int)H, pass);
         } else if (xf32) {
             if (precision == 0)
                 hipLaunchKernelGGL((moe_xprep_kernel<true, 0>), dim3(SP), dim3(256), 0, st, x, rowmap, meta, x16, texp,
