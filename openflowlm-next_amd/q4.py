@@ -54,10 +54,16 @@ def _device(dev=None) -> torch.device:
     return d if d.index is not None else torch.device("cuda", torch.cuda.current_device())
 
 
+# torch's raw getter: torch.cuda.current_stream builds a Stream object first (1.9 us against 0.1,
+# twice per call with a cached workspace). It is not public API, so a torch without it takes the
+# object's handle.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or \
+    (lambda index: torch.cuda.current_stream(index).cuda_stream)
+
+
 def _stream(dev: torch.device) -> int:
-    """The handle of torch's current stream on dev. The raw getter, as torch.cuda.current_stream
-    builds a Stream object first (1.9 us against 0.1, twice per call with a cached workspace)."""
-    return torch._C._cuda_getCurrentRawStream(dev.index)
+    """The handle of torch's current stream on dev."""
+    return _raw_stream(dev.index)
 
 
 _HERE = contextlib.nullcontext()
