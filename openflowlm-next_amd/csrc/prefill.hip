@@ -490,8 +490,8 @@ __device__ __forceinline__ void dma_tile(uint8_t* lds, const uint8_t* __restrict
 }
 
 // dma_tile with the smallest token tile that covers the valid tokens [t0, T) of a tile of
-// 64 * FTMAX (workgroup-uniform). A 256-row stage takes ~0.55, 0.68, 0.85 and 1.0 us with 1 to 4
-// groups of 64 tokens: the dequantization and the LDS traffic of the weights remain.
+// 64 * FTMAX (workgroup-uniform). A 256-row stage takes 0.66, 0.88, 1.05 and 1.28 us with 1 to 4
+// groups of 64 tokens (tile_us): the dequantization and the LDS traffic of the weights remain.
 template <int PREC, int KBS, int FN, int FTMAX, bool SWI = false, bool GATHER = false, bool TAIL = false, class... A>
 __device__ __forceinline__ void dma_tile_valid(uint8_t* lds, const uint8_t* packed, const uint16_t* x16,
                                                const int* texp, const int* wexp, const uint32_t* s16, float* y, int T,
@@ -1076,7 +1076,7 @@ int device_cus() {
 // and for the 256-row form the rows covered by 256-row tiles ([0, narrow_row0), wide_wgs
 // workgroups) and by 192-row tiles (the rest; K % 64 == 0). Both forms hold one workgroup per
 // CU (160 KB of LDS). Three levers fit the work to the CUs: the tile (128 x 128: four times
-// the tiles, so small grids need fewer K splits and their partial traffic, at two thirds
+// the tiles, so small grids need fewer K splits and their partial traffic, at 0.5 to 0.6
 // of the MFMA rate), a K split (partial sums
 // reduced in order afterwards) and 192-row tiles, which fill the CUs the last round of 256-row
 // tiles leaves idle without any partial traffic (Llama-3-8B gate_up at T = 2048: 448 tiles of
@@ -2015,7 +2015,8 @@ __global__ __launch_bounds__(512) void moe_ragged_kernel(const uint8_t* __restri
 
 // The grouped expert GEMM of a launch: one ragged tile per expert, so up to kMoeFullTiles tiles per
 // expert on average the kernel whose tiles follow their valid slots (128 experts, top-8 of
-// 2048 tokens, 128 of a tile's 256 slots valid: gate/up 191 -> 165 us, down 147 -> 118), beyond
+// 2048 tokens, 128 of a tile's 256 slots valid: gate/up 191 -> 165 us, down 147 -> 118; 144 and
+// 103 with the runs above, in the middle of 400 passes), beyond
 // that the one-body kernel, where at most 1 / kMoeFullTiles of the tiles could gain.
 constexpr int kMoeFullTiles = 16;
 template <int PREC, bool SWI = false, bool GATHER = false>
